@@ -369,11 +369,11 @@ struct TeamFft {
   // Stockham stage of radix RAD after span NS.  Reads the stage input from
   // LDS line s.  OUT 0: results back to LDS (Stockham positions);
   // OUT 1: final results into registers (v[m] = X[q + T m]).
-  // In the natural mapping a line of T = 64 threads is exactly one
-  // wavefront (wave64), so LDS traffic that stays inside a line needs only
-  // wavefront-scope ordering (a wavefront's LDS operations are executed in
-  // order); traffic across lines needs the work-group barrier.
-  static constexpr bool kWaveLines = (T == 64);
+  // In the natural mapping a line of T <= 64 threads (a power of two) lies
+  // in one wavefront (wave64), so LDS traffic that stays inside a line needs
+  // only wavefront-scope ordering (a wavefront's LDS operations are executed
+  // in order); traffic across lines needs the work-group barrier.
+  static constexpr bool kWaveLines = (T <= 64);
   // The work-group case orders LDS only (the transforms exchange data
   // through LDS alone): it waits for this wave's LDS operations, not for
   // its outstanding global loads and stores, so copies issued before a

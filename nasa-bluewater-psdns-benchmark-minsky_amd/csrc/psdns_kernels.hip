@@ -511,7 +511,11 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
 template <typename R, int N>
 struct XPass {
   static constexpr int M = N / 2;
-  static constexpr int T = Team<M, 8>::T, E = Team<M, 8>::E;
+  // points per thread: 8 from M = 256 on (three stages, 8 8 4, where four of
+  // radix 4 exchanged through LDS once more: 512^3 FP32 1.14 -> 0.87 ms per
+  // launch, with two scalars 2.81 -> 2.07 ms), 4 below (M = 64 with 8 is
+  // slower, 33 against 25 us at 128^3 FP32; M = 128 the same either way)
+  static constexpr int E = M >= 256 ? 8 : Team<M, 8>::E, T = M / E;
   static constexpr int K = RunLines<R>::B;          // one 64-byte run of z (or of kx in X)
   // z lines per tile (one run; two runs per tile measured slower: the
   // LDS of 16 lines leaves one work-group per CU)
