@@ -46,6 +46,8 @@ uint64_t splitmix64(uint64_t x) {
 
 }  // namespace
 
+constexpr int kLossBlock = 1024;  // steps of a training call between two reads of their losses
+
 struct psdns_sgs {
   int n = 0;          // LES grid
   size_t P = 0;       // n^3
@@ -65,9 +67,9 @@ struct psdns_sgs {
   float *theta = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr;
   long long adam_t = 0;
   // minibatch work
-  int work_B = 0;
-  float* work = nullptr;
-  S::Work w{};
+  int work_rows = 0;
+  float* work = nullptr;       // partial rows of the gradient
+  double* losses = nullptr;    // of up to kLossBlock steps
   double* lpart = nullptr;  // loss / error partial sums
   size_t lpart_n = 0;
 };
@@ -91,34 +93,14 @@ int ensure_lpart(psdns_sgs* m, size_t cnt) {
 }
 
 int ensure_work(psdns_sgs* m, int B) {
-  if (m->work_B >= B) return 0;
+  const int rows = S::train_rows(B);
+  if (m->work_rows >= rows) return 0;
   if (m->work) (void)hipFree(m->work);
   m->work = nullptr;
-  m->work_B = 0;
-  if (int rc = dalloc(&m->work, S::work_floats(B), "the minibatch work arrays")) return rc;
-  float* p = m->work;
-  auto take = [&](size_t cnt) {
-    float* r = p;
-    p += cnt;
-    return r;
-  };
-  S::Work& w = m->w;
-  w.X0 = take((size_t)B * S::kIn0);
-  w.X1 = take((size_t)B * S::kIn1);
-  w.H1 = take((size_t)B * S::kHid);
-  w.H2 = take((size_t)B * S::kHid);
-  w.H3 = take((size_t)B * S::kHid);
-  w.G = take((size_t)B * S::kBasis);
-  w.Tb = take((size_t)B * 24);
-  w.taub = take((size_t)B * 6);
-  w.dG = take((size_t)B * S::kBasis);
-  w.D3 = take((size_t)B * S::kHid);
-  w.D2 = take((size_t)B * S::kHid);
-  w.D1 = take((size_t)B * S::kHid);
-  w.D0 = take((size_t)B * S::kConv);
-  w.part = p;
-  m->work_B = B;
-  return ensure_lpart(m, (size_t)(B + 255) / 256);
+  m->work_rows = 0;
+  if (int rc = dalloc(&m->work, (size_t)rows * S::kParams, "the gradient's partial rows")) return rc;
+  m->work_rows = rows;
+  return 0;
 }
 
 // fold n partial sums on the host in order
@@ -181,7 +163,7 @@ int psdns_sgs_create(int n, int max_snapshots, psdns_sgs** out) {
       hipMemsetAsync(m->m, 0, sizeof(float) * S::kParams, m->stream) != hipSuccess ||
       hipMemsetAsync(m->v, 0, sizeof(float) * S::kParams, m->stream) != hipSuccess)
     return bail(set_error(PSDNS_EHIP, "hipMemsetAsync failed"));
-  if ((rc = ensure_lpart(m, 1024))) return bail(rc);
+  if ((rc = ensure_lpart(m, 1024)) || (rc = dalloc(&m->losses, kLossBlock, "the losses"))) return bail(rc);
   if ((rc = sync(m))) return bail(rc);
   *out = m;
   return PSDNS_OK;
@@ -191,7 +173,7 @@ int psdns_sgs_destroy(psdns_sgs* m) {
   if (!m) return PSDNS_OK;
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   void* ptrs[] = {m->cyl, m->yw, m->xi, m->A, m->lam, m->T, m->tau, m->tau_hat, m->h0, m->lam_s, m->T_s,
-                  m->tau_s, m->theta, m->m, m->v, m->grad, m->work, m->lpart};
+                  m->tau_s, m->theta, m->m, m->v, m->grad, m->work, m->lpart, m->losses};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -378,13 +360,11 @@ int psdns_sgs_gradient(psdns_sgs* m, int batch, unsigned long long seed, long lo
   if (!m || !grad || !loss) return set_error(PSDNS_EINVAL, "null argument");
   if (int rc = batch_args(m, batch, sigma2)) return rc;
   if (int rc = ensure_work(m, batch)) return rc;
-  const float inv = (float)(1.0 / ((double)batch * sigma2));
-  S::launch_train_batch(m->stream, m->w, m->theta, m->lam_s, m->T_s, m->tau_s, m->n, m->nsnap,
-                        batch_base(seed, step), batch, inv, m->grad, m->lpart);
+  const double scale = 1.0 / ((double)batch * sigma2);
+  S::launch_train_batch(m->stream, m->theta, m->lam_s, m->T_s, m->tau_s, m->n, m->nsnap, batch_base(seed, step), batch,
+                        (float)scale, m->work, m->lpart, scale, m->grad, m->losses, nullptr, nullptr, 0.f, 0);
   SGSCHK(hipGetLastError());
-  double s;
-  if (int rc = fold(m, (size_t)(batch + 255) / 256, &s)) return rc;
-  *loss = s / ((double)batch * sigma2);
+  SGSCHK(hipMemcpyAsync(loss, m->losses, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   SGSCHK(hipMemcpyAsync(grad, m->grad, sizeof(float) * S::kParams, hipMemcpyDeviceToHost, m->stream));
   return sync(m);
 }
@@ -396,20 +376,16 @@ int psdns_sgs_train(psdns_sgs* m, int nsteps, int batch, double lr, unsigned lon
   if (!(lr > 0)) return set_error(PSDNS_EINVAL, "lr must be positive");
   if (int rc = batch_args(m, batch, sigma2)) return rc;
   if (int rc = ensure_work(m, batch)) return rc;
-  const float inv = (float)(1.0 / ((double)batch * sigma2));
-  const size_t nb = (size_t)(batch + 255) / 256;
+  const double scale = 1.0 / ((double)batch * sigma2);
   for (int i = 0; i < nsteps; i++) {
     const long long t = ++m->adam_t;
-    S::launch_train_batch(m->stream, m->w, m->theta, m->lam_s, m->T_s, m->tau_s, m->n, m->nsnap,
-                          batch_base(seed, t), batch, inv, m->grad, m->lpart);
-    const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, (double)t)));
-    const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)t)));
-    S::launch_adam(m->stream, m->theta, m->m, m->v, m->grad, (float)lr, c1, c2);
+    const int j = i % kLossBlock;
+    S::launch_train_batch(m->stream, m->theta, m->lam_s, m->T_s, m->tau_s, m->n, m->nsnap, batch_base(seed, t), batch,
+                          (float)scale, m->work, m->lpart, scale, m->grad, m->losses + j, m->m, m->v, (float)lr, t);
     SGSCHK(hipGetLastError());
-    if (losses) {
-      double s;
-      if (int rc = fold(m, nb, &s)) return rc;
-      losses[i] = s / ((double)batch * sigma2);
+    if (losses && (j == kLossBlock - 1 || i == nsteps - 1)) {
+      SGSCHK(hipMemcpyAsync(losses + (i - j), m->losses, sizeof(double) * (j + 1), hipMemcpyDeviceToHost, m->stream));
+      if (int rc = sync(m)) return rc;
     }
   }
   m->have_pred = false;

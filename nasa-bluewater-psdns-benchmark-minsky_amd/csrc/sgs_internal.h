@@ -32,20 +32,12 @@ constexpr int kIn0 = kLam * kTaps;  // conv inputs per point
 constexpr int kIn1 = kLam + kConv;  // first MLP layer inputs
 constexpr int kParams = kConv * kIn0 + kConv + kHid * kIn1 + kHid + 2 * (kHid * kHid + kHid) + kBasis * kHid + kBasis;
 constexpr double kQeps = 1e-30;     // floor of q = |S|^2 + |W|^2
-constexpr int kChunk = 512;         // samples per partial sum of a weight gradient
 constexpr int kMaxBatch = 65536;
 
-// minibatch work arrays (row-major per sample)
-struct Work {
-  float *X0, *X1, *H1, *H2, *H3, *G, *Tb, *taub;  // inputs, activations
-  float *dG, *D3, *D2, *D1, *D0;                  // pre-activation gradients
-  float* part;                                    // weight-gradient chunk sums
-};
-inline size_t work_floats(int B) {
-  const size_t nch = (B + kChunk - 1) / kChunk;
-  return (size_t)B * (kIn0 + kIn1 + 3 * kHid + kBasis + 24 + 6 + kBasis + 3 * kHid + kConv) +
-         nch * (size_t)kHid * (kIn0 + 1);
-}
+// work-groups of a training step's gradient kernel = partial rows of kParams
+// floats: one per tile of 64 points up to one per CU (its LDS fills a CU, and
+// more rows would only lengthen the fold)
+constexpr int train_rows(int B) { return (B + 63) / 64 < 256 ? (B + 63) / 64 : 256; }
 
 void launch_box_filter(hipStream_t st, int prec, const void* u, int n, int r, void* ubar, float* tau);
 // i k_j u_i on the mask; with a stage (1|2) the state is first phase shifted
@@ -59,10 +51,9 @@ void launch_add_stress(hipStream_t st, int prec, void* ux, const float* tau, siz
 int field_err_blocks();
 void launch_field_err(hipStream_t st, const float* tp, const float* tt, size_t P, double* part);
 void launch_target_norm(hipStream_t st, const float* tau_s, size_t P, int nsnap, double* part);
-void launch_train_batch(hipStream_t st, const Work& w, const float* theta, const float* lam_s, const float* T_s,
-                        const float* tau_s, int n, int nsnap, uint64_t base, int B, float inv, float* grad,
-                        double* lpart);
-void launch_adam(hipStream_t st, float* th, float* m, float* v, const float* g, float lr, float c1, float c2);
+void launch_train_batch(hipStream_t st, float* theta, const float* lam_s, const float* T_s, const float* tau_s, int n,
+                        int nsnap, uint64_t base, int B, float inv, float* part, double* lpart, double scale,
+                        float* grad, double* loss, float* m, float* v, float lr, long long t);
 
 }  // namespace sgs
 }  // namespace psdns

@@ -20,6 +20,7 @@
 //   W4[4][64]   b4[4]    basis coefficients g; tau = sum_n g_n T_n
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 
 #include "fft_line.hpp"
@@ -186,146 +187,377 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// conv input k of point (y, z, x): lambda[k / 27] at the neighbour d = k % 27
-// (n a power of two: the periodic wrap is a mask)
-__device__ __forceinline__ float conv_in(const float* __restrict__ lam, size_t P, int n, int y, int z, int x, int k) {
-  const int ch = k / kTaps, d = k % kTaps;
-  const int dy = d / 9 - 1, dz = (d / 3) % 3 - 1, dx = d % 3 - 1, w = n - 1;
-  return lam[ch * P + pidx((y + dy) & w, (z + dz) & w, (x + dx) & w, n)];
-}
-
 // ---------------------------------------------------------------------------
 // Training (FP32).  A minibatch of B points is drawn from the snapshot store
 // by the counter map g = splitmix64(base + b) mod (S P), base =
-// splitmix64(seed * 0xD1B54A32D192ED03 + step); its network inputs are
-// gathered into row-major arrays; each layer is a dense kernel; the weight
-// gradients are summed in fixed chunks and folded in chunk order (no
-// atomics: a step gives the same bits every time).
+// splitmix64(seed * 0xD1B54A32D192ED03 + step).  k_train takes tiles of 64
+// points through the whole network and back in one work-group: the gather,
+// the layers, the loss, the gradients of the pre-activations and the weight
+// gradients, which stay in the registers of its four waves over its tiles
+// (tile t to work-group t mod gridDim) and leave as one row of partial sums;
+// k_train_fold adds the rows in row order in FP64 and applies Adam.  No
+// atomics and a grid that depends on B only: a step gives the same bits
+// every time.
+//
+// The layers run on v_mfma_f32_16x16x4_f32 (FP32 operands, products and sums),
+// transposed (Y^T = W X^T) with a wave's 16 points as the columns.  Lane l
+// (r or c = l % 16, g = l / 16) supplies A[r][k] and B[k][c] for one k per
+// instruction and receives D[4 g + jj][c].  With the K order k = 16 ob + 4 g +
+// jj for step (ob, jj) the accumulators of a layer are the next layer's
+// operand B, forward and (with W^T as operand A) backward, so activations and
+// gradients stay in registers; the weights are read from LDS.  A weight
+// gradient is dZ X^T over the tile's 64 points: dZ and X pass through LDS as
+// [feature][point] rows, wave w forms the row block o = 16 w .. of it.
+// What bounds it: the chain of a tile (gather, about 560 matrix instructions
+// of 32 cycles, 52 tanhf, five exchanges through LDS) with one wave per SIMD:
+// 52 us at B = 16384 (a tile per CU), 35 us at B = 1000; its arithmetic (6 x
+// 12164 flops per point) would take 8 us on the matrix cores.
+// 20 steps of B = 16384 took 37.4 ms as a gather, five layer kernels, four
+// backward ones, five weight-gradient kernels with their folds and Adam (one
+// thread per output: 286 us for a 64 x 64 weight gradient); 1.18 ms this way.
 // ---------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kTS = 64;        // points per tile
+constexpr int kLd = kTS + 4;   // row stride of the [feature][point] and 64-wide weight rows
+constexpr int kW0ld = kIn0 + 2;  // W0 rows, zero at k = 135 (K runs in fours)
+
 __global__ void __launch_bounds__(256)
-    k_gather(const float* __restrict__ lam_s, const float* __restrict__ T_s, const float* __restrict__ tau_s, int n,
-             int nsnap, uint64_t base, int B, float* __restrict__ X0, float* __restrict__ X1, float* __restrict__ Tb,
-             float* __restrict__ taub) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
+    k_train(const float* __restrict__ lam_s, const float* __restrict__ T_s, const float* __restrict__ tau_s, int n,
+            int nsnap, uint64_t base, int B, float inv, const float* __restrict__ theta, float* __restrict__ part,
+            double* __restrict__ lpart) {
+  __shared__ float W0s[kConv * kW0ld], W1s[kHid * kIn1], W4s[kBasis * kLd];
+  __shared__ __attribute__((aligned(16))) float W2s[kHid * kLd], W3s[kHid * kLd];
+  __shared__ float b0s[kConv], b1s[kHid], b2s[kHid], b3s[kHid], b4s[kBasis];
+  __shared__ __attribute__((aligned(16))) float X0s[144 * kLd];  // conv inputs, rows 135.. zero
+  __shared__ __attribute__((aligned(16))) float Ps[kHid * kLd], Qs[kHid * kLd];
+  __shared__ float Ts[24 * kTS], taus[6 * kTS];
+  __shared__ double red[4];
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  for (int i = tid; i < kConv * kW0ld; i += 256) {
+    const int o = i / kW0ld, k = i % kW0ld;
+    W0s[i] = k < kIn0 ? theta[oW0 + o * kIn0 + k] : 0.f;
+  }
+  for (int i = tid; i < kHid * kIn1; i += 256) W1s[i] = theta[oW1 + i];
+  for (int i = tid; i < kHid * kHid; i += 256) {
+    W2s[i / kHid * kLd + i % kHid] = theta[oW2 + i];
+    W3s[i / kHid * kLd + i % kHid] = theta[oW3 + i];
+  }
+  W4s[tid / kHid * kLd + tid % kHid] = theta[oW4 + tid];
+  if (tid < kHid) {
+    b1s[tid] = theta[ob1 + tid];
+    b2s[tid] = theta[ob2 + tid];
+    b3s[tid] = theta[ob3 + tid];
+  }
+  if (tid < kConv) b0s[tid] = theta[ob0 + tid];
+  if (tid < kBasis) b4s[tid] = theta[ob4 + tid];
+  for (int i = tid; i < (144 - kIn0) * kLd; i += 256) X0s[kIn0 * kLd + i] = 0.f;
+
+  auto mm = [](float a, float b, f32x4 d) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, d, 0, 0, 0); };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 gW0[3] = {zero, zero, zero}, gW1[2] = {zero, zero}, gW2[4] = {zero, zero, zero, zero},
+        gW3[4] = {zero, zero, zero, zero}, gW4 = zero;
+  float gb0 = 0.f, gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, gb4 = 0.f;
+  double lsum = 0.0;
   const size_t P = (size_t)n * n * n;
-  const uint64_t gidx = splitmix64(base + (uint64_t)b) % ((uint64_t)nsnap * P);
-  const size_t s = gidx / P, p = gidx % P;
-  const int y = (int)(p / ((size_t)n * n)), z = (int)((p / n) % n), x = (int)(p % n);
-  const float* lam = lam_s + s * kLam * P;
-  for (int k = 0; k < kIn0; k++) X0[(size_t)b * kIn0 + k] = conv_in(lam, P, n, y, z, x, k);
-  for (int c = 0; c < kLam; c++) X1[(size_t)b * kIn1 + c] = lam[c * P + p];
-  for (int e = 0; e < 24; e++) Tb[(size_t)b * 24 + e] = T_s[(s * 24 + e) * P + p];
-  for (int c = 0; c < 6; c++) taub[(size_t)b * 6 + c] = tau_s[(s * 6 + c) * P + p];
-}
-
-// Y[b][yo + o] = act(bias[o] + sum_i X[b][xo + i] W[o][i])
-template <bool TANH>
-__global__ void __launch_bounds__(256)
-    k_dense_fwd(const float* __restrict__ X, int ldx, int xo, const float* __restrict__ W,
-                const float* __restrict__ bias, int I, int O, float* __restrict__ Y, int ldy, int yo, int B) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B * O) return;
-  const int b = t / O, o = t % O;
-  const float* x = X + (size_t)b * ldx + xo;
-  const float* w = W + (size_t)o * I;
-  float acc = bias[o];
-  for (int i = 0; i < I; i++) acc = fmaf(x[i], w[i], acc);
-  Y[(size_t)b * ldy + yo + o] = TANH ? tanhf(acc) : acc;
-}
-
-// loss terms: e = sum_n g_n T_n - tau; dG[b][n] = 2 inv sum_c cw_c e_c T_n,c;
-// part[block] = sum over the block's samples of sum_c cw_c e_c^2 (FP64,
-// fixed tree order)
-__global__ void __launch_bounds__(256)
-    k_loss(const float* __restrict__ G, const float* __restrict__ Tb, const float* __restrict__ taub, int B,
-           float inv, float* __restrict__ dG, double* __restrict__ part) {
-  __shared__ double red[256];
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  double l = 0.0;
-  if (b < B) {
-    float e[6];
-    const float* T = Tb + (size_t)b * 24;
-    for (int c = 0; c < 6; c++) {
-      float s = -taub[(size_t)b * 6 + c];
-      for (int k = 0; k < kBasis; k++) s = fmaf(G[(size_t)b * kBasis + k], T[k * 6 + c], s);
-      e[c] = s;
-      l += (double)kCw[c] * (double)s * (double)s;
+  const int m = n - 1, col = 16 * w + c;
+  // rows 16 ob + 4 g + jj of a layer's D to an LDS array
+  auto put = [&](float* S, const f32x4* d, int nob) {
+#pragma unroll
+    for (int o = 0; o < 4; o++)
+      if (o < nob)
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) S[(16 * o + 4 * g + jj) * kLd + col] = d[o][jj];
+  };
+  // acc += the 16 x 16 block (rows of dz, rows of x) of dZ X^T over 64 points
+  auto wgrad = [&](f32x4& acc, const float* dz, const float* x) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const f32x4 a = *(const f32x4*)(dz + c * kLd + 16 * q + 4 * g), b = *(const f32x4*)(x + c * kLd + 16 * q + 4 * g);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) acc = mm(a[jj], b[jj], acc);
     }
-    for (int k = 0; k < kBasis; k++) {
-      float d = 0.f;
-      for (int c = 0; c < 6; c++) d = fmaf(kCw[c] * e[c], T[k * 6 + c], d);
-      dG[(size_t)b * kBasis + k] = 2.f * inv * d;
+  };
+  // row sums (this lane's share) of a 16-row block
+  auto bgrad = [&](float& acc, const float* dz) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const f32x4 a = *(const f32x4*)(dz + c * kLd + 16 * q + 4 * g);
+      acc += (a[0] + a[1]) + (a[2] + a[3]);
     }
-  }
-  red[threadIdx.x] = l;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+  };
+  // dense 64 -> 64: rows of W (or, TR, of W^T) against the registers x
+  auto dense = [&](const float* W, const f32x4* x, f32x4 d, int ob, bool tr) {
+#pragma unroll
+    for (int o = 0; o < 4; o++) {
+      f32x4 a;
+      if (tr) {
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) a[jj] = W[(16 * o + 4 * g + jj) * kLd + 16 * ob + c];
+      } else {
+        a = *(const f32x4*)(W + (16 * ob + c) * kLd + 16 * o + 4 * g);
+      }
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d = mm(a[jj], x[o][jj], d);
+    }
+    return d;
+  };
+
+  const int ntiles = (B + kTS - 1) / kTS;
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    // gather: point lane of the tile; wave w takes every fourth row of three
+    // x neighbours, basis entry and stress component (points past B read
+    // point 0 and are left out of the loss)
+    {
+      const int b = t * kTS + lane;
+      const uint64_t gidx = b < B ? splitmix64(base + (uint64_t)b) % ((uint64_t)nsnap * P) : 0;
+      const size_t s = gidx / P, p = gidx % P;
+      const int y = (int)(p / ((size_t)n * n)), z = (int)((p / n) & m), x = (int)(p & m);
+      const float* lam = lam_s + s * kLam * P;
+      float v[12][3], tv[6], uv[2];
+#pragma unroll
+      for (int i = 0; i < 12; i++) {
+        const int row = min(w + 4 * i, kLam * 9 - 1);  // ch, dy, dz
+        const float* src = lam + (row / 9) * P +
+                           (((size_t)((y + (row / 3) % 3 - 1) & m) * n + ((z + row % 3 - 1) & m)) * n);
+        v[i][0] = src[(x - 1) & m];
+        v[i][1] = src[x];
+        v[i][2] = src[(x + 1) & m];
+      }
+#pragma unroll
+      for (int i = 0; i < 6; i++) tv[i] = T_s[(s * 24 + w + 4 * i) * P + p];
+#pragma unroll
+      for (int i = 0; i < 2; i++) uv[i] = tau_s[(s * 6 + min(w + 4 * i, 5)) * P + p];
+#pragma unroll
+      for (int i = 0; i < 12; i++)
+        if (w + 4 * i < kLam * 9)
+#pragma unroll
+          for (int d = 0; d < 3; d++) X0s[(3 * (w + 4 * i) + d) * kLd + lane] = v[i][d];
+#pragma unroll
+      for (int i = 0; i < 6; i++) Ts[(w + 4 * i) * kTS + lane] = tv[i];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+        if (w + 4 * i < 6) taus[(w + 4 * i) * kTS + lane] = uv[i];
+    }
     __syncthreads();
+    // forward
+    f32x4 h0, h1[4], h2[4], h3[4];
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) h0[jj] = b0s[4 * g + jj];
+#pragma unroll
+    for (int k = 0; k < 136; k += 4) h0 = mm(W0s[c * kW0ld + k + g], X0s[(k + g) * kLd + col], h0);
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) h0[jj] = tanhf(h0[jj]);
+    const float l0 = X0s[(27 * g + 13) * kLd + col], l1 = g == 0 ? X0s[(27 * 4 + 13) * kLd + col] : 0.f;
+#pragma unroll
+    for (int ob = 0; ob < 4; ob++) {
+      const float* wr = W1s + (16 * ob + c) * kIn1;
+      f32x4 d;
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d[jj] = b1s[16 * ob + 4 * g + jj];
+      d = mm(wr[g], l0, d);
+      d = mm(wr[4], l1, d);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d = mm(wr[kLam + 4 * g + jj], h0[jj], d);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) h1[ob][jj] = tanhf(d[jj]);
+    }
+#pragma unroll
+    for (int ob = 0; ob < 4; ob++) {
+      f32x4 d;
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d[jj] = b2s[16 * ob + 4 * g + jj];
+      d = dense(W2s, h1, d, ob, false);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) h2[ob][jj] = tanhf(d[jj]);
+    }
+#pragma unroll
+    for (int ob = 0; ob < 4; ob++) {
+      f32x4 d;
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d[jj] = b3s[16 * ob + 4 * g + jj];
+      d = dense(W3s, h2, d, ob, false);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) h3[ob][jj] = tanhf(d[jj]);
+    }
+    // output layer: rows 0..3 (lanes 0..15) are the coefficients of point col
+    f32x4 gc;
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) gc[jj] = b4s[jj];
+#pragma unroll
+    for (int o = 0; o < 4; o++)
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++)
+        gc = mm(W4s[(c & 3) * kLd + 16 * o + 4 * g + jj], h3[o][jj], gc);
+    // loss terms: e = sum_n g_n T_n - tau; dG_n = 2 inv sum_c cw_c e_c T_n,c
+    double l = 0.0;
+    if (g == 0) {
+      const bool live = t * kTS + col < B;
+      float dg[kBasis] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < 6; q++) {
+        float e = -taus[q * kTS + col];
+#pragma unroll
+        for (int k = 0; k < kBasis; k++) e = fmaf(gc[k], Ts[(k * 6 + q) * kTS + col], e);
+        l += (double)kCw[q] * (double)e * (double)e;
+#pragma unroll
+        for (int k = 0; k < kBasis; k++) dg[k] = fmaf(kCw[q] * e, Ts[(k * 6 + q) * kTS + col], dg[k]);
+      }
+      if (!live) l = 0.0;
+#pragma unroll
+      for (int k = 0; k < kBasis; k++) Ps[k * kLd + col] = live ? 2.f * inv * dg[k] : 0.f;
+    }
+    for (int off = 8; off > 0; off >>= 1) l += __shfl_xor(l, off);
+    lsum += l;
+    put(Qs, h3, 4);
+    __syncthreads();
+    // W4 (rows 4 .. 15 of the block are not used) and dZ3 = W4^T dG (1 - h3^2)
+    wgrad(gW4, Ps, Qs + 16 * w * kLd);
+    bgrad(gb4, Ps);
+    f32x4 d3[4], d2[4], d1[4], d0;
+    const float dgk = Ps[g * kLd + col];
+#pragma unroll
+    for (int ob = 0; ob < 4; ob++) {
+      d3[ob] = mm(W4s[g * kLd + 16 * ob + c], dgk, zero);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d3[ob][jj] *= 1.f - h3[ob][jj] * h3[ob][jj];
+    }
+    __syncthreads();
+    put(Ps, d3, 4);
+    put(Qs, h2, 4);
+    __syncthreads();
+#pragma unroll
+    for (int ib = 0; ib < 4; ib++) wgrad(gW3[ib], Ps + 16 * w * kLd, Qs + 16 * ib * kLd);
+    bgrad(gb3, Ps + 16 * w * kLd);
+#pragma unroll
+    for (int ob = 0; ob < 4; ob++) {
+      d2[ob] = dense(W3s, d3, zero, ob, true);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d2[ob][jj] *= 1.f - h2[ob][jj] * h2[ob][jj];
+    }
+    __syncthreads();
+    put(Ps, d2, 4);
+    put(Qs, h1, 4);
+    __syncthreads();
+#pragma unroll
+    for (int ib = 0; ib < 4; ib++) wgrad(gW2[ib], Ps + 16 * w * kLd, Qs + 16 * ib * kLd);
+    bgrad(gb2, Ps + 16 * w * kLd);
+#pragma unroll
+    for (int ob = 0; ob < 4; ob++) {
+      d1[ob] = dense(W2s, d2, zero, ob, true);
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++) d1[ob][jj] *= 1.f - h1[ob][jj] * h1[ob][jj];
+    }
+    __syncthreads();
+    put(Ps, d1, 4);
+    // the first layer's inputs [lambda, h0] (rows 21 .. 31 are not used)
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) Qs[(kLam + 4 * g + jj) * kLd + col] = h0[jj];
+    Qs[g * kLd + col] = l0;
+    if (g == 0) Qs[4 * kLd + col] = l1;
+    __syncthreads();
+#pragma unroll
+    for (int ib = 0; ib < 2; ib++) wgrad(gW1[ib], Ps + 16 * w * kLd, Qs + 16 * ib * kLd);
+    bgrad(gb1, Ps + 16 * w * kLd);
+    // dZ0 = (W1^T dZ1)(h0 inputs) (1 - h0^2)
+    d0 = zero;
+#pragma unroll
+    for (int o = 0; o < 4; o++)
+#pragma unroll
+      for (int jj = 0; jj < 4; jj++)
+        d0 = mm(W1s[(16 * o + 4 * g + jj) * kIn1 + kLam + c], d1[o][jj], d0);
+#pragma unroll
+    for (int jj = 0; jj < 4; jj++) d0[jj] *= 1.f - h0[jj] * h0[jj];
+    __syncthreads();
+    put(Ps, &d0, 1);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+      if (i < 2 || w == 0) wgrad(gW0[i], Ps, X0s + 16 * (w + 4 * i) * kLd);
+    bgrad(gb0, Ps);
+    __syncthreads();  // X0s, Ts and taus are refilled by the next tile
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-// dZp[b][i] = (sum_o dZ[b][o] W[o][i0 + i]) (1 - Xp[b][xo + i]^2), i < ni:
-// the pre-activation gradient of the previous (tanh) layer
-__global__ void __launch_bounds__(256)
-    k_dense_bwd_data(const float* __restrict__ dZ, int O, const float* __restrict__ W, int I, int i0, int ni,
-                     const float* __restrict__ Xp, int ldx, int xo, float* __restrict__ dZp, int B) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B * ni) return;
-  const int b = t / ni, i = t % ni;
-  float acc = 0.f;
-  for (int o = 0; o < O; o++) acc = fmaf(dZ[(size_t)b * O + o], W[(size_t)o * I + i0 + i], acc);
-  const float x = Xp[(size_t)b * ldx + xo + i];
-  dZp[(size_t)b * ni + i] = acc * (1.f - x * x);
-}
-
-// part[c][o][i] = sum over samples b of chunk c of dZ[b][o] X[b][xo + i]
-// (i < I), part[c][o][I] = sum dZ[b][o]; grid (ceil(O (I + 1) / 256), chunks)
-__global__ void __launch_bounds__(256)
-    k_dense_bwd_w(const float* __restrict__ dZ, int O, const float* __restrict__ X, int ldx, int xo, int I, int B,
-                  int chunk, float* __restrict__ part) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int per = O * (I + 1);
-  if (t >= per) return;
-  const int o = t / (I + 1), i = t % (I + 1);
-  const int b0 = blockIdx.y * chunk, b1 = min(B, b0 + chunk);
-  float acc = 0.f;
-  if (i < I) {
-    for (int b = b0; b < b1; b++) acc = fmaf(dZ[(size_t)b * O + o], X[(size_t)b * ldx + xo + i], acc);
-  } else {
-    for (int b = b0; b < b1; b++) acc += dZ[(size_t)b * O + o];
+  // the partial sums in the layout of theta: D rows o, column i
+  float* row = part + (size_t)blockIdx.x * kParams;
+#pragma unroll
+  for (int jj = 0; jj < 4; jj++) {
+    const int o = 16 * w + 4 * g + jj;
+#pragma unroll
+    for (int ib = 0; ib < 4; ib++) {
+      row[oW2 + o * kHid + 16 * ib + c] = gW2[ib][jj];
+      row[oW3 + o * kHid + 16 * ib + c] = gW3[ib][jj];
+    }
+#pragma unroll
+    for (int ib = 0; ib < 2; ib++)
+      if (16 * ib + c < kIn1) row[oW1 + o * kIn1 + 16 * ib + c] = gW1[ib][jj];
+    if (g == 0) row[oW4 + jj * kHid + 16 * w + c] = gW4[jj];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const int k = 16 * (w + 4 * i) + c;
+      if ((i < 2 || w == 0) && k < kIn0) row[oW0 + (4 * g + jj) * kIn0 + k] = gW0[i][jj];
+    }
   }
-  part[(size_t)blockIdx.y * per + t] = acc;
+  auto rows = [](float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+  };
+  const float s0 = rows(gb0), s1 = rows(gb1), s2 = rows(gb2), s3 = rows(gb3), s4 = rows(gb4);
+  if (g == 0) {
+    row[ob1 + 16 * w + c] = s1;
+    row[ob2 + 16 * w + c] = s2;
+    row[ob3 + 16 * w + c] = s3;
+    if (w == 0) row[ob0 + c] = s0;
+    if (w == 0 && c < kBasis) row[ob4 + c] = s4;
+  }
+  if (lane == 0) red[w] = lsum;
+  __syncthreads();
+  if (tid == 0) lpart[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// grad[oW + o I + i] = sum_c part[c][o][i], grad[ob + o] = sum_c part[c][o][I]
+// grad = the sum of the nrow partial rows (FP64, in a fixed order: four
+// interleaved sums per parameter, then those four), and with an Adam state the
+// update of theta (Kingma & Ba, Algorithm 1, the bias corrections c1 = 1/(1 -
+// b1^t) and c2 = 1/(1 - b2^t) from the host).  The last work-group folds the
+// loss: loss[0] = scale sum lpart.
+struct Adam {
+  float *th, *m, *v;
+  float lr, b1, b2, eps, c1, c2;
+};
 __global__ void __launch_bounds__(256)
-    k_fold(const float* __restrict__ part, int O, int I, int nchunk, float* __restrict__ grad, int oW, int ob) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int per = O * (I + 1);
-  if (t >= per) return;
+    k_train_fold(const float* __restrict__ part, int nrow, const double* __restrict__ lpart, double scale,
+                 float* __restrict__ grad, double* __restrict__ loss, Adam ad) {
+  __shared__ double red[256];
+  const int tid = threadIdx.x;
+  if (blockIdx.x == gridDim.x - 1) {
+    double l = 0.0;
+    for (int i = tid; i < nrow; i += 256) l += lpart[i];
+    red[tid] = l;
+    __syncthreads();
+    for (int h = 128; h > 0; h >>= 1) {
+      if (tid < h) red[tid] += red[tid + h];
+      __syncthreads();
+    }
+    if (tid == 0) loss[0] = red[0] * scale;
+    return;
+  }
+  const int p = blockIdx.x * 64 + (tid & 63), q = tid >> 6;
   double s = 0.0;
-  for (int c = 0; c < nchunk; c++) s += (double)part[(size_t)c * per + t];
-  const int o = t / (I + 1), i = t % (I + 1);
-  if (i < I) grad[oW + o * I + i] = (float)s;
-  else grad[ob + o] = (float)s;
-}
-
-// Adam (Kingma & Ba, Algorithm 1) with the bias corrections c1 = 1/(1 - b1^t),
-// c2 = 1/(1 - b2^t) from the host
-__global__ void __launch_bounds__(256)
-    k_adam(float* __restrict__ th, float* __restrict__ m, float* __restrict__ v, const float* __restrict__ g, int np,
-           float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  th[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+  if (p < kParams) {
+#pragma unroll 8
+    for (int r = q; r < nrow; r += 4) s += (double)part[(size_t)r * kParams + p];
+  }
+  red[tid] = s;
+  __syncthreads();
+  if (q != 0 || p >= kParams) return;
+  const float gi = (float)((red[tid] + red[tid + 64]) + (red[tid + 128] + red[tid + 192]));
+  grad[p] = gi;
+  if (ad.th) {
+    const float mi = ad.b1 * ad.m[p] + (1.f - ad.b1) * gi;
+    const float vi = ad.b2 * ad.v[p] + (1.f - ad.b2) * gi * gi;
+    ad.m[p] = mi;
+    ad.v[p] = vi;
+    ad.th[p] -= ad.lr * (mi * ad.c1) / (sqrtf(vi * ad.c2) + ad.eps);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -461,7 +693,6 @@ __global__ void __launch_bounds__(256)
 // accumulators' initial values.  Bias and tanh are FP32.
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 4;  // waves per work-group
 
@@ -770,58 +1001,22 @@ void launch_target_norm(hipStream_t st, const float* tau_s, size_t P, int nsnap,
   hipLaunchKernelGGL(k_target_norm, dim3(1024), dim3(256), 0, st, tau_s, P, nsnap, part);
 }
 
-// One minibatch: gather, forward, loss, backward into grad (kParams floats);
-// the loss partial sums (blocks(B) doubles) into lpart.  w = the work arrays.
-void launch_train_batch(hipStream_t st, const Work& w, const float* theta, const float* lam_s, const float* T_s,
-                        const float* tau_s, int n, int nsnap, uint64_t base, int B, float inv, float* grad,
-                        double* lpart) {
-  const dim3 blk(256);
-  hipLaunchKernelGGL(k_gather, dim3(blocks(B)), blk, 0, st, lam_s, T_s, tau_s, n, nsnap, base, B, w.X0, w.X1, w.Tb,
-                     w.taub);
-  // forward
-  hipLaunchKernelGGL(k_dense_fwd<true>, dim3(blocks((size_t)B * kConv)), blk, 0, st, w.X0, kIn0, 0, theta + oW0,
-                     theta + ob0, kIn0, kConv, w.X1, kIn1, kLam, B);
-  hipLaunchKernelGGL(k_dense_fwd<true>, dim3(blocks((size_t)B * kHid)), blk, 0, st, w.X1, kIn1, 0, theta + oW1,
-                     theta + ob1, kIn1, kHid, w.H1, kHid, 0, B);
-  hipLaunchKernelGGL(k_dense_fwd<true>, dim3(blocks((size_t)B * kHid)), blk, 0, st, w.H1, kHid, 0, theta + oW2,
-                     theta + ob2, kHid, kHid, w.H2, kHid, 0, B);
-  hipLaunchKernelGGL(k_dense_fwd<true>, dim3(blocks((size_t)B * kHid)), blk, 0, st, w.H2, kHid, 0, theta + oW3,
-                     theta + ob3, kHid, kHid, w.H3, kHid, 0, B);
-  hipLaunchKernelGGL(k_dense_fwd<false>, dim3(blocks((size_t)B * kBasis)), blk, 0, st, w.H3, kHid, 0, theta + oW4,
-                     theta + ob4, kHid, kBasis, w.G, kBasis, 0, B);
-  hipLaunchKernelGGL(k_loss, dim3(blocks(B)), blk, 0, st, w.G, w.Tb, w.taub, B, inv, w.dG, lpart);
-  // backward: pre-activation gradients layer by layer
-  hipLaunchKernelGGL(k_dense_bwd_data, dim3(blocks((size_t)B * kHid)), blk, 0, st, w.dG, kBasis, theta + oW4, kHid,
-                     0, kHid, w.H3, kHid, 0, w.D3, B);
-  hipLaunchKernelGGL(k_dense_bwd_data, dim3(blocks((size_t)B * kHid)), blk, 0, st, w.D3, kHid, theta + oW3, kHid, 0,
-                     kHid, w.H2, kHid, 0, w.D2, B);
-  hipLaunchKernelGGL(k_dense_bwd_data, dim3(blocks((size_t)B * kHid)), blk, 0, st, w.D2, kHid, theta + oW2, kHid, 0,
-                     kHid, w.H1, kHid, 0, w.D1, B);
-  hipLaunchKernelGGL(k_dense_bwd_data, dim3(blocks((size_t)B * kConv)), blk, 0, st, w.D1, kHid, theta + oW1, kIn1,
-                     kLam, kConv, w.X1, kIn1, kLam, w.D0, B);
-  // weight gradients: chunked sums, folded in chunk order
-  const int chunk = kChunk, nch = (B + chunk - 1) / chunk;
-  struct L {
-    const float* dZ;
-    int O;
-    const float* X;
-    int ldx, I, oW, ob;
-  } layers[5] = {{w.dG, kBasis, w.H3, kHid, kHid, oW4, ob4},
-                 {w.D3, kHid, w.H2, kHid, kHid, oW3, ob3},
-                 {w.D2, kHid, w.H1, kHid, kHid, oW2, ob2},
-                 {w.D1, kHid, w.X1, kIn1, kIn1, oW1, ob1},
-                 {w.D0, kConv, w.X0, kIn0, kIn0, oW0, ob0}};
-  for (const L& l : layers) {
-    const int per = l.O * (l.I + 1);
-    hipLaunchKernelGGL(k_dense_bwd_w, dim3(blocks(per), nch), blk, 0, st, l.dZ, l.O, l.X, l.ldx, 0, l.I, B, chunk,
-                       w.part);
-    hipLaunchKernelGGL(k_fold, dim3(blocks(per)), blk, 0, st, w.part, l.O, l.I, nch, grad, l.oW, l.ob);
-  }
-}
-
-void launch_adam(hipStream_t st, float* th, float* m, float* v, const float* g, float lr, float c1, float c2) {
-  hipLaunchKernelGGL(k_adam, dim3(blocks(kParams)), dim3(256), 0, st, th, m, v, g, kParams, lr, 0.9f, 0.999f, 1e-8f,
-                     c1, c2);
+// One minibatch: the partial rows (train_rows(B) of kParams floats) into part
+// and the loss partial sums into lpart, then their fold into grad and loss
+// (scale: of the loss), and with t > 0 Adam step t of learning rate lr on
+// theta and its moments.
+void launch_train_batch(hipStream_t st, float* theta, const float* lam_s, const float* T_s, const float* tau_s, int n,
+                        int nsnap, uint64_t base, int B, float inv, float* part, double* lpart, double scale,
+                        float* grad, double* loss, float* m, float* v, float lr, long long t) {
+  const int rows = train_rows(B);
+  hipLaunchKernelGGL(k_train, dim3(rows), dim3(256), 0, st, lam_s, T_s, tau_s, n, nsnap, base, B, inv, theta, part,
+                     lpart);
+  Adam ad = {nullptr, nullptr, nullptr, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (t > 0)
+    ad = {theta, m, v, lr, 0.9f, 0.999f, 1e-8f, (float)(1.0 / (1.0 - std::pow(0.9, (double)t))),
+          (float)(1.0 / (1.0 - std::pow(0.999, (double)t)))};
+  hipLaunchKernelGGL(k_train_fold, dim3((kParams + 63) / 64 + 1), dim3(256), 0, st, part, rows, lpart, scale, grad,
+                     loss, ad);
 }
 
 }  // namespace sgs

@@ -154,6 +154,36 @@ def test_minibatch_gradient_matches_oracle(O, P):
         off += cnt
 
 
+@pytest.mark.parametrize("B", [1, 63, 65, 16385])
+def test_minibatch_gradient_tile_edges(O, P, B):
+    """a lone point, a tile of 64 points less one and one more, and one point
+    more than a tile for each of the 256 work-groups; the tolerances are those
+    of the gradient test above (FP32 sums of up to 135 terms through five
+    layers: about 1e-5 of the gradient, a block's smallest entries more)"""
+    print("[gpu case] sgs gradient tiles", B, flush=True)
+    n, nsnap, seed, step = 32, 2, 5, 3
+    m, lam_s, T_s, tau_s = _store(O, P, n, nsnap, 61)
+    theta = _theta(7)
+    try:
+        sigma2 = m.target_scale()
+        m.set_params(theta)
+        grad, loss = m.gradient(B, seed, step, sigma2)
+        again, loss2 = m.gradient(B, seed, step, sigma2)
+    finally:
+        m.close()
+    idx = SG.sample_points(seed, step, B, nsnap, n ** 3)
+    X0, lam_pt, T, tau = SG.batch_arrays(lam_s, T_s.reshape(nsnap, 4, 6, n, n, n), tau_s, idx)
+    L, g = SG.loss_and_grad(theta.astype(np.float64), X0, lam_pt, T, tau, sigma2)
+    assert np.array_equal(grad, again) and loss == loss2
+    assert abs(loss - L) <= 1e-5 * L
+    assert rel(grad, g) < 1e-4
+    off = 0
+    for name, shape in SG.PARAM_SHAPES:
+        cnt = int(np.prod(shape))
+        assert rel(grad[off:off + cnt], g[off:off + cnt]) < 1e-3, name
+        off += cnt
+
+
 def test_adam_step_matches_oracle(O, P):
     print("[gpu case] sgs adam", flush=True)
     n, nsnap, B, seed, lr = 32, 2, 1024, 9, 1e-3
