@@ -223,8 +223,8 @@ int psdns_shell_stats_noalloc(psdns_ctx *c, double *ek, double *dk, int nshell, 
  * un (on the mask, unshifted grid) in physical space, dudx[m-1] and
  * dwdz[m-1] = sum of the m-th power over the grid / (nx ny nz), m = 1..8,
  * FP64 sums.  Skewness = [2] / [1]^1.5, flatness = [3] / [1]^2 (the
- * normalised moments of vgmomt.f:152-156).  Uses the u slots 4 and 5
- * (1-based) and the physical array ux(1:2) as work space. */
+ * normalised moments of vgmomt.f:152-156).  Overwrites the transforms' work
+ * arrays. */
 int psdns_vg_moments(psdns_ctx *c, double *dudx, double *dwdz);
 
 /* Random-phase solenoidal initial field on the device (homogeneous/field.f:

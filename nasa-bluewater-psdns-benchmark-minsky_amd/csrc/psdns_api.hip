@@ -1004,18 +1004,10 @@ int psdns_vg_moments(psdns_ctx* c, double* dudx, double* dwdz) {
   if (int rc = ready_clobber(c)) return rc;
   if (!dudx || !dwdz) return fail(PSDNS_EINVAL, "null moment arrays");
   int rc;
-  if ((rc = ensure_ux(c))) return rc;
-  // i kx u and i kz w into the u slots 3 and 4, inverse transform into ux
-  // slots 0 and 1 (vgmomt's utx), power sums in FP64
-  void* d = (char*)c->d_u + 3 * c->csize() * c->cyl_elems();
-  psdns::launch_vg_deriv(c->c, d);
-  Ctx k = c->c;
-  k.u = d;
-  if (psdns::launch_pass(k, Pass::YInvKx, 2, 0) || psdns::launch_pass(k, Pass::ZInv, 2, 0) ||
-      psdns::launch_pass(k, Pass::XC2R, 2, 0))
-    return fail(PSDNS_EINVAL, "unsupported grid n = %d", c->n);
-  HIPCHK(hipMemsetAsync(c->d_red, 0, sizeof(double) * 16, c->c.stream));
-  psdns::launch_moments(c->c, c->d_red);
+  // i kx u and i kz w of un formed on load by the inverse y pass, the power
+  // sums in FP64 taken by the x pass (the physical fields are not stored)
+  if ((rc = pass(c, Pass::YInvGrad, 2)) || (rc = pass(c, Pass::ZInv, 2))) return rc;
+  if (psdns::launch_x_moments(c->c, c->d_red)) return fail(PSDNS_EINVAL, "unsupported grid n = %d", c->n);
   HIPCHK(hipGetLastError());
   double sums[16];
   HIPCHK(hipMemcpyAsync(sums, c->d_red, sizeof sums, hipMemcpyDeviceToHost, c->c.stream));

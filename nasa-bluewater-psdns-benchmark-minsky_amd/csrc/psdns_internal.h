@@ -79,6 +79,7 @@ enum class Pass {
   YInvPhase,  // phase1 + y c2c +i, u -> yw (arg: number of variables)
   YInvKx,     // kxtran: zero y Nyquist + y c2c +i, u -> yw
   YInvPlain,  // y c2c +i, u -> yw
+  YInvGrad,   // du/dx, dw/dz of un on the mask + y c2c +i, un -> yw (two variables)
   ZInv,       // gather yw + z c2c +i -> xi (args: number of variables; source 0 W1, 1 y-blocked yw in u, 2 a scalar's two gradient slots in W1 -> three xi slots)
   XC2R,       // gather xi + x c2r -> physical (arg: number of variables)
   XR2C,       // physical -> x r2c / n (arg: number of variables)
@@ -134,15 +135,14 @@ void launch_shifts(const Ctx& c, double2* s64, void* sr, const double gsh[6]);
 int launch_y_grad(const Ctx& c, const void* phi, void* yw);
 int launch_sc_update(const Ctx& c, int stage, void* u, void* un, const void* tr, double dt2, double rpr,
                      double* dif, void* u1 = nullptr);
-// velocity-gradient moments: i kx u, i kz w of un into cylinder slots d[0..1];
-// power sums 1..8 of ux slots 0 and 1 added into d_out[16]
-void launch_vg_deriv(const Ctx& c, void* d);
+// velocity-gradient moments: the x c2r of xi slots 0 and 1 and the FP64 sums
+// of the powers 1..8 of its values, out[16] (X is overwritten)
+int launch_x_moments(const Ctx& c, double* out);
 // EPFOR forcing increments on u (and un): mode 1 proc4a/advanc_1 (sphere,
 // per-entry tally terms[3 nlist], then efkz[3 nxh] folded in list order),
 // 2 proc4b, 3 advanc_2/advanc_3; list entries (a, y, for index, shell | 0)
 void launch_epfor(const Ctx& c, int mode, const int4* list, int nlist, const double2* forc, int fstride,
                   double* terms, double* efkz);
-void launch_moments(const Ctx& c, double* d_out);
 // Lagrangian particles: the spline's shift tables (stage-1 shifts times
 // the spline factors, sr layout, state precision, at sr) for the inverse y
 // pass's phase mode, the interpolation of the coefficients in ux[0..2] at

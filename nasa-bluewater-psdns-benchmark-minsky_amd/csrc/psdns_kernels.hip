@@ -258,6 +258,9 @@ struct BufView {
 //         overwrites u in place).
 // MODE 1: kxtran (kxtran.f:36): zero the y Nyquist row.
 // MODE 2: plain inverse transform (itransform_vel on an already shifted u).
+// MODE 3: du/dx and dw/dz of the state (vgmomt.f:68-143): variable 0 is i kx
+//         times slot 0, variable 1 i kz times slot 2, on the mask (kx and kz
+//         are constant along a column).
 // Then y c2c +i (kxcomm1_clean.f:118).  A tile is B consecutive columns of
 // one variable; loads and stores both run along y (natural mapping), so the
 // pass streams whole columns in and out.  The transpose towards z lines
@@ -293,7 +296,7 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
   // are applied in finish, so that the next tile's loads stay in flight
   auto load = [&](Regs<R, E>& b, int t, bool valid) {
     const int var = t / nab, a0 = (t % nab) * B;
-    const BufView<R> src(u + ((size_t)var * g.na + a0) * N, valid ? kOob : 0u);
+    const BufView<R> src(u + ((size_t)(MODE == 3 ? 2 * var : var) * g.na + a0) * N, valid ? kOob : 0u);
     // lines past the last column re-read the last column (never stored), so
     // that no branch depends on the tile
     const int li = line_of(), q = opaque(io.q);
@@ -303,7 +306,7 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
     for (int j = 0; j < E; j++) {
       const int y = q + T * j;
       bool keep = true;
-      if constexpr (MODE == 0) keep = in_mask(x, kwave(y, N), kz, y, z, N);
+      if constexpr (MODE == 0 || MODE == 3) keep = in_mask(x, kwave(y, N), kz, y, z, N);
       if constexpr (MODE == 1) keep = y != N / 2;
       b.v[j] = src.load(keep ? ((unsigned)lc * N + y) * (unsigned)sizeof(C<R>) : kOob);
     }
@@ -316,6 +319,13 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
       const C<R> sxz = cmul(sr[colx[a]], sr[g.nxh + N + colz[a]]);
 #pragma unroll
       for (int j = 0; j < E; j++) b.v[j] = cmul(b.v[j], cmul(ssy[q + T * j], sxz));
+    }
+    if constexpr (MODE == 3) {
+      const int li = line_of();
+      const int a = a0 + li < g.na ? a0 + li : g.na - 1;
+      const R k = (R)(var == 0 ? colx[a] : kwave(colz[a], N));
+#pragma unroll
+      for (int j = 0; j < E; j++) b.v[j] = {-k * b.v[j].y, k * b.v[j].x};
     }
     F::template run<false, false, false, false>(b.v, lds, io, io, stw);
     const int li = line_of(), q = opaque(io.q);
@@ -720,23 +730,111 @@ struct XPass {
   }
 };
 
-// inverse x pass alone: xi (nv variables) -> physical ux
-template <typename R, int N>
+// The wave's sums over its lanes, by pairs (a fixed order).
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  return v;
+}
+
+// inverse x pass alone, variable blockIdx.y of xi.  MOM false: -> physical ux.
+// MOM true (velocity-gradient moments, vgmomt.f:134-143): the physical values
+// f are not stored; part[(var gridDim.x + b) 8 + m - 1] = the work-group's sum
+// of f^m, m = 1..8, in FP64 (each thread over its points, then the waves'
+// lanes, then the waves, in fixed orders).
+// Persistent over tiles and staged as k_x_fused: the copy of the next tile's
+// rows into LDS runs under the transform of the current one.  Three variables
+// at 512^3 FP32: 760 us with one tile per work-group and gathered register
+// loads, 575 us this way (3.1 GB, 5.4 TB/s: the copy rate).  The moments of two
+// variables there: 339 us, bound by VALU (the transform and 12 FP64 operations
+// per value), against 508 us for the transform, 1016 us for a kernel over the
+// stored fields with one FP64 atomic per wave and power, and 212 us for one
+// that formed the derivatives (now on load in the y pass).
+template <typename R, int N, bool MOM>
 __global__ void __launch_bounds__((XPass<R, N>::NT))
-    k_x_c2r(const C<R>* __restrict__ xi, R* __restrict__ ux, Geo g, const C<R>* __restrict__ tw) {
+    k_x_c2r(const C<R>* __restrict__ xi, R* __restrict__ ux, Geo g, const C<R>* __restrict__ tw,
+            double* __restrict__ part) {
   using X = XPass<R, N>;
+  constexpr int E = X::E, B = X::B, NZB = N / B;
   __shared__ R lds[X::kLdsReals];
   __shared__ C<R> stw[X::kTw], xtw[X::M];
+  __shared__ __attribute__((aligned(16))) C<R> S[X::M * B];
   X::fill(stw, xtw, tw);
-  const int2 blk = xcd_block2();
-  const int var = blk.y;
-  const int y = blk.x / (N / X::B), z0 = (blk.x % (N / X::B)) * X::B;
-  C<R> v[X::E];
-  X::c2r(v, xi, var, y, z0, g, lds, stw, xtw);
-  const int line = X::FI::natural_line(threadIdx.x), q = threadIdx.x % X::T;
-  C<R>* dst = reinterpret_cast<C<R>*>(ux + (((size_t)var * N + y) * N + z0 + line) * N);
+  const int var = blockIdx.y;
+  const TileWalk w = tile_walk(N * NZB);
+  double s[MOM ? 8 : 1];
 #pragma unroll
-  for (int j = 0; j < X::E; j++) dst[q + X::T * j] = v[j];
+  for (int m = 0; m < (MOM ? 8 : 1); m++) s[m] = 0.0;
+  int t = w.t;
+  if (t < w.end) {
+    X::stage_load(S, xi, var, t / NZB, (t % NZB) * B, g, true);
+    for (;;) {
+      const int y = t / NZB, z0 = (t % NZB) * B, tn = t + w.step;
+      C<R> v[E];
+      X::stage_publish();
+      X::c2r_staged_pre(v, S, xtw);
+      if (tn < w.end) X::stage_load(S, xi, var, tn / NZB, (tn % NZB) * B, g, true);
+      X::c2r_staged_fft(v, lds, stw);
+      if constexpr (MOM) {
+#pragma unroll
+        for (int j = 0; j < E; j++) {
+          const double ab[2] = {(double)v[j].x, (double)v[j].y};
+#pragma unroll
+          for (int i = 0; i < 2; i++) {
+            // three products and the rest in fused multiply-adds (a product
+            // and a sum per power, 15 operations: 351 against 339 us at 512^3)
+            const double a = ab[i], a2 = a * a, a3 = a2 * a, a4 = a2 * a2;
+            s[0] += a;
+            s[1] = fma(a, a, s[1]);
+            s[2] = fma(a2, a, s[2]);
+            s[3] = fma(a2, a2, s[3]);
+            s[4] = fma(a4, a, s[4]);
+            s[5] = fma(a4, a2, s[5]);
+            s[6] = fma(a4, a3, s[6]);
+            s[7] = fma(a4, a4, s[7]);
+          }
+        }
+      } else {
+        const int tid = opaque(threadIdx.x), line = X::FI::natural_line(tid), q = (int)((unsigned)tid % X::T);
+        C<R>* dst = reinterpret_cast<C<R>*>(ux + (((size_t)var * N + y) * N + z0 + line) * N);
+#pragma unroll
+        for (int j = 0; j < E; j++) dst[q + X::T * j] = v[j];
+      }
+      if (tn >= w.end) break;
+      t = tn;
+    }
+  }
+  if constexpr (MOM) {
+    constexpr int NW = (X::NT + 63) / 64;
+    __shared__ double red[NW][8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const double v = wave_sum(s[m]);
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][m] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 8) {
+      double v = 0.0;
+      for (int i = 0; i < NW; i++) v += red[i][threadIdx.x];
+      part[((size_t)var * gridDim.x + blockIdx.x) * 8 + threadIdx.x] = v;
+    }
+  }
+}
+
+// out[8 var + m - 1] = the sum of the nb partial rows of variable blockIdx.x
+__global__ void __launch_bounds__(256) k_moments_fold(const double* __restrict__ part, int nb, double* __restrict__ out) {
+  __shared__ double red[256];
+  const int m = threadIdx.x & 7, q = threadIdx.x >> 3;
+  const double* p = part + (size_t)blockIdx.x * nb * 8 + m;
+  double v = 0.0;
+#pragma unroll 4
+  for (int i = q; i < nb; i += 32) v += p[(size_t)i * 8];
+  red[threadIdx.x] = v;
+  __syncthreads();
+  if (q == 0) {
+    double r = 0.0;
+    for (int i = 0; i < 32; i++) r += red[8 * i + m];
+    out[8 * blockIdx.x + m] = r;
+  }
 }
 
 // forward x pass alone: physical ux (nv variables) -> X, x 1/n
@@ -2037,49 +2135,6 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T))
 }
 
 // ---------------------------------------------------------------------------
-// Velocity-gradient moments (vgmomt.f:68-156): du/dx and dw/dz in physical
-// space, from i kx u and i kz w of the state on the mask (k_vg_deriv, into
-// two cylinder slots for the inverse transform), then the sums of their
-// powers 1..8 over the grid in FP64 (k_moments: out[8 v + m - 1] += sum
-// f_v^m for the two fields v = 0, 1).
-// ---------------------------------------------------------------------------
-template <typename R>
-__global__ void __launch_bounds__(256) k_vg_deriv(const C<R>* __restrict__ un, C<R>* __restrict__ d, Geo g) {
-  const size_t tot = (size_t)g.na * g.n;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < tot; i += (size_t)gridDim.x * blockDim.x) {
-    const Pt p = point(i, g);
-    const C<R> a = un[i], w = un[2 * tot + i];
-    d[i] = p.m ? C<R>{-(R)p.x * a.y, (R)p.x * a.x} : C<R>{0, 0};
-    d[tot + i] = p.m ? C<R>{-(R)p.kz * w.y, (R)p.kz * w.x} : C<R>{0, 0};
-  }
-}
-
-template <typename R>
-__global__ void __launch_bounds__(256) k_moments(const R* __restrict__ f, size_t n3, double* __restrict__ out) {
-  double s[16];
-#pragma unroll
-  for (int m = 0; m < 16; m++) s[m] = 0;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n3; i += (size_t)gridDim.x * blockDim.x) {
-#pragma unroll
-    for (int v = 0; v < 2; v++) {
-      const double a = (double)f[v * n3 + i];
-      double pw = a;
-#pragma unroll
-      for (int m = 0; m < 8; m++) {
-        s[8 * v + m] += pw;
-        pw *= a;
-      }
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < 16; m++) {
-    double t = s[m];
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off);
-    if ((threadIdx.x & 63) == 0) atomicAdd(out + m, t);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Lagrangian particles (hooks/LAG_LOCAL).
 // Spline coefficients (spxyz_m.f: periodic (1,4,1) solves along x, z and y,
 // the z solve on 216 times the data, splz.f:22-28) of the velocity on the
@@ -2404,6 +2459,11 @@ struct Launch {
       static const unsigned grid = persistent_grid((const void*)kern, NT);
       hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(NT), 0, c.stream, (const CR*)c.u, (CR*)c.w1, c.geo, sr,
                          (const CR*)c.tw, nv, c.geo.colx, c.geo.colz);
+    } else if (mode == 3) {
+      const auto kern = k_y_inv<R, N, 3>;
+      static const unsigned grid = persistent_grid((const void*)kern, NT);
+      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(NT), 0, c.stream, (const CR*)c.un, (CR*)c.w1, c.geo, sr,
+                         (const CR*)c.tw, nv, c.geo.colx, c.geo.colz);
     } else {
       const auto kern = k_y_inv<R, N, 2>;
       static const unsigned grid = persistent_grid((const void*)kern, NT);
@@ -2437,9 +2497,21 @@ struct Launch {
   }
   static void x_c2r(const Ctx& c, int nv) {
     using X = XPass<R, N>;
-    dim3 grid(N * (N / X::B), nv);
-    hipLaunchKernelGGL((k_x_c2r<R, N>), grid, dim3(X::NT), 0, c.stream, (const CR*)c.xi, (R*)c.ux, c.geo,
-                       (const CR*)c.tw);
+    const auto kern = k_x_c2r<R, N, false>;
+    static const unsigned grid = persistent_grid((const void*)kern, X::NT);
+    hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, N * (N / X::B)), nv), dim3(X::NT), 0, c.stream, (const CR*)c.xi,
+                       (R*)c.ux, c.geo, (const CR*)c.tw, (double*)nullptr);
+  }
+  // the moments of the variables 0 and 1 of xi into out[16]; X holds the
+  // partial rows
+  static void x_moments(const Ctx& c, double* out) {
+    using X = XPass<R, N>;
+    const auto kern = k_x_c2r<R, N, true>;
+    static const unsigned full = persistent_grid((const void*)kern, X::NT, 4);
+    const unsigned grid = tiles_grid(full, N * (N / X::B));
+    hipLaunchKernelGGL(kern, dim3(grid, 2), dim3(X::NT), 0, c.stream, (const CR*)c.xi, (R*)nullptr, c.geo,
+                       (const CR*)c.tw, (double*)c.xs);
+    hipLaunchKernelGGL(k_moments_fold, dim3(2), dim3(256), 0, c.stream, (const double*)c.xs, (int)grid, out);
   }
   static void x_r2c(const Ctx& c, int nv) {
     using X = XPass<R, N>;
@@ -2589,18 +2661,6 @@ struct LaunchP {
     hipLaunchKernelGGL((k_consym<R>), dim3(grid1d((size_t)c.geo.n * c.geo.n, 256)), dim3(256), 0, c.stream,
                        (CR*)c.un, c.geo, d_colz0);
   }
-  // i kx u, i kz w of un into d[0..1] (cylinder slots)
-  static void vg_deriv(const Ctx& c, void* d) {
-    size_t tot = (size_t)c.geo.na * c.geo.n;
-    hipLaunchKernelGGL((k_vg_deriv<R>), dim3(grid1d(tot, 256 * 4)), dim3(256), 0, c.stream, (const CR*)c.un,
-                       (CR*)d, c.geo);
-  }
-  // power sums of physical slots 0 and 1 of ux (a fixed grid: few atomics)
-  static void moments(const Ctx& c, double* d_out) {
-    const size_t n3 = (size_t)c.geo.n * c.geo.n * c.geo.n;
-    hipLaunchKernelGGL((k_moments<R>), dim3(grid1d(n3, 256 * 8) < 2048u ? grid1d(n3, 256 * 8) : 2048u), dim3(256), 0, c.stream,
-                       (const R*)c.ux, n3, d_out);
-  }
   static void scale(const Ctx& c, void* p, size_t cnt, double s) {
     hipLaunchKernelGGL((k_scale<R>), dim3(grid1d(cnt, 256 * 4)), dim3(256), 0, c.stream, (CR*)p, cnt, s);
   }
@@ -2615,6 +2675,7 @@ static void run_pass(const Ctx& c, Pass p, int a0, int a1) {
     case Pass::YInvPhase: Launch<R, N>::y_inv(c, a0, 0); break;
     case Pass::YInvKx: Launch<R, N>::y_inv(c, a0, 1); break;
     case Pass::YInvPlain: Launch<R, N>::y_inv(c, a0, 2); break;
+    case Pass::YInvGrad: Launch<R, N>::y_inv(c, 2, 3); break;
     case Pass::ZInv: Launch<R, N>::z_inv(c, a0, a1); break;
     case Pass::XC2R: Launch<R, N>::x_c2r(c, a0); break;
     case Pass::XR2C: Launch<R, N>::x_r2c(c, a0); break;
@@ -2847,13 +2908,20 @@ void launch_lag_interp(const Ctx& c, double* pp, int np, const double gsh1[3], c
 void launch_lag_advpos(const Ctx& c, double* pp, int np, int pstep, double fact1, double fact2) {
   hipLaunchKernelGGL(k_lag_advpos, dim3((np + 255) / 256), dim3(256), 0, c.stream, pp, np, pstep, fact1, fact2);
 }
-void launch_vg_deriv(const Ctx& c, void* d) {
-  if (c.prec == 8) LaunchP<double>::vg_deriv(c, d);
-  else LaunchP<float>::vg_deriv(c, d);
+template <typename R>
+static int moments_r(const Ctx& c, double* out) {
+  switch (c.geo.n) {
+    case 32: Launch<R, 32>::x_moments(c, out); return 0;
+    case 64: Launch<R, 64>::x_moments(c, out); return 0;
+    case 128: Launch<R, 128>::x_moments(c, out); return 0;
+    case 256: Launch<R, 256>::x_moments(c, out); return 0;
+    case 512: Launch<R, 512>::x_moments(c, out); return 0;
+    case 1024: Launch<R, 1024>::x_moments(c, out); return 0;
+  }
+  return -1;
 }
-void launch_moments(const Ctx& c, double* d_out) {
-  if (c.prec == 8) LaunchP<double>::moments(c, d_out);
-  else LaunchP<float>::moments(c, d_out);
+int launch_x_moments(const Ctx& c, double* out) {
+  return c.prec == 8 ? moments_r<double>(c, out) : moments_r<float>(c, out);
 }
 
 }  // namespace psdns

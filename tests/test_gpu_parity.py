@@ -270,3 +270,23 @@ def test_vg_moments(O, P, ctxs, n, prec):
         scale = np.maximum(np.abs(ref), np.abs(ref[1]) ** (np.arange(1, 9) / 2.0))
         assert np.all(np.abs(got - ref) <= tol * scale), (got, ref)
     assert du[1] > 0 and dw[1] > 0
+
+
+@pytest.mark.parametrize("n,prec", [(32, 4), (256, 4), (256, 8)])
+def test_vg_moments_reproducible(O, P, ctxs, n, prec):
+    """The x pass takes the moments in a fixed order: the same bits twice, for
+    a work-group of half a wavefront (32^3) and one of several tiles (256^3),
+    and the physical fields of kxtran from the same pass match the oracle."""
+    banner("vg_moments twice", n, prec)
+    g, s = O.Grid(n), ctxs(n, prec)
+    u0 = g.field(seed=17 + n)
+    s.put_state(u0)
+    du, dw = s.vg_moments()
+    again = s.vg_moments()
+    assert np.array_equal(du, again[0]) and np.array_equal(dw, again[1])
+    tol = 1e-11 if prec == 8 else 2e-5
+    for got, ref in zip((du, dw), g.vg_moments(u0)):
+        scale = np.maximum(np.abs(ref), np.abs(ref[1]) ** (np.arange(1, 9) / 2.0))
+        assert np.all(np.abs(got - ref) <= tol * scale), (got, ref)
+    s.kxtran(3)
+    assert rel(s.get_field(P.FIELD_UX, 3), g.kxtran(u0, 3)) < (1e-12 if prec == 8 else 3e-6)
