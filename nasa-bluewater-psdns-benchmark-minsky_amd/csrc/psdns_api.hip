@@ -105,10 +105,15 @@ struct psdns_ctx {
   void* d_shiftr = nullptr;    // per stage: sx[nxh] | sy[n] | sz[n], precision prec
   double* d_fac = nullptr;     // xfac[nxh], yfac[n], zfac[n]
   double* h_fac = nullptr;     // pinned host staging of the same, one copy per upload
+  // after the factors in the same pinned allocation, what kernels write to
+  // the host: velmax's bits, then the FEK energies (launch_ek_force)
+  unsigned long long* h_velmax = nullptr;
+  double* h_ek = nullptr;
+  bool velmax_clear = false;   // the velmax slots are zero
   double* d_red = nullptr;     // reductions scratch: [2 + 2*n + n]
   unsigned long long* d_velmax = nullptr;
   int2* d_force = nullptr;
-  double* d_force_terms = nullptr;  // 2 doubles per force-list entry (fixed-order shell sums)
+  double* d_force_terms = nullptr;  // a double and an int per force-list entry (shell sums)
   int force_kfor = -1, nforce = 0;
   double* d_shell_part = nullptr;   // partial rows of psdns_shell_stats, allocated on first use
   double* d_scratch = nullptr;      // device address of `scratch` on dev (psdns_shell_stats_noalloc)
@@ -211,7 +216,7 @@ int ensure_force_list(psdns_ctx* c, int kfor) {
   c->nforce = (int)list.size();
   if (!list.empty()) {
     HIPCHK(hipMalloc(&c->d_force, sizeof(int2) * list.size()));
-    HIPCHK(hipMalloc(&c->d_force_terms, 2 * sizeof(double) * list.size()));
+    HIPCHK(hipMalloc(&c->d_force_terms, (sizeof(double) + sizeof(int)) * list.size()));
     HIPCHK(hipMemcpy(c->d_force, list.data(), sizeof(int2) * list.size(), hipMemcpyHostToDevice));
   }
   c->c.force_list = c->d_force;
@@ -222,28 +227,40 @@ int ensure_force_list(psdns_ctx* c, int kfor) {
 
 // the three arrays go through the pinned staging buffer as one copy; the
 // staging buffer is free again once the stream has passed the copy (every
-// caller synchronises before returning)
-int upload_factors(psdns_ctx* c, const double* xfac, const double* yfac, const double* zfac) {
+// caller synchronises before another one fills it)
+int stage_factors(psdns_ctx* c, const double* xfac, const double* yfac, const double* zfac) {
   if (!xfac || !yfac || !zfac) return fail(PSDNS_EINVAL, "null integrating-factor array");
   std::memcpy(c->h_fac, xfac, sizeof(double) * c->nxh);
   std::memcpy(c->h_fac + c->nxh, yfac, sizeof(double) * c->n);
   std::memcpy(c->h_fac + c->nxh + c->n, zfac, sizeof(double) * c->n);
+  return 0;
+}
+int copy_factors(psdns_ctx* c) {
   HIPCHK(hipMemcpyAsync(c->d_fac, c->h_fac, sizeof(double) * (c->nxh + 2 * (size_t)c->n), hipMemcpyHostToDevice,
                         c->c.stream));
   return 0;
 }
+int upload_factors(psdns_ctx* c, const double* xfac, const double* yfac, const double* zfac) {
+  if (int rc = stage_factors(c, xfac, yfac, zfac)) return rc;
+  return copy_factors(c);
+}
 
 constexpr size_t kVelmaxBytes = sizeof(unsigned long long) * psdns::kVelmaxSlots * psdns::kVelmaxStride;
 
+// before a kernel that takes velmax: the slots are zero (each reduction leaves
+// them so, unless a call failed between the two)
+int clear_velmax(psdns_ctx* c) {
+  if (!c->velmax_clear) HIPCHK(hipMemsetAsync(c->d_velmax, 0, kVelmaxBytes, c->c.stream));
+  c->velmax_clear = false;
+  return 0;
+}
+
 int read_velmax(psdns_ctx* c, double* velmax) {
-  unsigned long long bits = 0;
-  psdns::launch_velmax_reduce(c->c);
+  psdns::launch_velmax_reduce(c->c, c->h_velmax);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(&bits, c->d_velmax, sizeof bits, hipMemcpyDeviceToHost, c->c.stream));
   HIPCHK(hipStreamSynchronize(c->c.stream));
-  double v;
-  std::memcpy(&v, &bits, sizeof v);
-  if (velmax) *velmax = v;
+  c->velmax_clear = true;
+  if (velmax) std::memcpy(velmax, c->h_velmax, sizeof *velmax);
   return 0;
 }
 
@@ -308,7 +325,7 @@ int flush(psdns_ctx* c) {
   if (!c->pending_update) return 0;
   c->pending_update = false;
   int rc;
-  if ((rc = y_update(c, 1, c->pending_norm, false))) return rc;
+  if ((rc = copy_factors(c)) || (rc = y_update(c, 1, c->pending_norm, false))) return rc;
   if ((rc = sync(c))) return rc;
   return add_time(c, 5, 6, kTYUpd, 0);
 }
@@ -531,8 +548,12 @@ int psdns_create(const psdns_params* p, psdns_ctx** out) {
   ALLOC(c->d_shift, sizeof(double2) * 2 * (c->nxh + 2 * n));
   ALLOC(c->d_shiftr, c->csize() * 2 * (c->nxh + 2 * n));
   ALLOC(c->d_fac, sizeof(double) * (c->nxh + 2 * n));
-  if (hipHostMalloc((void**)&c->h_fac, sizeof(double) * (c->nxh + 2 * n), hipHostMallocDefault) != hipSuccess)
+  // one pinned allocation: the factors, then what kernels write to the host
+  if (hipHostMalloc((void**)&c->h_fac, sizeof(double) * (c->nxh + 2 * n + 2 + 2 * psdns::kMaxKfor),
+                    hipHostMallocDefault) != hipSuccess)
     return bail(fail(PSDNS_ENOMEM, "hipHostMalloc of the factor staging buffer failed"));
+  c->h_velmax = (unsigned long long*)(c->h_fac + c->nxh + 2 * n);
+  c->h_ek = (double*)(c->h_velmax + 1);
   ALLOC(c->d_red, sizeof(double) * (2 + 3 * (size_t)n + 64));
   ALLOC(c->d_velmax, kVelmaxBytes);
   CHK(hipMemcpy(c->d_colx, c->colx.data(), sizeof(int) * c->na, hipMemcpyHostToDevice));
@@ -678,14 +699,14 @@ int psdns_stage_nonlinear(psdns_ctx* c, int kstep, double* velmax) {
   const bool fused = kstep == 2 && c->pending_update;
   if (fused) {
     c->pending_update = false;
-    if ((rc = y_update(c, 1, c->pending_norm, true))) return rc;
+    if ((rc = copy_factors(c)) || (rc = y_update(c, 1, c->pending_norm, true))) return rc;
   } else if ((rc = flush(c))) {
     return rc;
   }
   // RK4's stages 3 and 4 use the shifts of stages 1 and 2 (shifts.f:133-137:
   // gsh(:,3) = gsh(:,1), gsh(:,4) = gsh(:,2))
   c->c.kstep = (kstep - 1) % 2;
-  if (kstep == 1) HIPCHK(hipMemsetAsync(c->d_velmax, 0, kVelmaxBytes, c->c.stream));
+  if (kstep == 1 && (rc = clear_velmax(c))) return rc;
   if ((rc = mark(c, 0))) return rc;
   if (!fused && kstep == 1 && c->u_stale) {
     // the state is in un only (the last stage-2 update wrote un alone)
@@ -735,21 +756,21 @@ int psdns_stage_update(psdns_ctx* c, int kstep, double dt, const double* xfac, c
     return fail(PSDNS_ESTATE, "stage_update(%d) without a preceding stage_nonlinear(%d)", kstep, kstep);
   if (!(dt > 0.0)) return fail(PSDNS_EINVAL, "dt = %g must be positive", dt);
   int rc;
-  // proc4b (stage 2) has no integrating factors: they are used by stage 1 only
-  if (kstep == 1) {
-    if ((rc = upload_factors(c, xfac, yfac, zfac))) return rc;
-  }
   const double dt2 = dt / 2.0;
   const double norm = dt2 / c->n / c->n;  // wavespace_vel.f:80
+  // proc4b (stage 2) has no integrating factors: they are used by stage 1 only
+  if (kstep == 1 && (rc = stage_factors(c, xfac, yfac, zfac))) return rc;
   c->last_nonlinear = 0;
   if (kstep == 1 && c->nc == 0 && !forcing) {
-    // deferred (the factors are on the device already); proc4a zeroes
-    // efkz when forcing is on (proc4a.f:66)
-    if (c->epf_kfor) HIPCHK(hipMemsetAsync(c->d_efkz, 0, sizeof(double) * 3 * c->nxh, c->c.stream));
+    // deferred with the factors, which go to the device with the update;
+    // proc4a zeroes efkz when forcing is on (proc4a.f:66)
     c->pending_update = true;
     c->pending_norm = norm;
+    if (!c->epf_kfor) return PSDNS_OK;
+    HIPCHK(hipMemsetAsync(c->d_efkz, 0, sizeof(double) * 3 * c->nxh, c->c.stream));
     return sync(c);
   }
+  if (kstep == 1 && (rc = copy_factors(c))) return rc;
   if (forcing && (rc = upload_forcing(c, forcing))) return rc;
   // stage 2 without EPFOR increments writes un only (proc4b's u = un)
   if ((rc = y_update(c, kstep, norm, false, kstep == 2 && !forcing))) return rc;
@@ -916,34 +937,29 @@ int psdns_ek_shell(psdns_ctx* c, int kfor, double* ek) {
   if (kfor < 1 || kfor > 64 || !ek) return fail(PSDNS_EINVAL, "kfor = %d: need 1..64 and an output array", kfor);
   int rc;
   if ((rc = ensure_force_list(c, kfor))) return rc;
-  psdns::launch_ek_shell(c->c, kfor, c->d_red, c->d_force_terms);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(ek, c->d_red, sizeof(double) * kfor, hipMemcpyDeviceToHost, c->c.stream));
-  return sync(c);
+  psdns::launch_ek_force(c->c, kfor, 0, psdns::EkInf{}, c->d_force_terms, c->d_red, c->h_ek);
+  if ((rc = sync(c))) return rc;
+  std::memcpy(ek, c->h_ek, sizeof(double) * kfor);
+  return PSDNS_OK;
 }
 
 int psdns_ek_force(psdns_ctx* c, int kf_shell, int kfor, const double* ekinf, double* ek_out) {
   if (int rc = ready(c)) return rc;
   if (kf_shell < 1 || kf_shell > kfor || !ekinf)
     return fail(PSDNS_EINVAL, "need 1 <= kf_shell (%d) <= kfor (%d) and ekinf", kf_shell, kfor);
-  std::vector<double> ek(kfor), ratio(kfor, 0.0);
+  if (kfor > psdns::kMaxKfor) return fail(PSDNS_EINVAL, "kfor = %d: need 1..64 and an output array", kfor);
   int rc;
-  if ((rc = psdns_ek_shell(c, kfor, ek.data()))) return rc;
-  // ek_force.f:31-35
-  ratio[0] = 0.0;
-  for (int ik = 2; ik <= kfor; ik++) {
-    if (!(ek[ik - 1] > 0.0)) return fail(PSDNS_EINVAL, "shell %d has no energy to rescale", ik);
-    ratio[ik - 1] = std::sqrt(ekinf[ik - 1] / ek[ik - 1]);
-  }
-  HIPCHK(hipMemcpyAsync(c->d_red + 64, ratio.data(), sizeof(double) * kfor, hipMemcpyHostToDevice, c->c.stream));
-  if (c->nforce) {
-    Ctx k = c->c;
-    if (c->u_stale) k.u = nullptr;  // u does not hold the state: un only
-    psdns::launch_ek_scale(k, kf_shell, c->d_red + 64);
-  }
-  HIPCHK(hipGetLastError());
+  if ((rc = ensure_force_list(c, kfor))) return rc;
+  psdns::EkInf inf{};
+  std::memcpy(inf.e, ekinf, sizeof(double) * kfor);
+  Ctx k = c->c;
+  if (c->u_stale) k.u = nullptr;  // u does not hold the state: un only
+  psdns::launch_ek_force(k, kfor, kf_shell, inf, c->d_force_terms, c->d_red, c->h_ek);
   if ((rc = sync(c))) return rc;
-  if (ek_out) return psdns_ek_shell(c, kfor, ek_out);
+  if (c->h_ek[2 * psdns::kMaxKfor] != 0.0)  // ek_force.f:31-35 divides by every shell 2 .. kfor
+    for (int ik = 2; ik <= kfor; ik++)
+      if (!(c->h_ek[ik - 1] > 0.0)) return fail(PSDNS_EINVAL, "shell %d has no energy to rescale", ik);
+  if (ek_out) std::memcpy(ek_out, c->h_ek + psdns::kMaxKfor, sizeof(double) * kfor);
   return PSDNS_OK;
 }
 
@@ -1110,7 +1126,7 @@ int psdns_realspace_vel(psdns_ctx* c, int rkstep, double* velmax) {
   if (int rc = ready_clobber(c)) return rc;
   int rc;
   if ((rc = ensure_ux(c))) return rc;
-  HIPCHK(hipMemsetAsync(c->d_velmax, 0, kVelmaxBytes, c->c.stream));
+  if (rkstep == 1 && (rc = clear_velmax(c))) return rc;
   psdns::launch_realspace(c->c, rkstep == 1);
   HIPCHK(hipGetLastError());
   if (rkstep == 1) return read_velmax(c, velmax);

@@ -96,18 +96,23 @@ int launch_pass(const Ctx& c, Pass p, int a0, int a1);
 int launch_y_update(const Ctx& c, int stage, double norm, bool inv2, bool unonly = false);
 void launch_phshift(const Ctx& c, int nv);
 void launch_realspace(const Ctx& c, int want_velmax);
-// fold the velmax slots into slot 0
-void launch_velmax_reduce(const Ctx& c);
+// the maximum of the velmax slots into *out (pinned host memory); the slots are cleared
+void launch_velmax_reduce(const Ctx& c, unsigned long long* out);
 void launch_wavespace(const Ctx& c, double norm);
 void launch_update(const Ctx& c, int stage);
 void launch_wavespace_update(const Ctx& c, double norm, int stage);
 // RK4 substep k = 1..4 in the fused y forward kernel (W1 -> u, un, u1); -1 for an unsupported grid
 int launch_y_rk4(const Ctx& c, int k, double norm, void* u1);
-// FEK shell energies of the force list: per-entry terms (2 doubles each)
-// summed per shell in list order
-void launch_ek_shell(const Ctx& c, int kfor, double* d_ek, double* terms);
-// (c.u null: only un is scaled)
-void launch_ek_scale(const Ctx& c, int kf_shell, const double* d_ratio);
+// FEK forcing on the force list: shell energies 1 .. kfor of un and, with
+// kf_shell > 0, the scaling of un and u (c.u null: un only) towards inf and the
+// energies after it; out (pinned host memory, 2 kMaxKfor + 1 doubles): before |
+// after | 1 if a shell without energy stopped the scaling.  terms: 12 bytes per
+// entry, ek: kfor doubles, both for lists too long for one work-group.
+constexpr int kMaxKfor = 64;
+struct EkInf {
+  double e[kMaxKfor];
+};
+void launch_ek_force(const Ctx& c, int kfor, int kf_shell, const EkInf& inf, double* terms, double* ek, double* out);
 // FP64 shell statistics in a fixed order: kShellBlocks partial rows of
 // 2 shell_rows(n) doubles in part, then out[0..nshell) = E,
 // out[nshell..2 nshell) = D, out[2 nshell] = TKE, out[2 nshell + 1] = eps

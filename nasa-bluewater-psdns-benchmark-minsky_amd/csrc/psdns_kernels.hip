@@ -860,8 +860,8 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
 // work-group reduces its threads' values (wavefront shuffles, then LDS), and
 // one thread applies it with an atomic max to one of kVelmaxSlots slots,
 // 256 bytes apart, chosen by work-group, so that the atomics spread over
-// the L2 channels instead of queueing on one address; k_velmax_reduce folds
-// the slots into slot 0.  Non-negative doubles order as their bit patterns.
+// the L2 channels instead of queueing on one address; k_velmax_reduce takes
+// the maximum of the slots and clears them for the next use.  Non-negative doubles order as their bit patterns.
 // Every thread of the work-group calls it (one barrier inside).
 __device__ __forceinline__ void velmax_commit(double m, unsigned long long* velmax) {
   __shared__ double wmax[16];
@@ -877,15 +877,19 @@ __device__ __forceinline__ void velmax_commit(double m, unsigned long long* velm
   }
 }
 
-__global__ void __launch_bounds__(kVelmaxSlots) k_velmax_reduce(unsigned long long* velmax) {
+// out: pinned host memory (the caller reads it after the stream's
+// synchronisation; a copy of the value and a fill of the slots were two more
+// launches of every step)
+__global__ void __launch_bounds__(kVelmaxSlots) k_velmax_reduce(unsigned long long* velmax, unsigned long long* out) {
   __shared__ unsigned long long s[kVelmaxSlots];
   s[threadIdx.x] = velmax[(size_t)threadIdx.x * kVelmaxStride];
+  velmax[(size_t)threadIdx.x * kVelmaxStride] = 0;
   __syncthreads();
   for (int h = kVelmaxSlots / 2; h > 0; h >>= 1) {
     if ((int)threadIdx.x < h) s[threadIdx.x] = s[threadIdx.x] > s[threadIdx.x + h] ? s[threadIdx.x] : s[threadIdx.x + h];
     __syncthreads();
   }
-  if (threadIdx.x == 0) velmax[0] = s[0];
+  if (threadIdx.x == 0) *out = s[0];
 }
 
 // realspace_vel.f:105-113 (b = 1): slot s of u^2-v^2, uv, w^2-v^2, vw, uw
@@ -1716,58 +1720,126 @@ __global__ void __launch_bounds__((RunLines<R>::B * YUpd<R, N>::T))
 }
 
 // ---------------------------------------------------------------------------
-// FEK forcing over a short list of (a, y) entries with |k| < kf_shell + 1.5
-// (ek_shell.f:131-168, ek_force.f:47-66), FP64 sums.
+// FEK forcing over a list of the (a, y) entries with int(|k| + 1.5) <= kfor
+// (ek_shell.f:131-168, ek_force.f:27-71), FP64 sums: the shell energies of un,
+// and with kf_shell > 0 the scaling of un (and of u, unless null) by
+// sqrt(ekinf(ik) / ek(ik)) for ik <= kf_shell (0 for ik = 1) and the energies
+// after it.  out (pinned host memory): ek[kMaxKfor] before, ek[kMaxKfor] after,
+// and 1 if a shell 2 .. kfor has no energy, in which case nothing is scaled.
+// A shell's sum: lane l of one wave adds the entries l, l + 64, .. in order,
+// then the lanes by pairs, so it has the same bits every time.
+// One work-group does it all for lists of up to kEkSmall entries (kfor <= 12);
+// 4.4 us for the usual 4 shells, where the energies, their copy to the host,
+// the ratios' copy back, the scaling, and the energies again were five kernels
+// (one summing a shell per thread: 14 us, twice), three copies and three waits;
+// with velmax's copy and clearing gone too a 32^3 FP32 step and the read of its
+// state went from 246 to 154 us.  Longer lists take three kernels (terms, one
+// wave per shell, scaling) and the first two again.
 // ---------------------------------------------------------------------------
-// per entry of the list: terms[2 i] = tfact |u|^2 / 2, terms[2 i + 1] = its
-// shell (0 past kfor); k_ek_fold sums each shell in list order
+constexpr int kEkSmall = 4096, kEkThreads = 1024;
+
+// the energy term of entry j and its shell
 template <typename R>
-__global__ void __launch_bounds__(256)
-    k_ek_terms(const C<R>* __restrict__ un, Geo g, const int2* __restrict__ list, int nlist, int kfor,
-               double* __restrict__ terms) {
-  const size_t tot = (size_t)g.na * g.n;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nlist; i += gridDim.x * blockDim.x) {
-    const int a = list[i].x, y = list[i].y;
-    const int x = g.colx[a], z = g.colz[a];
-    const double kx = x, ky = kwave(y, g.n), kz = kwave(z, g.n);
-    const int ik = (int)(sqrt(kx * kx + ky * ky + kz * kz) + 1.5);
-    const size_t j = (size_t)a * g.n + y;
-    double s = 0;
-    for (int v = 0; v < 3; v++) {
-      const C<R> q = un[v * tot + j];
-      s += (double)q.x * q.x + (double)q.y * q.y;
-    }
-    terms[2 * (size_t)i] = ik <= kfor ? s / 2.0 * (x == 0 ? 1.0 : 2.0) : 0.0;
-    terms[2 * (size_t)i + 1] = ik <= kfor ? (double)ik : 0.0;
-  }
-}
-__global__ void __launch_bounds__(64)
-    k_ek_fold(const double* __restrict__ terms, int nlist, int kfor, double* __restrict__ ek) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  if (k > kfor) return;
+__device__ __forceinline__ double ek_term(const C<R>* __restrict__ un, size_t tot, size_t j, int x) {
   double s = 0;
-  for (int i = 0; i < nlist; i++)
-    if (terms[2 * (size_t)i + 1] == (double)k) s += terms[2 * (size_t)i];
-  ek[k - 1] = s;
+#pragma unroll
+  for (int v = 0; v < 3; v++) {
+    const C<R> q = un[v * tot + j];
+    s += (double)q.x * q.x + (double)q.y * q.y;
+  }
+  return s / 2.0 * (x == 0 ? 1.0 : 2.0);
+}
+__device__ __forceinline__ int ek_shell_of(const Geo& g, int2 e) {
+  const double kx = g.colx[e.x], ky = kwave(e.y, g.n), kz = kwave(g.colz[e.x], g.n);
+  return (int)(sqrt(kx * kx + ky * ky + kz * kz) + 1.5);
+}
+// one wave: the sum of the terms of shell k
+__device__ __forceinline__ double ek_shell_sum(const double* terms, const int* shell, int nlist, int k) {
+  double s = 0.0;
+  for (int i = threadIdx.x & 63; i < nlist; i += 64) s += shell[i] == k ? terms[i] : 0.0;
+  return wave_sum(s);
+}
+// the scaling factor of shell k (ek_force.f:31-35)
+__device__ __forceinline__ double ek_ratio(int k, const double* ek, const EkInf& inf) {
+  return k == 1 ? 0.0 : sqrt(inf.e[k - 1] / ek[k - 1]);
+}
+__device__ __forceinline__ bool ek_all_positive(const double* ek, int kfor) {
+  bool ok = true;
+  for (int k = 2; k <= kfor; k++) ok = ok && ek[k - 1] > 0.0;
+  return ok;
+}
+template <typename R>
+__device__ __forceinline__ void ek_scale_entry(C<R>* __restrict__ u, C<R>* __restrict__ un, size_t tot, size_t j, R r) {
+#pragma unroll
+  for (int v = 0; v < 3; v++) {
+    un[v * tot + j] = cscale(un[v * tot + j], r);
+    if (u) u[v * tot + j] = cscale(u[v * tot + j], r);  // null: u does not hold the state
+  }
 }
 
 template <typename R>
-__global__ void k_ek_scale(C<R>* __restrict__ u, C<R>* __restrict__ un, Geo g, const int2* __restrict__ list,
-                           int nlist, int kf_shell, const double* __restrict__ ratio) {
+__global__ void __launch_bounds__(kEkThreads)
+    k_ek_small(C<R>* __restrict__ u, C<R>* __restrict__ un, Geo g, const int2* __restrict__ list, int nlist, int kfor,
+               int kf_shell, EkInf inf, double* __restrict__ out) {
+  __shared__ double terms[kEkSmall], ek[kMaxKfor];
+  __shared__ int shell[kEkSmall];
   const size_t tot = (size_t)g.na * g.n;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nlist; i += gridDim.x * blockDim.x) {
-    const int a = list[i].x, y = list[i].y;
-    const int x = g.colx[a], z = g.colz[a];
-    const double kx = x, ky = kwave(y, g.n), kz = kwave(z, g.n);
-    const int ik = (int)(sqrt(kx * kx + ky * ky + kz * kz) + 1.5);
-    if (ik > kf_shell) continue;
-    const size_t j = (size_t)a * g.n + y;
-    const R r = (R)ratio[ik - 1];
-    for (int v = 0; v < 3; v++) {
-      un[v * tot + j] = cscale(un[v * tot + j], r);
-      if (u) u[v * tot + j] = cscale(u[v * tot + j], r);  // null: u does not hold the state
-    }
+  const int wave = threadIdx.x >> 6;
+  for (int i = threadIdx.x; i < nlist; i += kEkThreads) {
+    const int2 e = list[i];
+    shell[i] = ek_shell_of(g, e);
+    terms[i] = ek_term(un, tot, (size_t)e.x * g.n + e.y, g.colx[e.x]);
   }
+  __syncthreads();
+  for (int k = 1 + wave; k <= kfor; k += kEkThreads / 64) {
+    const double s = ek_shell_sum(terms, shell, nlist, k);
+    if ((threadIdx.x & 63) == 0) out[k - 1] = ek[k - 1] = s;
+  }
+  if (kf_shell == 0) return;
+  __syncthreads();
+  const bool ok = ek_all_positive(ek, kfor);
+  if (threadIdx.x == 0) out[2 * kMaxKfor] = ok ? 0.0 : 1.0;
+  if (!ok) return;
+  for (int i = threadIdx.x; i < nlist; i += kEkThreads) {
+    const int2 e = list[i];
+    const size_t j = (size_t)e.x * g.n + e.y;
+    if (shell[i] <= kf_shell) ek_scale_entry(u, un, tot, j, (R)ek_ratio(shell[i], ek, inf));
+    terms[i] = ek_term(un, tot, j, g.colx[e.x]);
+  }
+  __syncthreads();
+  for (int k = 1 + wave; k <= kfor; k += kEkThreads / 64) {
+    const double s = ek_shell_sum(terms, shell, nlist, k);
+    if ((threadIdx.x & 63) == 0) out[kMaxKfor + k - 1] = s;
+  }
+}
+
+template <typename R>
+__global__ void __launch_bounds__(256)
+    k_ek_terms(const C<R>* __restrict__ un, Geo g, const int2* __restrict__ list, int nlist, double* __restrict__ terms,
+               int* __restrict__ shell) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nlist) return;
+  const int2 e = list[i];
+  shell[i] = ek_shell_of(g, e);
+  terms[i] = ek_term(un, (size_t)g.na * g.n, (size_t)e.x * g.n + e.y, g.colx[e.x]);
+}
+// work-group k - 1: shell k
+__global__ void __launch_bounds__(64)
+    k_ek_sums(const double* __restrict__ terms, const int* __restrict__ shell, int nlist, double* __restrict__ ek,
+              double* __restrict__ out) {
+  const double s = ek_shell_sum(terms, shell, nlist, blockIdx.x + 1);
+  if (threadIdx.x == 0) out[blockIdx.x] = ek[blockIdx.x] = s;
+}
+template <typename R>
+__global__ void __launch_bounds__(256)
+    k_ek_scale(C<R>* __restrict__ u, C<R>* __restrict__ un, Geo g, const int2* __restrict__ list,
+               const int* __restrict__ shell, int nlist, int kfor, int kf_shell, EkInf inf,
+               const double* __restrict__ ek, double* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool ok = ek_all_positive(ek, kfor);
+  if (i == 0) out[2 * kMaxKfor] = ok ? 0.0 : 1.0;
+  if (!ok || i >= nlist || shell[i] > kf_shell) return;
+  ek_scale_entry(u, un, (size_t)g.na * g.n, (size_t)list[i].x * g.n + list[i].y, (R)ek_ratio(shell[i], ek, inf));
 }
 
 // ---------------------------------------------------------------------------
@@ -2635,15 +2707,23 @@ struct LaunchP {
                          (CR*)c.u, (CR*)c.un, c.geo, norm, c.sx[c.kstep], c.sy[c.kstep], c.sz[c.kstep], c.xfac,
                          c.yfac, c.zfac);
   }
-  static void ek_shell(const Ctx& c, int kfor, double* d_ek, double* terms) {
-    if (c.nforce > 0)
-      hipLaunchKernelGGL((k_ek_terms<R>), dim3(grid1d(c.nforce, 256)), dim3(256), 0, c.stream, (const CR*)c.un,
-                         c.geo, c.force_list, c.nforce, kfor, terms);
-    hipLaunchKernelGGL(k_ek_fold, dim3((kfor + 63) / 64), dim3(64), 0, c.stream, terms, c.nforce, kfor, d_ek);
-  }
-  static void ek_scale(const Ctx& c, int kf_shell, const double* d_ratio) {
-    hipLaunchKernelGGL((k_ek_scale<R>), dim3(grid1d(c.nforce, 256)), dim3(256), 0, c.stream, (CR*)c.u,
-                       (CR*)c.un, c.geo, c.force_list, c.nforce, kf_shell, d_ratio);
+  static void ek_force(const Ctx& c, int kfor, int kf_shell, const EkInf& inf, double* terms, double* ek, double* out) {
+    const int nl = c.nforce;
+    if (nl <= kEkSmall) {
+      hipLaunchKernelGGL((k_ek_small<R>), dim3(1), dim3(kEkThreads), 0, c.stream, (CR*)c.u, (CR*)c.un, c.geo,
+                         c.force_list, nl, kfor, kf_shell, inf, out);
+      return;
+    }
+    int* shell = (int*)(terms + nl);
+    const dim3 grid(grid1d(nl, 256));
+    for (int pass = 0; pass < (kf_shell > 0 ? 2 : 1); pass++) {
+      hipLaunchKernelGGL((k_ek_terms<R>), grid, dim3(256), 0, c.stream, (const CR*)c.un, c.geo, c.force_list, nl, terms,
+                         shell);
+      hipLaunchKernelGGL(k_ek_sums, dim3(kfor), dim3(64), 0, c.stream, terms, shell, nl, ek, out + pass * kMaxKfor);
+      if (pass == 0 && kf_shell > 0)
+        hipLaunchKernelGGL((k_ek_scale<R>), grid, dim3(256), 0, c.stream, (CR*)c.u, (CR*)c.un, c.geo, c.force_list,
+                           shell, nl, kfor, kf_shell, inf, ek, out);
+    }
   }
   static void shell_stats(const Ctx& c, double viscos, int nshell, double* part, double* out) {
     const int nh = shell_rows(c.geo.n);
@@ -2740,8 +2820,8 @@ int launch_pass(const Ctx& c, Pass p, int a0, int a1) {
   return c.prec == 8 ? run_pass_n<double>(c, p, a0, a1) : run_pass_n<float>(c, p, a0, a1);
 }
 
-void launch_velmax_reduce(const Ctx& c) {
-  hipLaunchKernelGGL(k_velmax_reduce, dim3(1), dim3(kVelmaxSlots), 0, c.stream, c.velmax_bits);
+void launch_velmax_reduce(const Ctx& c, unsigned long long* out) {
+  hipLaunchKernelGGL(k_velmax_reduce, dim3(1), dim3(kVelmaxSlots), 0, c.stream, c.velmax_bits, out);
 }
 
 void launch_realspace(const Ctx& c, int want_velmax) {
@@ -2764,13 +2844,9 @@ void launch_wavespace_update(const Ctx& c, double norm, int stage) {
   if (c.prec == 8) LaunchP<double>::wavespace_update(c, norm, stage);
   else LaunchP<float>::wavespace_update(c, norm, stage);
 }
-void launch_ek_shell(const Ctx& c, int kfor, double* d_ek, double* terms) {
-  if (c.prec == 8) LaunchP<double>::ek_shell(c, kfor, d_ek, terms);
-  else LaunchP<float>::ek_shell(c, kfor, d_ek, terms);
-}
-void launch_ek_scale(const Ctx& c, int kf_shell, const double* d_ratio) {
-  if (c.prec == 8) LaunchP<double>::ek_scale(c, kf_shell, d_ratio);
-  else LaunchP<float>::ek_scale(c, kf_shell, d_ratio);
+void launch_ek_force(const Ctx& c, int kfor, int kf_shell, const EkInf& inf, double* terms, double* ek, double* out) {
+  if (c.prec == 8) LaunchP<double>::ek_force(c, kfor, kf_shell, inf, terms, ek, out);
+  else LaunchP<float>::ek_force(c, kfor, kf_shell, inf, terms, ek, out);
 }
 void launch_shell_stats(const Ctx& c, double viscos, int nshell, double* part, double* out) {
   if (c.prec == 8) LaunchP<double>::shell_stats(c, viscos, nshell, part, out);

@@ -290,3 +290,35 @@ def test_vg_moments_reproducible(O, P, ctxs, n, prec):
         assert np.all(np.abs(got - ref) <= tol * scale), (got, ref)
     s.kxtran(3)
     assert rel(s.get_field(P.FIELD_UX, 3), g.kxtran(u0, 3)) < (1e-12 if prec == 8 else 3e-6)
+
+
+@pytest.mark.parametrize("prec", [8, 4])
+@pytest.mark.parametrize("kfor", [2, 12, 13, 20])
+def test_ek_force_list_lengths(O, P, ctxs, kfor, prec):
+    """FEK energies and scaling for lists that one work-group takes (kfor <= 12:
+    at most 4096 entries) and longer ones: the energies are FP64 sums of the
+    state's own values, the scaling one rounding in the state precision."""
+    n = 64
+    banner("ek_force", kfor, prec)
+    g, s = O.Grid(n), ctxs(n, prec)
+    s.put_state(g.field(seed=29))
+    u0 = s.get_state().astype(np.complex128)
+    ref = g.ek_shell(u0, kfor)
+    ek = s.ek_shell(kfor)
+    assert np.allclose(ek, ref, rtol=1e-12, atol=0)
+    kf = kfor - 1
+    target = ref * np.linspace(0.5, 1.5, kfor)
+    out = s.ek_force(kf, kfor, target)
+    want = np.where(np.arange(1, kfor + 1) <= kf, target, ref)
+    want[0] = 0.0
+    assert np.allclose(out, want, rtol=1e-12 if prec == 8 else 1e-6, atol=0)
+    kx, ky, kz = kgrid(n, g.col_x, g.col_z)
+    ik = (np.sqrt(kx ** 2 + ky ** 2 + kz ** 2) + 1.5).astype(int)
+    ratio = np.ones(n + 2)
+    ratio[1:kf + 1] = np.sqrt(want[:kf] / np.where(ref[:kf] > 0, ref[:kf], 1.0))
+    got = s.get_state()
+    assert rel(got, u0 * ratio[np.minimum(ik, n + 1)]) < (1e-14 if prec == 8 else 1e-7)
+    # a shell without energy stops the scaling
+    s.put_state(np.zeros_like(u0))
+    with pytest.raises(P.PsdnsError, match="no energy"):
+        s.ek_force(kf, kfor, target)
