@@ -32,6 +32,17 @@ constexpr int kVelmaxStride = 32;
 // columns per y-pass group (64-byte runs of complex values in W)
 inline int y_group_lines(int prec) { return prec == 8 ? 4 : 8; }
 
+// Work-groups are handed to the 8 XCDs round-robin by linear block id, and
+// each XCD has its own L2.  Give every XCD a contiguous range of logical
+// blocks so that neighbouring tiles (which share cache lines and DRAM pages)
+// are worked on by the same L2.  Bijective for any grid size.
+__device__ __forceinline__ int xcd_block(int bid, int nblocks) {
+  constexpr int kXcd = 8;
+  const int q = nblocks / kXcd, r = nblocks % kXcd;
+  const int x = bid % kXcd, k = bid / kXcd;
+  return x * q + (x < r ? x : r) + k;
+}
+
 // Everything a launcher needs; owned by psdns_ctx.
 // mean scalar gradients (G1, G2, G3) of up to kMaxSc scalars, passed to the
 // fused x pass by value

@@ -80,16 +80,6 @@ __device__ __forceinline__ C<R> to_c(double2 a) {
   return {(R)a.x, (R)a.y};
 }
 
-// Work-groups are handed to the 8 XCDs round-robin by linear block id, and
-// each XCD has its own L2.  Give every XCD a contiguous range of logical
-// blocks so that neighbouring tiles (which share cache lines and DRAM pages)
-// are worked on by the same L2.  Bijective for any grid size.
-__device__ __forceinline__ int xcd_block(int bid, int nblocks) {
-  constexpr int kXcd = 8;
-  const int q = nblocks / kXcd, r = nblocks % kXcd;
-  const int x = bid % kXcd, k = bid / kXcd;
-  return x * q + (x < r ? x : r) + k;
-}
 // logical (block.x, block.y) of a 2-D grid after the XCD remap
 __device__ __forceinline__ int2 xcd_block2() {
   const int n = gridDim.x * gridDim.y;

@@ -210,7 +210,8 @@ int psdns_sgs_filter(psdns_sgs* m, psdns_ctx* fine, psdns_ctx* coarse) {
   if (cf.prec != cc.prec) return set_error(PSDNS_EINVAL, "fine and coarse contexts differ in precision");
   if (nf % nc || (nf / nc) % 2) return set_error(PSDNS_EINVAL, "n_fine / n_coarse = %d / %d: an even ratio", nf, nc);
   if ((rc = psdns::ctx_sync(fine))) return rc;
-  S::launch_box_filter(cc.stream, cc.prec, cf.ux, nf, nf / nc, cc.ux, m->tau);
+  if (S::launch_box_filter(cc.stream, cc.prec, cf.ux, nf, nf / nc, cc.ux, m->tau))
+    return set_error(PSDNS_EINVAL, "unsupported filter ratio %d", nf / nc);
   SGSCHK(hipGetLastError());
   if ((rc = psdns::ctx_sync(coarse))) return rc;
   m->have_target = true;

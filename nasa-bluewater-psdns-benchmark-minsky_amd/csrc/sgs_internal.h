@@ -39,7 +39,8 @@ constexpr int kMaxBatch = 65536;
 // more rows would only lengthen the fold)
 constexpr int train_rows(int B) { return (B + 63) / 64 < 256 ? (B + 63) / 64 : 256; }
 
-void launch_box_filter(hipStream_t st, int prec, const void* u, int n, int r, void* ubar, float* tau);
+// r = 2, 4, .., 32 (the ratios of two grids between 32 and 1024); -1 for another
+int launch_box_filter(hipStream_t st, int prec, const void* u, int n, int r, void* ubar, float* tau);
 // i k_j u_i on the mask; with a stage (1|2) the state is first phase shifted
 // by that stage's factors (phase1 on the fly), stage 0 takes u as it is
 void launch_grad_spec(const Ctx& c, const void* u, void* d, int stage);

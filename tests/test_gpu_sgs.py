@@ -41,6 +41,38 @@ def test_box_filter_matches_oracle(O, P, n, nc, prec):
     assert np.abs(tau).max() > 1e-3
 
 
+@pytest.mark.parametrize("n,nc,prec", [(64, 32, 4), (256, 64, 8), (256, 32, 4), (512, 32, 4)])
+def test_box_filter_ratios(O, P, n, nc, prec):
+    """ratios 2, 4, 8 and 16 on a random physical field, at coarse points that
+    wrap around each side and one inside, against direct FP64 sums (the
+    stress is stored in FP32, the velocity in the state precision)"""
+    print("[gpu case] sgs box ratios", n, nc, prec, flush=True)
+    r = n // nc
+    u = np.random.default_rng(n + nc).random((3, n, n, n), dtype=np.float32)
+    fine, coarse = P.Solver(n, prec), P.Solver(nc, prec)
+    m = P.Closure(nc)
+    try:
+        fine.put_field(P.FIELD_UX, u)
+        m.filter(fine, coarse)
+        got_u = coarse.get_field(P.FIELD_UX, 3)
+        got_t = m.field(P.SGS_TARGET)
+    finally:
+        m.close()
+        fine.close()
+        coarse.close()
+    offs, w = SG.box_weights(r)
+    w3 = w[:, None, None] * w[None, :, None] * w[None, None, :]
+    for c in [(0, 0, 0), (nc - 1, 0, nc - 1), (0, nc - 1, 1), (5, 7, nc // 2)]:
+        at = np.ix_(range(3), *[(r * ci + offs) % n for ci in c])
+        b = u[at].astype(np.float64)
+        ub = (b * w3).sum((1, 2, 3))
+        tau = np.array([(b[i] * b[j] * w3).sum() - ub[i] * ub[j] for i, j in SG.SYM])
+        tau[[0, 3, 5]] -= (tau[0] + tau[3] + tau[5]) / 3.0
+        y, z, x = c
+        assert rel(got_u[:, y, z, x], ub) < (1e-13 if prec == 8 else 1.2e-7)
+        assert np.abs(got_t[:, y, z, x] - tau).max() < 1.2e-7 * np.abs(tau).max()
+
+
 @pytest.mark.parametrize("shifted", [False, True], ids=["unshifted", "phase1"])
 def test_features_match_oracle(O, P, shifted):
     print("[gpu case] sgs features", shifted, flush=True)
