@@ -59,7 +59,6 @@ struct psdns_sgs {
   int A_prec = 0;     // precision of the gradient in A (that of the last features context)
   // current field: features, target, prediction
   float *lam = nullptr, *T = nullptr, *tau = nullptr, *tau_hat = nullptr;
-  float* h0 = nullptr;  // the convolution's 16 channels of the last prediction
   bool have_features = false, have_target = false, have_pred = false;
   // training store
   float *lam_s = nullptr, *T_s = nullptr, *tau_s = nullptr;
@@ -150,7 +149,6 @@ int psdns_sgs_create(int n, int max_snapshots, psdns_sgs** out) {
   const size_t P = m->P;
   if ((rc = dalloc(&m->lam, 5 * P, "the invariants")) || (rc = dalloc(&m->T, 24 * P, "the tensor basis")) ||
       (rc = dalloc(&m->tau, 6 * P, "the target stress")) || (rc = dalloc(&m->tau_hat, 6 * P, "the predicted stress")) ||
-      (rc = dalloc(&m->h0, 16 * P, "the convolution channels")) ||
       (rc = dalloc(&m->theta, S::kParams, "theta")) || (rc = dalloc(&m->m, S::kParams, "the Adam moments")) ||
       (rc = dalloc(&m->v, S::kParams, "the Adam moments")) || (rc = dalloc(&m->grad, S::kParams, "the gradient")))
     return bail(rc);
@@ -172,7 +170,7 @@ int psdns_sgs_create(int n, int max_snapshots, psdns_sgs** out) {
 int psdns_sgs_destroy(psdns_sgs* m) {
   if (!m) return PSDNS_OK;
   if (m->stream) (void)hipStreamSynchronize(m->stream);
-  void* ptrs[] = {m->cyl, m->yw, m->xi, m->A, m->lam, m->T, m->tau, m->tau_hat, m->h0, m->lam_s, m->T_s,
+  void* ptrs[] = {m->cyl, m->yw, m->xi, m->A, m->lam, m->T, m->tau, m->tau_hat, m->lam_s, m->T_s,
                   m->tau_s, m->theta, m->m, m->v, m->grad, m->work, m->lpart, m->losses};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -396,7 +394,7 @@ int psdns_sgs_train(psdns_sgs* m, int nsteps, int batch, double lr, unsigned lon
 int psdns_sgs_predict(psdns_sgs* m, int bf16) {
   if (!m) return set_error(PSDNS_EINVAL, "null argument");
   if (!m->have_features) return set_error(PSDNS_ESTATE, "no features (psdns_sgs_features)");
-  S::launch_predict(m->stream, bf16 != 0, m->lam, m->T, m->n, m->theta, m->h0, m->tau_hat);
+  S::launch_predict(m->stream, bf16 != 0, m->lam, m->T, m->n, m->theta, m->tau_hat);
   SGSCHK(hipGetLastError());
   if (int rc = sync(m)) return rc;
   m->have_pred = true;

@@ -45,9 +45,9 @@ int launch_box_filter(hipStream_t st, int prec, const void* u, int n, int r, voi
 // by that stage's factors (phase1 on the fly), stage 0 takes u as it is
 void launch_grad_spec(const Ctx& c, const void* u, void* d, int stage);
 void launch_invariants(hipStream_t st, int prec, const void* A, size_t P, double delta2, float* lam, float* T);
-// conv (FP32) into h0[16][P], then the dense layers (FP32 or bf16 matrix cores)
-void launch_predict(hipStream_t st, bool bf16, const float* lam, const float* T, int n, const float* theta,
-                    float* h0, float* tau);
+// the closure's stress of the features: the convolution in FP32, the dense
+// layers in FP32 or on bf16 operands
+void launch_predict(hipStream_t st, bool bf16, const float* lam, const float* T, int n, const float* theta, float* tau);
 void launch_add_stress(hipStream_t st, int prec, void* ux, const float* tau, size_t P);
 int field_err_blocks();
 void launch_field_err(hipStream_t st, const float* tp, const float* tt, size_t P, double* part);

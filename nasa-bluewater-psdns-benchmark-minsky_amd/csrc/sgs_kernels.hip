@@ -614,140 +614,56 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------------------
-// Inference.  k_conv: the 3x3x3 convolution of the invariant field (FP32,
-// one thread per point, the 135 taps and 16 output channels unrolled, the
-// weights read once per work-group from LDS), h0 = tanh(conv) into
-// h0[16][P].  The dense layers then read [lambda(p), h0(p)] of their own
-// point only: k_mlp_f32 (one thread per point, theta in LDS) or
-// k_mlp_bf16 (matrix cores).
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-    k_conv(const float* __restrict__ lam, int n, const float* __restrict__ theta, float* __restrict__ h0) {
-  // the weights tap-major in LDS: wt[k] = W0[0..15][k] as four float4
-  __shared__ float4 wt[kIn0][kConv / 4];
-  __shared__ float bias[kConv];
-  for (int i = threadIdx.x; i < kIn0 * kConv; i += blockDim.x) {
-    const int k = i / kConv, c = i % kConv;
-    reinterpret_cast<float*>(&wt[k][0])[c] = theta[oW0 + c * kIn0 + k];
-  }
-  if (threadIdx.x < kConv) bias[threadIdx.x] = theta[ob0 + threadIdx.x];
-  __syncthreads();
-  // one point per thread; the (ch, dy, dz) rows run as a loop (unrolled,
-  // the 2160 weight reads would be scheduled ahead into spilled registers)
-  const size_t P = (size_t)n * n * n;
-  const int w = n - 1;
-  const size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (p < P) {
-    const int y = (int)(p / ((size_t)n * n)), z = (int)((p / n) & w), x = (int)(p & w);
-    float h[kConv];
-#pragma unroll
-    for (int c = 0; c < kConv; c++) h[c] = bias[c];
-#pragma unroll 1
-    for (int row = 0; row < kLam * 9; row++) {
-      const int ch = row / 9, dy = (row / 3) % 3 - 1, dz = row % 3 - 1;
-      const float* src = lam + ch * P + (((size_t)((y + dy) & w) * n + ((z + dz) & w)) * n);
-      const float v[3] = {src[(x - 1) & w], src[x], src[(x + 1) & w]};
-#pragma unroll
-      for (int dx = 0; dx < 3; dx++) {
-        const int k = row * 3 + dx;  // = ch * 27 + ((dy + 1) * 3 + dz + 1) * 3 + dx
-#pragma unroll
-        for (int q = 0; q < kConv / 4; q++) {
-          const float4 wv = wt[k][q];
-          h[4 * q + 0] = fmaf(wv.x, v[dx], h[4 * q + 0]);
-          h[4 * q + 1] = fmaf(wv.y, v[dx], h[4 * q + 1]);
-          h[4 * q + 2] = fmaf(wv.z, v[dx], h[4 * q + 2]);
-          h[4 * q + 3] = fmaf(wv.w, v[dx], h[4 * q + 3]);
-        }
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < kConv; c++) h0[c * P + p] = tanhf(h[c]);
-  }
-}
-
-__global__ void __launch_bounds__(256)
-    k_mlp_f32(const float* __restrict__ lam, const float* __restrict__ h0, const float* __restrict__ T, int n,
-              const float* __restrict__ theta, float* __restrict__ tau) {
-  __shared__ float th[kParams - ob0 - kConv];  // W1 onwards
-  for (int i = threadIdx.x; i < kParams - oW1; i += blockDim.x) th[i] = theta[oW1 + i];
-  __syncthreads();
-  const float* W1 = th;
-  const float* b1 = th + (ob1 - oW1);
-  const float* W2 = th + (oW2 - oW1);
-  const float* b2 = th + (ob2 - oW1);
-  const float* W3 = th + (oW3 - oW1);
-  const float* b3 = th + (ob3 - oW1);
-  const float* W4 = th + (oW4 - oW1);
-  const float* b4 = th + (ob4 - oW1);
-  const size_t P = (size_t)n * n * n;
-  const size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x;  // one point per thread, as k_conv
-  if (p < P) {
-    float x1[kIn1];
-#pragma unroll
-    for (int c = 0; c < kLam; c++) x1[c] = lam[c * P + p];
-#pragma unroll
-    for (int c = 0; c < kConv; c++) x1[kLam + c] = h0[c * P + p];
-    float ha[kHid], hb[kHid];
-#pragma unroll
-    for (int o = 0; o < kHid; o++) {
-      float a = b1[o];
-#pragma unroll
-      for (int i = 0; i < kIn1; i++) a = fmaf(x1[i], W1[o * kIn1 + i], a);
-      ha[o] = tanhf(a);
-    }
-#pragma unroll
-    for (int o = 0; o < kHid; o++) {
-      float a = b2[o];
-#pragma unroll
-      for (int i = 0; i < kHid; i++) a = fmaf(ha[i], W2[o * kHid + i], a);
-      hb[o] = tanhf(a);
-    }
-#pragma unroll
-    for (int o = 0; o < kHid; o++) {
-      float a = b3[o];
-#pragma unroll
-      for (int i = 0; i < kHid; i++) a = fmaf(hb[i], W3[o * kHid + i], a);
-      ha[o] = tanhf(a);
-    }
-    float g[kBasis];
-#pragma unroll
-    for (int o = 0; o < kBasis; o++) {
-      float a = b4[o];
-#pragma unroll
-      for (int i = 0; i < kHid; i++) a = fmaf(ha[i], W4[o * kHid + i], a);
-      g[o] = a;
-    }
-#pragma unroll
-    for (int c = 0; c < 6; c++) {
-      float s = 0.f;
-#pragma unroll
-      for (int k = 0; k < kBasis; k++) s = fmaf(g[k], T[(k * 6 + c) * P + p], s);
-      tau[c * P + p] = s;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Dense layers on the matrix cores: v_mfma_f32_16x16x32_bf16 (bf16 operands,
-// FP32 accumulation), D[16][16] = A[16][32] B[32][16] + C with lane l
-// holding A[l % 16][slot], B[slot][l % 16] for the eight K slots 8 (l / 16)
-// + j, and D[4 (l / 16) + jj][l % 16] (jj < 4).  The K order inside a
-// product is free as long as A and B use the same one.
-// Each layer is computed transposed, Y^T[O][16 points] = W X^T: operand A
-// is a 16-row block ob of the weights, operand B the activations, and the
-// accumulator of block ob leaves lane l with outputs o = 16 ob + 4 (l / 16)
-// + jj of point l % 16.  Those 16 values per lane are exactly the operand B
-// of the next layer if its K slots are ordered as
-//   step s, slot (g, j) <-> input k = 16 (2 s + j / 4) + 4 g + j % 4,
-// so the activations stay in the lane's registers from layer to layer (no
-// LDS tile, no cross-lane exchange).  The weights are stored as operand-A
-// blocks in LDS in that K order (layer 1 in natural order: its operand B is
-// the lane's own inputs k = 8 (l / 16) + j), and the biases as the
-// accumulators' initial values.  Bias and tanh are FP32.
+// Inference in one kernel, k_closure<BF16>: the 3x3x3 convolution of the
+// invariant field and the dense layers on the matrix cores, and the stress
+// tau = sum_n g_n T_n; only lambda and T are read and tau written.
+//
+// A work-group (8 waves) takes blocks of 32 x 4 x 4 points: the block's
+// lambda with a halo of one goes to LDS (5 channels of 6 x 6 rows of 34, row
+// stride 36), a wave takes its 16 consecutive points along x per tile.  All layers
+// are computed transposed, Y^T[O][16 points] = W X^T: lane l (r or c = l % 16,
+// g = l / 16) supplies A = W and B = X for its K slots and receives D[4 g +
+// jj][c], the outputs o = 16 ob + 4 g + jj of its own point c.
+//
+// The convolution runs on v_mfma_f32_16x16x4_f32 (FP32 operands and sums), K =
+// 135 in 34 steps: steps 0 .. 26 are the taps of channels 0 .. 3 (slot g =
+// channel g, so a tap's LDS reads differ by a lane constant and hit all 64
+// banks once), steps 27 .. 33 four taps each of channel 4.  On the VALU, a
+// point per thread with its 135 neighbours from the cache, it took 178 us at
+// 128^3 (116 us at the full FP32 rate; packed FP32 is off), and an earlier
+// matrix form with gathered global reads and a fourth of its slots empty 207.
+//
+// The dense layers, BF16: v_mfma_f32_16x16x32_bf16 (bf16 operands, FP32
+// accumulation), eight K slots (g, j) per lane and step; else
+// v_mfma_f32_16x16x4_f32.  The K order inside a product is free as long as A
+// and B use the same one: with k = 16 (2 s + j / 4) + 4 g + j % 4 (BF16) or k =
+// 16 ob + 4 g + jj (FP32) the accumulators of a layer are the next layer's
+// operand B, so the activations stay in the lane's registers from layer to
+// layer (no LDS tile, no cross-lane exchange).  The weights are in LDS, for
+// BF16 as operand-A blocks in that order; the biases are the accumulators'
+// initial values.  The sums, biases and tanh are FP32.
+//
+// What bounds it, BF16 at 128^3: issue. Per 16 points 1,440 cycles of matrix
+// instructions and about 3,000 of VALU (52 tanh per lane, two quarter-rate
+// instructions each), 236 us on end where nothing overlaps; 270 us per call
+// (253 us with the halo left in place, 209 without the tanh, 218 without the
+// convolution's products), against 178 us for the convolution with its 16
+// channels stored and 189 us for the dense layers that read them back. 64^3:
+// 47 us (75), with FP32 layers 89 us (179). Two tiles per wave, sharing each
+// weight read, came to 262-360 us for 2 to 4 waves per SIMD.
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kWaves = 4;  // waves per work-group
+constexpr int kCWaves = 8;                          // waves per work-group
+constexpr int kBx = 32, kBy = 4, kBz = 4;           // points of a block
+constexpr int kHs = kBx + 4;                        // halo row stride
+constexpr int kHrows = (kBy + 2) * (kBz + 2);       // halo rows of a channel
+constexpr int kHch = kHrows * kHs;                  // channel stride (16 banks apart)
+static_assert(kHch % 64 == 16, "the four channels of a step on different banks");
+// offset of tap (dy, dz, dx) = (tap / 9, tap / 3 % 3, tap % 3) - 1 from that of tap 0
+__device__ __forceinline__ constexpr int tap_off(int tap) {
+  return (tap / 9 * (kBz + 2) + tap / 3 % 3) * kHs + tap % 3;
+}
 
 // an opaque copy of the lane index: addresses formed from it are recomputed
 // where they are used
@@ -759,6 +675,12 @@ __device__ __forceinline__ int opaque_lane(int v) {
 // input k of K step s and slot (g, j) of a layer fed by a 64-wide layer
 __device__ __forceinline__ constexpr int slot_k(int s, int g, int j) { return 16 * (2 * s + j / 4) + 4 * g + j % 4; }
 
+// layer 1's input of K slot (g, j): the lane's own h0 channels, lambda_g, and
+// lambda_4 in the lane group that reads it for the convolution (-1: none)
+__device__ __forceinline__ constexpr int in_k(int g, int j) {
+  return j < 4 ? kLam + 4 * g + j : (j == 4 ? g : (j == 5 && g == 1 ? 4 : -1));
+}
+
 // operand-A blocks in LDS, 64 lanes x 16 bytes each: W1 ob 0..3, W2 (s, ob)
 // 4..11, W3 (s, ob) 12..19, W4 s 20..21 (rows 0..3 of 16)
 constexpr int kOpBlocks = 22;
@@ -769,8 +691,8 @@ __device__ __forceinline__ bf16x8 a_block(const float* __restrict__ theta, int b
     const int o = 16 * blk + r;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-      const int k = 8 * g + j;
-      v[j] = (__bf16)(k < kIn1 ? theta[oW1 + o * kIn1 + k] : 0.f);
+      const int k = in_k(g, j);
+      v[j] = (__bf16)(k >= 0 ? theta[oW1 + o * kIn1 + k] : 0.f);
     }
     return v;
   }
@@ -801,7 +723,8 @@ __device__ __forceinline__ f32x4 bias_block(const float* __restrict__ theta, int
 // (even __fdividef) compiles to the full IEEE sequence, several times the
 // cost of the rest of the activation.
 __device__ __forceinline__ float tanh_fast(float x) {
-  return 1.f - 2.f * __builtin_amdgcn_rcpf(__expf(2.f * x) + 1.f);
+  // exp(2 x) as v_exp_f32 (2^v) of 2 x log2(e)
+  return fmaf(-2.f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(2.8853900817779268f * x) + 1.f), 1.f);
 }
 // operand B of K step s of the next layer: tanh of accumulator blocks 2 s
 // and 2 s + 1 of this lane
@@ -815,98 +738,204 @@ __device__ __forceinline__ bf16x8 act_operand(f32x4 d0, f32x4 d1) {
   return r;
 }
 
-__global__ void __launch_bounds__(64 * kWaves)
-    k_mlp_bf16(const float* __restrict__ lam, const float* __restrict__ h0, const float* __restrict__ T, int n,
-               const float* __restrict__ theta, float* __restrict__ tau) {
-  __shared__ bf16x8 wop[kOpBlocks][64];
-  __shared__ f32x4 bias[13][4];  // [3 layers x 4 ob + the output layer][g]
-  for (int i = threadIdx.x; i < kOpBlocks * 64; i += blockDim.x) wop[i / 64][i % 64] = a_block(theta, i / 64, i % 64);
-  for (int i = threadIdx.x; i < 13 * 4; i += blockDim.x) {
-    const int b = i / 4, g = i % 4;
-    bias[b][g] = b < 12 ? bias_block(theta, b / 4, b % 4, g) : bias_block(theta, 3, 0, g);
+// the dense layers' weights in LDS
+template <bool BF16>
+struct DenseWeights;
+template <>
+struct DenseWeights<true> {
+  bf16x8 op[kOpBlocks][64];
+  __device__ __forceinline__ void fill(const float* __restrict__ theta, int tid, int nt) {
+    for (int i = tid; i < kOpBlocks * 64; i += nt) op[i / 64][i % 64] = a_block(theta, i / 64, i % 64);
   }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // operand A of block blk and the bias of accumulator block b, read per use
-  // (through an opaque lane index, so that they are not hoisted out of the
-  // tile loop into registers)
-  auto wa = [&](int blk) { return wop[blk][opaque_lane(lane)]; };
+};
+template <>
+struct DenseWeights<false> {
+  __attribute__((aligned(16))) float W2[kHid * kLd], W3[kHid * kLd], W4[kBasis * kLd];
+  float W1[kHid * kIn1];
+  __device__ __forceinline__ void fill(const float* __restrict__ theta, int tid, int nt) {
+    for (int i = tid; i < kHid * kIn1; i += nt) W1[i] = theta[oW1 + i];
+    for (int i = tid; i < kHid * kHid; i += nt) {
+      W2[i / kHid * kLd + i % kHid] = theta[oW2 + i];
+      W3[i / kHid * kLd + i % kHid] = theta[oW3 + i];
+    }
+    for (int i = tid; i < kBasis * kHid; i += nt) W4[i / kHid * kLd + i % kHid] = theta[oW4 + i];
+  }
+};
+
+template <bool BF16>
+__global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
+    k_closure(const float* __restrict__ lam, const float* __restrict__ T, int n, const float* __restrict__ theta,
+              float* __restrict__ tau) {
+  __shared__ __attribute__((aligned(16))) DenseWeights<BF16> wt;
+  __shared__ f32x4 bias[13][4];  // [3 layers x 4 ob + the output layer][g]
+  __shared__ float halo[kLam * kHch];
+  constexpr int NT = 64 * kCWaves;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+  wt.fill(theta, tid, NT);
+  for (int i = tid; i < 13 * 4; i += NT) {
+    const int b = i / 4;
+    bias[b][i % 4] = b < 12 ? bias_block(theta, b / 4, b % 4, i % 4) : bias_block(theta, 3, 0, i % 4);
+  }
+  // this lane's convolution weights (row c) and bias (rows 4 g + jj)
+  constexpr int kSteps = 34;
+  float wc[kSteps];
+#pragma unroll
+  for (int s = 0; s < kSteps; s++) {
+    const int k = s < kTaps ? g * kTaps + s : 4 * (s - kTaps) + g;
+    wc[s] = s < kTaps ? theta[oW0 + c * kIn0 + k] : (k < kTaps ? theta[oW0 + c * kIn0 + 4 * kTaps + k] : 0.f);
+  }
+  f32x4 b0;
+#pragma unroll
+  for (int jj = 0; jj < 4; jj++) b0[jj] = theta[ob0 + 4 * g + jj];
+  // channel 4's tap offsets of this lane group (the slot past the last tap has
+  // weight zero and reads the last tap)
+  int off4[kSteps - kTaps];
+#pragma unroll
+  for (int q = 0; q < kSteps - kTaps; q++) off4[q] = 4 * kHch + tap_off(min(4 * q + g, kTaps - 1));
   auto bc = [&](int b) { return bias[b][opaque_lane(lane) >> 4]; };
 
   const size_t P = (size_t)n * n * n;
-  const size_t ntiles = P / 16;  // n^3 is a multiple of 16 for n >= 4
-  // A tile's global reads, issued one tile ahead so that they are in flight
-  // while the previous tile runs through the layers: xin[j] = input k =
-  // 8 (lane / 16) + j of the lane's point ([lambda, h0], zero past 21), and
-  // for the stress lanes (lane < 48: point lane % 16, components
-  // 2 (lane / 16) + cc) tb[4 cc + k] = T[k][component].
-  auto load_tile = [&](float (&xin)[8], float (&tb)[8], size_t t) {
-    const size_t p = 16 * t + (lane & 15);
+  const int m = n - 1, nbx = n / kBx, nbz = n / kBz, nblk = nbx * nbz * (n / kBy);
+  // The next block's halo is on its way into registers while this one's points
+  // run through the layers (indices formed per block, not held across it).
+  constexpr int W = kBx + 2, kTot = kLam * kHrows * W, kPer = (kTot + NT - 1) / NT;
+  float hv[kPer];
+  auto load_halo = [&](int blk) {
+    const int x0 = blk % nbx * kBx, z0 = blk / nbx % nbz * kBz, y0 = blk / (nbx * nbz) * kBy, t0 = opaque_lane(tid);
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int k = 8 * (lane >> 4) + j;
-      xin[j] = k < kLam ? lam[k * P + p] : (k < kIn1 ? h0[(k - kLam) * P + p] : 0.f);
-    }
-    if (lane < 48) {
-      const int c0i = 2 * (lane >> 4);
-#pragma unroll
-      for (int cc = 0; cc < 2; cc++)
-#pragma unroll
-        for (int k = 0; k < kBasis; k++) tb[4 * cc + k] = T[(k * 6 + c0i + cc) * P + p];
+    for (int i0 = 0; i0 < kPer; i0++) {
+      const int i = min(t0 + i0 * NT, kTot - 1), row = i / W, xx = i % W, ch = row / kHrows, rr = row % kHrows;
+      const int y = (y0 + rr / (kBz + 2) - 1) & m, z = (z0 + rr % (kBz + 2) - 1) & m;
+      hv[i0] = lam[ch * P + ((size_t)y * n + z) * n + ((x0 + xx - 1) & m)];
     }
   };
-  const size_t step = (size_t)gridDim.x * kWaves;
-  size_t t = (size_t)blockIdx.x * kWaves + wave;
-  float xin[8] = {}, tb[8] = {};
-  if (t < ntiles) load_tile(xin, tb, t);
-  for (; t < ntiles; t += step) {
-    float xnext[8] = {}, tnext[8] = {};
-    if (t + step < ntiles) load_tile(xnext, tnext, t + step);
-    // layer 1: operand B the lane's own inputs
-    bf16x8 x;
+  auto store_halo = [&]() {
+    const int t0 = opaque_lane(tid);
 #pragma unroll
-    for (int j = 0; j < 8; j++) x[j] = (__bf16)xin[j];
-    f32x4 d[4];
+    for (int i0 = 0; i0 < kPer; i0++) {
+      const int i = t0 + i0 * NT, row = i / W, ch = row / kHrows, rr = row % kHrows;
+      if (i < kTot) halo[ch * kHch + rr * kHs + i % W] = hv[i0];
+    }
+  };
+  // blocks of an XCD are one contiguous range (their halos share an L2)
+  const int x8 = blockIdx.x % 8, per = gridDim.x / 8, q8 = nblk / 8, end = (x8 + 1) * q8;
+  int blk = x8 * q8 + blockIdx.x / 8;
+  if (blk < end) load_halo(blk);
+  for (; blk < end; blk += per) {
+    const int x0 = blk % nbx * kBx, z0 = blk / nbx % nbz * kBz, y0 = blk / (nbx * nbz) * kBy;
+    __syncthreads();  // the last block's halo is read
+    store_halo();
+    __syncthreads();  // (and the weights are there)
+    if (blk + per < end) load_halo(blk + per);
+#pragma unroll 1
+    for (int ty = 0; ty < kBy; ty++) {
+      const int tz = wave >> 1, tx = 16 * (wave & 1);
+      const size_t p = ((size_t)(y0 + ty) * n + z0 + tz) * n + x0 + tx + c;
+      // the basis of the stress lanes (lane < 48: point c, components 2 g + cc),
+      // in flight during the layers (from one address per tile: eight of them
+      // held across the loop would spill)
+      const size_t gp = (size_t)(2 * opaque_lane(g)) * P + p;
+      float tb[8];
+      if (lane < 48) {
+        const float* tp = T + gp;
 #pragma unroll
-    for (int ob = 0; ob < 4; ob++) d[ob] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(ob), x, bc(ob), 0, 0, 0);
-    // layers 2 and 3
+        for (int cc = 0; cc < 2; cc++)
 #pragma unroll
-    for (int layer = 1; layer < 3; layer++) {
-      const bf16x8 b0 = act_operand(d[0], d[1]), b1 = act_operand(d[2], d[3]);
-#pragma unroll
-      for (int ob = 0; ob < 4; ob++) {
-        const int blk = 4 + 8 * (layer - 1) + ob;
-        f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(blk), b0, bc(4 * layer + ob), 0, 0, 0);
-        d[ob] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(blk + 4), b1, acc, 0, 0, 0);
+          for (int k = 0; k < kBasis; k++) tb[4 * cc + k] = tp[(k * 6 + cc) * P];
       }
-    }
-    // output layer: rows 0..3 (lanes 0..15) are the basis coefficients g of
-    // point lane % 16
-    f32x4 g4;
-    {
-      const bf16x8 b0 = act_operand(d[0], d[1]), b1 = act_operand(d[2], d[3]);
-      g4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(20), b0, bc(12), 0, 0, 0);
-      g4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(21), b1, g4, 0, 0, 0);
-    }
-    // the stress: lanes < 48 take g of their point from lane lane % 16
-    float gk[kBasis];
+      // convolution
+      const float* hp = halo + (ty * (kBz + 2) + tz) * kHs + tx + c;
+      f32x4 ca = b0, cb = {0.f, 0.f, 0.f, 0.f};
+      float lg = 0.f, l4 = 0.f;  // lambda_g, and lambda_4 in group 1
+      static_for<kSteps>([&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        float v;
+        if constexpr (s < kTaps) v = hp[g * kHch + tap_off(s)];
+        else v = hp[off4[s - kTaps]];
+        if constexpr (s == 13) lg = v;
+        if constexpr (s == kTaps + 3) l4 = g == 1 ? v : 0.f;
+        f32x4& acc = s % 2 ? cb : ca;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[s], v, acc, 0, 0, 0);
+        // (the layers' weights not ahead of the convolution: registers)
+        if constexpr (s == kSteps - 1) __builtin_amdgcn_sched_barrier(0);
+      });
+      f32x4 h0;
+      f32x4 gc;  // rows 0..3 (lanes 0..15): the basis coefficients of point c
+      if constexpr (BF16) {
 #pragma unroll
-    for (int k = 0; k < kBasis; k++) gk[k] = __shfl(g4[k], lane & 15);
-    if (lane < 48) {
-      const int c0i = 2 * (lane >> 4);
-      const size_t q = 16 * t + (lane & 15);
+        for (int jj = 0; jj < 4; jj++) h0[jj] = tanh_fast(ca[jj] + cb[jj]);
+        auto wa = [&](int b) { return wt.op[b][opaque_lane(lane)]; };
+        const bf16x8 x = {(__bf16)h0[0], (__bf16)h0[1], (__bf16)h0[2], (__bf16)h0[3],
+                          (__bf16)lg,    (__bf16)l4,    (__bf16)0.f,   (__bf16)0.f};
+        f32x4 d[4];
 #pragma unroll
-      for (int cc = 0; cc < 2; cc++) {
-        float sacc = 0.f;
+        for (int ob = 0; ob < 4; ob++) d[ob] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(ob), x, bc(ob), 0, 0, 0);
 #pragma unroll
-        for (int k = 0; k < kBasis; k++) sacc = fmaf(gk[k], tb[4 * cc + k], sacc);
-        tau[(c0i + cc) * P + q] = sacc;
+        for (int layer = 1; layer < 3; layer++) {
+          const bf16x8 v0 = act_operand(d[0], d[1]), v1 = act_operand(d[2], d[3]);
+#pragma unroll
+          for (int ob = 0; ob < 4; ob++) {
+            const int b = 4 + 8 * (layer - 1) + ob;
+            const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(b), v0, bc(4 * layer + ob), 0, 0, 0);
+            d[ob] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(b + 4), v1, acc, 0, 0, 0);
+          }
+        }
+        const bf16x8 v0 = act_operand(d[0], d[1]), v1 = act_operand(d[2], d[3]);
+        gc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(20), v0, bc(12), 0, 0, 0);
+        gc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa(21), v1, gc, 0, 0, 0);
+      } else {
+        auto mm = [](float a, float b, f32x4 d) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, d, 0, 0, 0); };
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++) h0[jj] = tanhf(ca[jj] + cb[jj]);
+        f32x4 h[4], d[4];
+#pragma unroll
+        for (int ob = 0; ob < 4; ob++) {
+          const float* wr = wt.W1 + (16 * ob + c) * kIn1;
+          d[ob] = mm(wr[g], lg, bc(ob));
+          d[ob] = mm(wr[4], l4, d[ob]);
+#pragma unroll
+          for (int jj = 0; jj < 4; jj++) d[ob] = mm(wr[kLam + 4 * g + jj], h0[jj], d[ob]);
+        }
+#pragma unroll
+        for (int layer = 1; layer < 3; layer++) {
+          const float* W = layer == 1 ? wt.W2 : wt.W3;
+#pragma unroll
+          for (int ob = 0; ob < 4; ob++) {
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) h[ob][jj] = tanhf(d[ob][jj]);
+          }
+#pragma unroll
+          for (int ob = 0; ob < 4; ob++) {
+            d[ob] = bc(4 * layer + ob);
+#pragma unroll
+            for (int o = 0; o < 4; o++) {
+              const f32x4 a = *(const f32x4*)(W + (16 * ob + c) * kLd + 16 * o + 4 * g);
+#pragma unroll
+              for (int jj = 0; jj < 4; jj++) d[ob] = mm(a[jj], h[o][jj], d[ob]);
+            }
+          }
+        }
+        gc = bc(12);
+#pragma unroll
+        for (int o = 0; o < 4; o++) {
+          const f32x4 a = *(const f32x4*)(wt.W4 + (c & 3) * kLd + 16 * o + 4 * g);
+#pragma unroll
+          for (int jj = 0; jj < 4; jj++) gc = mm(a[jj], tanhf(d[o][jj]), gc);
+        }
       }
-    }
+      // the stress: lanes < 48 take the coefficients of their point from lane c
+      float gk[kBasis];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      xin[j] = xnext[j];
-      tb[j] = tnext[j];
+      for (int k = 0; k < kBasis; k++) gk[k] = __shfl(gc[k], c);
+      if (lane < 48) {
+#pragma unroll
+        for (int cc = 0; cc < 2; cc++) {
+          float sacc = 0.f;
+#pragma unroll
+          for (int k = 0; k < kBasis; k++) sacc = fmaf(gk[k], tb[4 * cc + k], sacc);
+          tau[gp + cc * P] = sacc;
+        }
+      }
     }
   }
 }
@@ -1021,29 +1050,28 @@ void launch_invariants(hipStream_t st, int prec, const void* A, size_t P, double
     hipLaunchKernelGGL(k_invariants<float>, dim3(blocks(P)), dim3(256), 0, st, (const float*)A, P, delta2, lam, T);
 }
 
+template <bool BF16>
+static void closure(hipStream_t st, const float* lam, const float* T, int n, const float* theta, float* tau) {
+  // as many work-groups as are resident (each fills the weights once and walks
+  // its blocks), at most one per block; n >= 32, so both are multiples of 8
+  static const unsigned resident = [] {
+    int dev = 0, cus = 0, per = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_closure<BF16>, 64 * kCWaves, 0) !=
+            hipSuccess ||
+        per < 1)
+      per = 1;
+    return (unsigned)((cus > 8 ? cus : 256) * per) / 8 * 8;
+  }();
+  const unsigned want = (unsigned)((size_t)n * n * n / (kBx * kBy * kBz));
+  hipLaunchKernelGGL(k_closure<BF16>, dim3(want < resident ? want : resident), dim3(64 * kCWaves), 0, st, lam, T, n,
+                     theta, tau);
+}
 void launch_predict(hipStream_t st, bool bf16, const float* lam, const float* T, int n, const float* theta,
-                    float* h0, float* tau) {
-  const size_t P = (size_t)n * n * n;
-  const unsigned one_per_thread = (unsigned)((P + 255) / 256);
-  hipLaunchKernelGGL(k_conv, dim3(one_per_thread), dim3(256), 0, st, lam, n, theta, h0);
-  if (bf16) {
-    // persistent: each wave converts the weights to operands once and then
-    // walks many 16-point tiles
-    static const unsigned resident = [] {
-      int dev = 0, cus = 0, per = 0;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_mlp_bf16, 64 * kWaves, 0) != hipSuccess ||
-          per < 1)
-        per = 1;
-      return (unsigned)((cus > 0 ? cus : 256) * per);
-    }();
-    const size_t want = (P / 16 + kWaves - 1) / kWaves;
-    const unsigned grid = (unsigned)(want < resident ? want : resident);
-    hipLaunchKernelGGL(k_mlp_bf16, dim3(grid), dim3(64 * kWaves), 0, st, lam, h0, T, n, theta, tau);
-  }
-  else
-    hipLaunchKernelGGL(k_mlp_f32, dim3(one_per_thread), dim3(256), 0, st, lam, h0, T, n, theta, tau);
+                    float* tau) {
+  if (bf16) closure<true>(st, lam, T, n, theta, tau);
+  else closure<false>(st, lam, T, n, theta, tau);
 }
 
 void launch_add_stress(hipStream_t st, int prec, void* ux, const float* tau, size_t P) {

@@ -118,6 +118,36 @@ def _theta(seed):
     return th.astype(np.float32)
 
 
+@pytest.mark.parametrize("n", [64, 128])
+def test_predict_blocks_match_oracle(O, P, n):
+    """several blocks along x and several per work-group (the next block's
+    halo loaded ahead): random features, points on every side of a block
+    and of the periodic box; the bounds are those of the test below"""
+    print("[gpu case] sgs predict blocks", n, flush=True)
+    rng = np.random.default_rng(n)
+    lam = (0.5 * rng.standard_normal((5, n, n, n))).astype(np.float32)
+    T = rng.standard_normal((4, 6, n, n, n)).astype(np.float32)
+    theta = _theta(5)
+    m = P.Closure(n)
+    try:
+        m.put_fields(lam, T)
+        m.set_params(theta)
+        m.predict(bf16=False)
+        got32 = m.field(P.SGS_PREDICTED)
+        m.predict(bf16=True)
+        got16 = m.field(P.SGS_PREDICTED)
+    finally:
+        m.close()
+    at = np.array([0, 1, 3, 4, 15, 16, 31, 32, n // 2, n - 5, n - 1])
+    pts = np.array([(y, z, x) for y in at for z in at for x in at])
+    y, z, x = pts.T
+    X0 = SG.conv_inputs(lam.astype(np.float64), pts)
+    want, _ = SG.forward(theta.astype(np.float64), X0, lam[:, y, z, x].T.astype(np.float64),
+                         T.reshape(4, 6, n, n, n)[:, :, y, z, x].transpose(2, 0, 1).astype(np.float64))
+    assert rel(got32[:, y, z, x], want.T) < 1e-5
+    assert rel(got16[:, y, z, x], want.T) < 3e-2
+
+
 def test_predict_fp32_and_bf16_match_oracle(O, P):
     print("[gpu case] sgs predict", flush=True)
     n = 32
