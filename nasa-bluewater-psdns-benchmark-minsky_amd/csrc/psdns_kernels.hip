@@ -501,34 +501,48 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
 
 // ---------------------------------------------------------------------------
 // x pass building blocks (kxcomm2.f:278-333 inverse, xkcomm1.f:97,135
-// forward): a tile is one y and B consecutive z.  The inverse transform
-// gathers its x lines from xi[v][y][kx][z] in 64-byte runs along z
-// (transposed mapping); the forward transform writes its x lines into the
-// kx blocks of X (natural mapping: each wave writes 64-byte runs, and the
-// tile's B lines together fill B x 64 contiguous bytes per block).  The real transform of length n runs as
-// a complex transform of length m = n/2 on packed pairs (x[2i], x[2i+1]).
+// forward): a tile is one y and B consecutive z.  Two neighbouring real lines
+// a (z even) and b run as one complex transform of length n: inverse, Z[k] =
+// A[k] + i B[k] for k < n/2 and conj A[n-k] + i conj B[n-k] above, whose
+// transform is a(x) + i b(x); forward, 2 A[k] = Z[k] + conj Z[n-k] and 2 B[k] =
+// -i (Z[k] - conj Z[n-k]).  Against a complex transform of length n/2 per line
+// on packed pairs (x[2i], x[2i+1]) that saves the twiddles of the real-data
+// steps, half of their sums and half of the forward step's reads of the
+// transform's result, in a pass that VALU, LDS and HBM bound together: the fused
+// pass per launch 8.07 -> 7.71 ms at 1024^3 FP32 (two work-groups of 4 waves
+// with 16 points per thread per CU; 8.73 with 8 points), 18.16 -> 16.84 ms FP64
+// (8 points), 873 -> 858 us at 512^3 FP32, 1909 -> 1805 us FP64, with two
+// scalars 2068 -> 1924 us, 256^3 FP64 240 -> 233 us.
+// The inverse transform takes its lines from xi[v][y][kx][z] in 64-byte runs
+// along z (transposed mapping; the two lines of a pair are one 16-byte read);
+// the forward transform writes its lines into the kx blocks of X (natural
+// mapping: the tile's B lines together fill B x 64 contiguous bytes per block).
 // ---------------------------------------------------------------------------
 template <typename R, int N>
 struct XPass {
   static constexpr int M = N / 2;
-  // points per thread: 8 from M = 256 on (three stages, 8 8 4, where four of
-  // radix 4 exchanged through LDS once more: 512^3 FP32 1.14 -> 0.87 ms per
-  // launch, with two scalars 2.81 -> 2.07 ms), 4 below (M = 64 with 8 is
-  // slower, 33 against 25 us at 128^3 FP32; M = 128 the same either way)
-  static constexpr int E = M >= 256 ? 8 : Team<M, 8>::E, T = M / E;
-  static constexpr int K = RunLines<R>::B;          // one 64-byte run of z (or of kx in X)
+  static constexpr int K = RunLines<R>::B;  // one 64-byte run of z (or of kx in X)
   // z lines per tile (one run; two runs per tile measured slower: the
   // LDS of 16 lines leaves one work-group per CU)
-  static constexpr int B = K;
-  static constexpr int NT = B * T;
+  static constexpr int B = K, PB = B / 2;
+  // points per thread, up to 16 in FP32 and 8 in FP64 (16 of its accumulators
+  // do not fit the registers)
+  static constexpr int EMAX = sizeof(R) == 4 ? 16 : 8;
+  static constexpr int E = Team<N, EMAX>::E, T = N / E;
+  static constexpr int NT = PB * T;
+  // waves per SIMD the registers of the fused pass are sized for
+  static constexpr int kWaves = E >= 16 ? 2 : 4;
 #ifndef PSDNS_XMFMA
 #define PSDNS_XMFMA 0
 #endif
   // radix-8 stages on the matrix cores: 0 VALU (default), 1 FP32 MFMA,
   // 2 split bf16 x 3 (a tuning build: build.py --define PSDNS_XMFMA=1)
   static constexpr int MX = PSDNS_XMFMA;
-  using FI = TeamFft<R, M, E, B, +1, LineShift<E, B>::IN, MX>;
-  using FF = TeamFft<R, M, E, B, -1, LineShift<E, B>::IN, MX>;
+  // line stride: bank model of the transposed first stage's writes, 2-way at
+  // most on 32 and 64 banks
+  static constexpr int SX = E >= 8 ? 4 : 2;
+  using FI = TeamFft<R, N, E, PB, +1, SX, MX>;
+  using FF = TeamFft<R, N, E, PB, -1, SX, MX>;
   static constexpr int kLdsReals = FI::kLdsReals;
   static constexpr int kTw = FI::kTwEntries;  // shared by FI and FF
 #ifndef PSDNS_XFRESH
@@ -538,76 +552,18 @@ struct XPass {
   // over tiles)
   static constexpr bool XFRESH = PSDNS_XFRESH;
 
-  // LDS tables of a work-group: stage twiddles (from tw of length N, every
-  // second entry) and xtw[k] = exp(-2 pi i k / N), k < M, for the real-data
-  // pre/post-processing (read before the first barrier of a transform, so
-  // fill ends with one).
-  static __device__ __forceinline__ void fill(C<R>* stw, C<R>* xtw, const C<R>* __restrict__ tw) {
-    FI::template fill_twiddles<2>(stw, tw, threadIdx.x, NT);
-    for (int k = threadIdx.x; k < M; k += NT) xtw[k] = tw[k];
+  // stage twiddles of a work-group in LDS (fill ends with a barrier)
+  static __device__ __forceinline__ void fill(C<R>* stw, const C<R>* __restrict__ tw) {
+    FI::template fill_twiddles<1>(stw, tw, threadIdx.x, NT);
     __syncthreads();
   }
 
-  // c2r of one xi variable (kx < max_al_x nonzero; kx Nyquist zero; Im X[0]
-  // ignored): Z[k] = (X[k] + conj X[m-k]) + i e^{+2 pi i k/n} (X[k] - conj X[m-k]).
-  // c2r_load issues the gathered loads of X[k] and X[m-k] (transposed
-  // mapping, no branch: out-of-range lanes read zeros without a memory
-  // access); c2r_finish forms Z and transforms it, leaving the packed
-  // physical values (x[2i], x[2i+1]) of this thread's line in the natural
-  // mapping.  Splitting the two lets a variable's loads be in flight during
-  // the transform of the previous one.
-  // Z[k] = (X[k] + conj X[m-k]) + i conj(t) (X[k] - conj X[m-k]) with
-  // t = e^{-2 pi i k/n}, the products fused into the sums
-  static __device__ __forceinline__ C<R> c2r_point(C<R> xk, C<R> xm, C<R> t) {
-    const C<R> sm = {xk.x + xm.x, xk.y - xm.y};
-    const C<R> d = {xk.x - xm.x, xk.y + xm.y};
-    return {fmar(t.y, d.x, fmar(-t.x, d.y, sm.x)),
-            fmar(t.y, d.y, fmar(t.x, d.x, sm.y))};
-  }
-  struct Raw {
-    C<R> k[E], m[E];
-  };
-  static __device__ __forceinline__ void c2r_load(Raw& r, const C<R>* __restrict__ xi, int var, int y, int z0,
-                                                  const Geo& g) {
-    const int tid = threadIdx.x;
-    const int l = FI::transposed_line(tid), q = (int)((unsigned)tid / B);
-    const BufView<R> src(xi + xiidx(var, y, 0, z0, g), kOob);
-#pragma unroll
-    for (int j = 0; j < E; j++) {
-      const int k = q + T * j;
-      const int km = M - k;
-      r.k[j] = src.load(k < g.max_al_x ? ((unsigned)k * N + l) * (unsigned)sizeof(C<R>) : kOob);
-      r.m[j] = src.load(km < g.max_al_x ? ((unsigned)km * N + l) * (unsigned)sizeof(C<R>) : kOob);
-    }
-  }
-  static __device__ __forceinline__ void c2r_finish(C<R>* v, Raw& r, R* lds, const C<R>* stw, const C<R>* xtw) {
-    const int tid = threadIdx.x;
-    const Slot<R> in = FI::transposed(lds, tid);
-    const Slot<R> out = FI::natural(lds, tid);
-#pragma unroll
-    for (int j = 0; j < E; j++) {
-      const int k = in.q + T * j;  // k > 0 for j > 0
-      C<R> xk = r.k[j];
-      if (j == 0 && k == 0) xk.y = 0;
-      const C<R> xm = r.m[j];
-      v[j] = c2r_point(xk, xm, xtw[k]);
-    }
-    FI::template run<false, true, true, false>(v, lds, in, out, stw);
-  }
-  static __device__ __forceinline__ void c2r(C<R>* v, const C<R>* __restrict__ xi, int var, int y, int z0,
-                                             const Geo& g, R* lds, const C<R>* stw, const C<R>* xtw) {
-    Raw r;
-    c2r_load(r, xi, var, y, z0, g);
-    c2r_finish(v, r, lds, stw, xtw);
-  }
-
-  // Staged variant for the fused pass: one variable of a tile, rows kx =
-  // 0..M-1 of B consecutive z (64 bytes per row; rows kx >= max_al_x and
-  // past the last tile read as zeros), is copied by the memory system
-  // straight into an LDS staging buffer S[M][B] (16 bytes per lane, no
-  // registers), so the copy of the next variable runs under the transform
-  // of the current one.  Each wave copies whole 16-row slices.
-  static constexpr int kStageBytes = M * B * (int)sizeof(C<R>);
+  // One variable of a tile, rows kx = 0..M-1 of B consecutive z (64 bytes
+  // per row; rows kx >= max_al_x and past the last tile read as zeros), is
+  // copied by the memory system straight into an LDS staging buffer S[M][B]
+  // (16 bytes per lane, no registers), so the copy of the next variable runs
+  // under the transform of the current one.  Each wave copies whole 16-row
+  // slices.
   static __device__ __forceinline__ void stage_load(C<R>* S, const C<R>* __restrict__ xi, int var, int y, int z0,
                                                     const Geo& g, bool valid) {
     constexpr int kRowBytes = B * (int)sizeof(C<R>);  // whole 64-byte runs
@@ -646,23 +602,31 @@ struct XPass {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
-  // c2r of the staged variable: c2r_staged_pre forms Z[k] from S[k] and
-  // conj S[m-k] (transposed mapping: 8 lanes read one 64-byte row) and ends
-  // with a barrier, after which S may be refilled; c2r_staged_fft then
-  // transforms
-  static __device__ __forceinline__ void c2r_staged_pre(C<R>* v, const C<R>* S, const C<R>* xtw) {
+  // c2r of the staged variable: c2r_staged_pre forms Z[k] of the pair's lines
+  // (transposed mapping) and ends with a barrier, after which S may be
+  // refilled; c2r_staged_fft then transforms: v[j] = (a, b) at x = q + T j of
+  // this thread's pair in the natural mapping.  kx Nyquist is zero, Im A[0]
+  // and Im B[0] are ignored.
+  static __device__ __forceinline__ void c2r_staged_pre(C<R>* v, const C<R>* S) {
     const int tid = opaque(threadIdx.x);  // per tile, not hoisted out of the tile loop
-    const int l = FI::transposed_line(tid), q = (int)((unsigned)tid / B);
+    const int l = FI::transposed_line(tid), q = (int)((unsigned)tid / PB);
+    struct alignas(2 * sizeof(C<R>) < 16 ? 2 * sizeof(C<R>) : 16) Two {
+      C<R> a, b;
+    };
+    const Two* rows = reinterpret_cast<const Two*>(S) + l;
 #pragma unroll
     for (int j = 0; j < E; j++) {
-      // k > 0 for j > 0; for k = 0 the row read (k itself) is discarded: X[m]
-      // (kx Nyquist) is zero
       const int k = q + T * j;
-      C<R> xk = S[k * B + l];
-      const C<R> xr = S[(j == 0 ? (M - k) & (M - 1) : M - k) * B + l];
-      if (j == 0 && k == 0) xk.y = 0;
-      const C<R> xm = j == 0 && k == 0 ? C<R>{0, 0} : xr;
-      v[j] = c2r_point(xk, xm, xtw[k]);
+      if (j < E / 2) {
+        Two t = rows[k * PB];
+        if (j == 0 && k == 0) t.a.y = t.b.y = 0;
+        v[j] = {t.a.x - t.b.y, t.a.y + t.b.x};
+      } else {
+        // row n - k (k = n/2: row 0 is read and discarded)
+        const Two t = rows[(j == E / 2 ? (N - k) & (M - 1) : N - k) * PB];
+        v[j] = {t.a.x + t.b.y, t.b.x - t.a.y};
+        if (j == E / 2 && k == M) v[j] = {0, 0};
+      }
     }
     lds_barrier();
   }
@@ -671,14 +635,13 @@ struct XPass {
     FI::template run<false, true, true, false>(v, lds, FI::transposed(lds, tid), FI::natural(lds, tid), stw);
   }
 
-  // r2c of packed physical values v of this thread's line, scaled by
-  // `scale` / 2: the last stage leaves Z in LDS; 2 X[k] = (Z[k] + conj Z[m-k])
-  // - i e^{-2 pi i k/n} (Z[k] - conj Z[m-k]) for kx < max_al_x (kx Nyquist
-  // dropped).  Without SCALE the values stored are 2 X[k] unnormalized, n
-  // times the transform / n (x 2n, exact in binary).
+  // r2c of the physical values v of this thread's pair, scaled by `scale` / 2:
+  // the last stage leaves Z in LDS; 2 A[k] and 2 B[k] for kx < max_al_x (kx
+  // Nyquist dropped).  Without SCALE the values stored are the transform x 2
+  // unnormalized, n times the transform / n (x 2n, exact in binary).
   template <bool SCALE>
   static __device__ __forceinline__ void r2c(C<R>* v, C<R>* __restrict__ xs, int var, int y, int z0,
-                                             const Geo& g, R* lds, const C<R>* stw, const C<R>* xtw, R scale) {
+                                             const Geo& g, R* lds, const C<R>* stw, R scale) {
     const int tid = XFRESH ? opaque(threadIdx.x) : (int)threadIdx.x;
     const Slot<R> s = FF::natural(lds, tid);
     FF::template run<true, XFRESH, false, false>(v, lds, s, s, stw);
@@ -686,35 +649,37 @@ struct XPass {
     // no branch per point: kx >= max_al_x lanes store nothing (out of range)
     const BufView<R> dst(xs + xidx<K>(var, y, z0, 0, g), kOob);
     const int q = s.q;
-    const unsigned lofs = (unsigned)FF::natural_line(tid) * K;
+    const unsigned lofs = (unsigned)(2 * FF::natural_line(tid)) * K;
     const R half = (R)0.5 * scale;
     // with T a multiple of K, point k = q + T j lies in kx block q / K + j T / K
     // at q % K: one lane offset, and j's part in the scalar offset
     const unsigned qu = (unsigned)q;
     const unsigned vq = (lofs + qu / K * (unsigned)(N * K) + qu % K) * (unsigned)sizeof(C<R>);
-    // m - k = (T - q) + (m - T (j + 1)) for j > 0: a lane part (kept opaque so
-    // that it is not folded back into m - k) and a constant
+    // n - k = (T - q) + (n - T (j + 1)): a lane part (kept opaque so that it
+    // is not folded back into n - k) and a constant
     const int tq = opaque(T - q);
 #pragma unroll
-    for (int j = 0; j < E; j++) {
+    for (int j = 0; j < E / 2; j++) {
       const int k = q + T * j;  // k > 0 for j > 0
-      const int pk = FF::out_pos(k), pm = FF::out_pos(j == 0 ? (M - k) & (M - 1) : tq + (M - T * (j + 1)));
-      const C<R> zk = {s.re[pk], s.im[pk]};
-      const C<R> zm = {s.re[pm], -s.im[pm]};  // conj Z[m-k]
-      const C<R> sm = zk + zm;
-      const C<R> d = zk - zm;
-      const C<R> t = xtw[k];
-      // sm - i t d, the products fused into the sums
-      C<R> o = {fmar(t.y, d.x, fmar(t.x, d.y, sm.x)),
-                fmar(t.y, d.y, fmar(-t.x, d.x, sm.y))};
-      if constexpr (SCALE) o = cscale(o, half);
+      const int pk = FF::out_pos(k), pm = FF::out_pos(j == 0 ? (N - k) & (N - 1) : tq + (N - T * (j + 1)));
+      const C<R> zk = {s.re[pk], s.im[pk]}, zm = {s.re[pm], s.im[pm]};
+      C<R> oa = {zk.x + zm.x, zk.y - zm.y}, ob = {zk.y + zm.y, zm.x - zk.x};
+      if constexpr (SCALE) {
+        oa = cscale(oa, half);
+        ob = cscale(ob, half);
+      }
+      constexpr unsigned kNext = K * (unsigned)sizeof(C<R>);  // line b: the next z of the block
       if constexpr (T % K == 0) {
         // k < max_al_x as q < max_al_x - T j (a scalar bound)
         const int lim = __builtin_amdgcn_readfirstlane(g.max_al_x - T * j);
-        dst.store(q < lim ? vq : kOob, o, (unsigned)(j * (T / K) * N * K * (int)sizeof(C<R>)));
+        const unsigned so = (unsigned)(j * (T / K) * N * K * (int)sizeof(C<R>));
+        dst.store(q < lim ? vq : kOob, oa, so);
+        dst.store(q < lim ? vq + kNext : kOob, ob, so);
       } else {
         const unsigned ku = (unsigned)k;
-        dst.store(k < g.max_al_x ? (lofs + ku / K * (unsigned)(N * K) + ku % K) * (unsigned)sizeof(C<R>) : kOob, o);
+        const unsigned o = (lofs + ku / K * (unsigned)(N * K) + ku % K) * (unsigned)sizeof(C<R>);
+        dst.store(k < g.max_al_x ? o : kOob, oa);
+        dst.store(k < g.max_al_x ? o + kNext : kOob, ob);
       }
     }
   }
@@ -746,9 +711,9 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
   using X = XPass<R, N>;
   constexpr int E = X::E, B = X::B, NZB = N / B;
   __shared__ R lds[X::kLdsReals];
-  __shared__ C<R> stw[X::kTw], xtw[X::M];
+  __shared__ C<R> stw[X::kTw];
   __shared__ __attribute__((aligned(16))) C<R> S[X::M * B];
-  X::fill(stw, xtw, tw);
+  X::fill(stw, tw);
   const int var = blockIdx.y;
   const TileWalk w = tile_walk(N * NZB);
   double s[MOM ? 8 : 1];
@@ -761,7 +726,7 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
       const int y = t / NZB, z0 = (t % NZB) * B, tn = t + w.step;
       C<R> v[E];
       X::stage_publish();
-      X::c2r_staged_pre(v, S, xtw);
+      X::c2r_staged_pre(v, S);
       if (tn < w.end) X::stage_load(S, xi, var, tn / NZB, (tn % NZB) * B, g, true);
       X::c2r_staged_fft(v, lds, stw);
       if constexpr (MOM) {
@@ -785,9 +750,12 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
         }
       } else {
         const int tid = opaque(threadIdx.x), line = X::FI::natural_line(tid), q = (int)((unsigned)tid % X::T);
-        C<R>* dst = reinterpret_cast<C<R>*>(ux + (((size_t)var * N + y) * N + z0 + line) * N);
+        R* dst = ux + (((size_t)var * N + y) * N + z0 + 2 * line) * N;
 #pragma unroll
-        for (int j = 0; j < E; j++) dst[q + X::T * j] = v[j];
+        for (int j = 0; j < E; j++) {
+          dst[q + X::T * j] = v[j].x;
+          dst[N + q + X::T * j] = v[j].y;
+        }
       }
       if (tn >= w.end) break;
       t = tn;
@@ -833,17 +801,17 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
     k_x_r2c(const R* __restrict__ ux, C<R>* __restrict__ xs, Geo g, const C<R>* __restrict__ tw) {
   using X = XPass<R, N>;
   __shared__ R lds[X::kLdsReals];
-  __shared__ C<R> stw[X::kTw], xtw[X::M];
-  X::fill(stw, xtw, tw);
+  __shared__ C<R> stw[X::kTw];
+  X::fill(stw, tw);
   const int2 blk = xcd_block2();
   const int var = blk.y;
   const int y = blk.x / (N / X::B), z0 = (blk.x % (N / X::B)) * X::B;
   const int line = X::FF::natural_line(threadIdx.x), q = threadIdx.x % X::T;
-  const C<R>* src = reinterpret_cast<const C<R>*>(ux + (((size_t)var * N + y) * N + z0 + line) * N);
+  const R* src = ux + (((size_t)var * N + y) * N + z0 + 2 * line) * N;
   C<R> v[X::E];
 #pragma unroll
-  for (int j = 0; j < X::E; j++) v[j] = src[q + X::T * j];
-  X::template r2c<true>(v, xs, var, y, z0, g, lds, stw, xtw, (R)1 / (R)N);
+  for (int j = 0; j < X::E; j++) v[j] = {src[q + X::T * j], src[N + q + X::T * j]};
+  X::template r2c<true>(v, xs, var, y, z0, g, lds, stw, (R)1 / (R)N);
 }
 
 // velmax (realspace_vel.f:108-110) is a maximum over the whole grid: each
@@ -917,7 +885,7 @@ __device__ __forceinline__ R product(int s, R u, R v, R w) {
 #endif
 template <typename R, int N, bool TAU, bool SC = false>
 __global__ void __launch_bounds__((XPass<R, N>::NT))
-__attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : 4, SC ? PSDNS_XSC_WAVES : 4)))
+__attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : XPass<R, N>::kWaves, SC ? PSDNS_XSC_WAVES : XPass<R, N>::kWaves)))
     k_x_fused(const C<R>* __restrict__ xi, C<R>* __restrict__ xs, Geo g, const C<R>* __restrict__ tw,
               unsigned long long* __restrict__ velmax, int want_velmax, const float* __restrict__ tau, int nsc,
               ScGrad scg) {
@@ -925,9 +893,9 @@ __attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : 4, SC ? PSDNS_XSC_WAVE
   using X = XPass<R, N>;
   constexpr int E = X::E, B = X::B;
   __shared__ R lds[X::kLdsReals];
-  __shared__ C<R> stw[X::kTw], xtw[X::M];
+  __shared__ C<R> stw[X::kTw];
   __shared__ __attribute__((aligned(16))) C<R> S[X::M * B];
-  X::fill(stw, xtw, tw);
+  X::fill(stw, tw);
   constexpr int NZB = N / B;
   const TileWalk w = tile_walk(N * NZB);
   int t = w.t;
@@ -938,15 +906,15 @@ __attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : 4, SC ? PSDNS_XSC_WAVE
       const int y = t / NZB, z0 = (t % NZB) * B;
       C<R> pu[E], pv[E], pw[E];
       X::stage_publish();
-      X::c2r_staged_pre(pu, S, xtw);
+      X::c2r_staged_pre(pu, S);
       X::stage_load(S, xi, 1, y, z0, g, true);
       X::c2r_staged_fft(pu, lds, stw);
       X::stage_publish();
-      X::c2r_staged_pre(pv, S, xtw);
+      X::c2r_staged_pre(pv, S);
       X::stage_load(S, xi, 2, y, z0, g, true);
       X::c2r_staged_fft(pv, lds, stw);
       X::stage_publish();
-      X::c2r_staged_pre(pw, S, xtw);
+      X::c2r_staged_pre(pw, S);
       const int tn = t + w.step;
       const bool more = tn < w.end;
       if (SC) X::stage_load(S, xi, 3, y, z0, g, true);
@@ -966,7 +934,7 @@ __attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : 4, SC ? PSDNS_XSC_WAVE
           for (int d = 0; d < 3; d++) {
             C<R> pb[E];
             X::stage_publish();
-            X::c2r_staged_pre(pb, S, xtw);
+            X::c2r_staged_pre(pb, S);
             if (d < 2 || s + 1 < nsc) X::stage_load(S, xi, 4 + 3 * s + d, y, z0, g, true);
             else if (more) X::stage_load(S, xi, 0, tn / NZB, (tn % NZB) * B, g, true);
             X::c2r_staged_fft(pb, lds, stw);
@@ -978,7 +946,7 @@ __attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : 4, SC ? PSDNS_XSC_WAVE
               acc[j] = d == 0 ? tj : acc[j] + tj;
             }
           }
-          X::template r2c<true>(acc, xs, 5 + s, y, z0, g, lds, stw, xtw, (R)1 / (R)N);
+          X::template r2c<true>(acc, xs, 5 + s, y, z0, g, lds, stw, (R)1 / (R)N);
         }
       }
 #pragma unroll
@@ -988,23 +956,23 @@ __attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : 4, SC ? PSDNS_XSC_WAVE
         for (int j = 0; j < E; j++)
           q[j] = {product(sl, pu[j].x, pv[j].x, pw[j].x), product(sl, pu[j].y, pv[j].y, pw[j].y)};
         if constexpr (TAU) {
-          // this thread's points: x = 2 i, 2 i + 1, i = q + T j, of line z0 + line
+          // this thread's points: x = q + T j of the lines z0 + 2 line and the next
           constexpr size_t P3 = (size_t)N * N * N;
           const int line = X::FI::natural_line(threadIdx.x), qq = (int)(threadIdx.x % X::T);
-          const float* base = tau + ((size_t)y * N + z0 + line) * N + 2 * qq;
+          const float* base = tau + ((size_t)y * N + z0 + 2 * line) * N + qq;
           constexpr int ca[5] = {0, 1, 5, 4, 2}, cb[5] = {3, -1, 3, -1, -1};  // + tau[ca] - tau[cb]
 #pragma unroll
           for (int j = 0; j < E; j++) {
-            const float2 a = *reinterpret_cast<const float2*>(base + ca[sl] * P3 + 2 * X::T * j);
-            float2 t = a;
+            const float* p = base + X::T * j;
+            float ta = p[ca[sl] * P3], tb = p[ca[sl] * P3 + N];
             if (cb[sl] >= 0) {
-              const float2 b = *reinterpret_cast<const float2*>(base + cb[sl] * P3 + 2 * X::T * j);
-              t = make_float2(a.x - b.x, a.y - b.y);
+              ta -= p[cb[sl] * P3];
+              tb -= p[cb[sl] * P3 + N];
             }
-            q[j] = {q[j].x + (R)t.x, q[j].y + (R)t.y};
+            q[j] = {q[j].x + (R)ta, q[j].y + (R)tb};
           }
         }
-        X::template r2c<false>(q, xs, sl, y, z0, g, lds, stw, xtw, (R)1);
+        X::template r2c<false>(q, xs, sl, y, z0, g, lds, stw, (R)1);
       }
       if (!more) break;
       t = tn;
