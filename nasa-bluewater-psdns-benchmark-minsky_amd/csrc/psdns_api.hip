@@ -106,9 +106,10 @@ struct psdns_ctx {
   double* d_fac = nullptr;     // xfac[nxh], yfac[n], zfac[n]
   double* h_fac = nullptr;     // pinned host staging of the same, one copy per upload
   // after the factors in the same pinned allocation, what kernels write to
-  // the host: velmax's bits, then the FEK energies (launch_ek_force)
+  // the host: velmax's bits, the FEK energies (launch_ek_force), and 2 n + 2
+  // doubles for the shell statistics and the moments
   unsigned long long* h_velmax = nullptr;
-  double* h_ek = nullptr;
+  double *h_ek = nullptr, *h_stat = nullptr;
   bool velmax_clear = false;   // the velmax slots are zero
   double* d_red = nullptr;     // reductions scratch: [2 + 2*n + n]
   unsigned long long* d_velmax = nullptr;
@@ -549,11 +550,12 @@ int psdns_create(const psdns_params* p, psdns_ctx** out) {
   ALLOC(c->d_shiftr, c->csize() * 2 * (c->nxh + 2 * n));
   ALLOC(c->d_fac, sizeof(double) * (c->nxh + 2 * n));
   // one pinned allocation: the factors, then what kernels write to the host
-  if (hipHostMalloc((void**)&c->h_fac, sizeof(double) * (c->nxh + 2 * n + 2 + 2 * psdns::kMaxKfor),
+  if (hipHostMalloc((void**)&c->h_fac, sizeof(double) * (c->nxh + 2 * n + 2 + 2 * psdns::kMaxKfor + 2 * n + 2),
                     hipHostMallocDefault) != hipSuccess)
     return bail(fail(PSDNS_ENOMEM, "hipHostMalloc of the factor staging buffer failed"));
   c->h_velmax = (unsigned long long*)(c->h_fac + c->nxh + 2 * n);
   c->h_ek = (double*)(c->h_velmax + 1);
+  c->h_stat = c->h_ek + 2 * psdns::kMaxKfor + 1;
   ALLOC(c->d_red, sizeof(double) * (2 + 3 * (size_t)n + 64));
   ALLOC(c->d_velmax, kVelmaxBytes);
   CHK(hipMemcpy(c->d_colx, c->colx.data(), sizeof(int) * c->na, hipMemcpyHostToDevice));
@@ -967,21 +969,17 @@ int psdns_ek_force(psdns_ctx* c, int kf_shell, int kfor, const double* ekinf, do
 
 namespace {
 
-// shell statistics into part (partial rows) and out (2 nshell + 2 doubles),
-// then to the host
-int shell_stats_into(psdns_ctx* c, double* part, double* out, double* ek, double* dk, int nshell, double* tke,
-                     double* eps) {
-  psdns::launch_shell_stats(c->c, c->viscos, nshell, part, out);
-  HIPCHK(hipGetLastError());
-  double tot[2];
-  HIPCHK(hipMemcpyAsync(tot, out + 2 * nshell, sizeof tot, hipMemcpyDeviceToHost, c->c.stream));
-  if (nshell > 0) {
-    HIPCHK(hipMemcpyAsync(ek, out, sizeof(double) * nshell, hipMemcpyDeviceToHost, c->c.stream));
-    HIPCHK(hipMemcpyAsync(dk, out + nshell, sizeof(double) * nshell, hipMemcpyDeviceToHost, c->c.stream));
-  }
+// shell statistics through part (partial rows) and the pinned result buffer
+int shell_stats_into(psdns_ctx* c, double* part, double* ek, double* dk, int nshell, double* tke, double* eps) {
+  const double* out = c->h_stat;
+  psdns::launch_shell_stats(c->c, c->viscos, nshell, part, c->h_stat);
   if (int rc = sync(c)) return rc;
-  if (tke) *tke = tot[0];
-  if (eps) *eps = tot[1];
+  if (nshell > 0) {
+    std::memcpy(ek, out, sizeof(double) * nshell);
+    std::memcpy(dk, out + nshell, sizeof(double) * nshell);
+  }
+  if (tke) *tke = out[2 * nshell];
+  if (eps) *eps = out[2 * nshell + 1];
   return PSDNS_OK;
 }
 
@@ -1003,7 +1001,7 @@ int psdns_shell_stats(psdns_ctx* c, double* ek, double* dk, int nshell, double* 
     if (hipMalloc(&c->d_shell_part, bytes) != hipSuccess)
       return fail(PSDNS_ENOMEM, "hipMalloc of the shell partial rows (%zu bytes) failed", bytes);
   }
-  return shell_stats_into(c, c->d_shell_part, c->d_red, ek, dk, nshell, tke, eps);
+  return shell_stats_into(c, c->d_shell_part, ek, dk, nshell, tke, eps);
 }
 
 int psdns_shell_stats_noalloc(psdns_ctx* c, double* ek, double* dk, int nshell, double* tke, double* eps) {
@@ -1013,7 +1011,7 @@ int psdns_shell_stats_noalloc(psdns_ctx* c, double* ek, double* dk, int nshell, 
     return fail(PSDNS_EINVAL, "n = %d: psdns_shell_stats_noalloc holds partial rows for n <= %d only", c->n,
                 kScratchMaxN);
   if (!c->d_scratch) return fail(PSDNS_ESTATE, "no scratch address for device %d", c->dev);
-  return shell_stats_into(c, c->d_scratch, c->d_red, ek, dk, nshell, tke, eps);
+  return shell_stats_into(c, c->d_scratch, ek, dk, nshell, tke, eps);
 }
 
 int psdns_vg_moments(psdns_ctx* c, double* dudx, double* dwdz) {
@@ -1023,11 +1021,9 @@ int psdns_vg_moments(psdns_ctx* c, double* dudx, double* dwdz) {
   // i kx u and i kz w of un formed on load by the inverse y pass, the power
   // sums in FP64 taken by the x pass (the physical fields are not stored)
   if ((rc = pass(c, Pass::YInvGrad, 2)) || (rc = pass(c, Pass::ZInv, 2))) return rc;
-  if (psdns::launch_x_moments(c->c, c->d_red)) return fail(PSDNS_EINVAL, "unsupported grid n = %d", c->n);
-  HIPCHK(hipGetLastError());
-  double sums[16];
-  HIPCHK(hipMemcpyAsync(sums, c->d_red, sizeof sums, hipMemcpyDeviceToHost, c->c.stream));
+  if (psdns::launch_x_moments(c->c, c->h_stat)) return fail(PSDNS_EINVAL, "unsupported grid n = %d", c->n);
   if ((rc = sync(c))) return rc;
+  const double* sums = c->h_stat;
   // vgmomt.f:134-138: divided by the number of grid points
   const double n3 = (double)c->n * c->n * c->n;
   for (int m = 0; m < 8; m++) {

@@ -126,7 +126,8 @@ struct EkInf {
 void launch_ek_force(const Ctx& c, int kfor, int kf_shell, const EkInf& inf, double* terms, double* ek, double* out);
 // FP64 shell statistics in a fixed order: kShellBlocks partial rows of
 // 2 shell_rows(n) doubles in part, then out[0..nshell) = E,
-// out[nshell..2 nshell) = D, out[2 nshell] = TKE, out[2 nshell + 1] = eps
+// out[nshell..2 nshell) = D, out[2 nshell] = TKE, out[2 nshell + 1] = eps (out:
+// pinned host memory)
 constexpr int kShellBlocks = 1024;
 // shells a mask mode can reach: ik = int(|k| + 1.5) with 9 |k|^2 <= 2 n^2
 constexpr int shell_rows(int n) {
@@ -152,7 +153,7 @@ int launch_y_grad(const Ctx& c, const void* phi, void* yw);
 int launch_sc_update(const Ctx& c, int stage, void* u, void* un, const void* tr, double dt2, double rpr,
                      double* dif, void* u1 = nullptr);
 // velocity-gradient moments: the x c2r of xi slots 0 and 1 and the FP64 sums
-// of the powers 1..8 of its values, out[16] (X is overwritten)
+// of the powers 1..8 of its values, out[16] (pinned host memory; X is overwritten)
 int launch_x_moments(const Ctx& c, double* out);
 // EPFOR forcing increments on u (and un): mode 1 proc4a/advanc_1 (sphere,
 // per-entry tally terms[3 nlist], then efkz[3 nxh] folded in list order),

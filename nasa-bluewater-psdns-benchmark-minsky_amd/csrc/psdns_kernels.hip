@@ -779,20 +779,23 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
 }
 
 // out[8 var + m - 1] = the sum of the nb partial rows of variable blockIdx.x
-__global__ void __launch_bounds__(256) k_moments_fold(const double* __restrict__ part, int nb, double* __restrict__ out) {
-  __shared__ double red[256];
+// (out: pinned host memory)
+constexpr int kMomFold = 1024;
+__global__ void __launch_bounds__(kMomFold)
+    k_moments_fold(const double* __restrict__ part, int nb, double* __restrict__ out) {
+  __shared__ double red[kMomFold];
   const int m = threadIdx.x & 7, q = threadIdx.x >> 3;
   const double* p = part + (size_t)blockIdx.x * nb * 8 + m;
   double v = 0.0;
-#pragma unroll 4
-  for (int i = q; i < nb; i += 32) v += p[(size_t)i * 8];
+#pragma unroll 8
+  for (int i = q; i < nb; i += kMomFold / 8) v += p[(size_t)i * 8];
   red[threadIdx.x] = v;
   __syncthreads();
-  if (q == 0) {
-    double r = 0.0;
-    for (int i = 0; i < 32; i++) r += red[8 * i + m];
-    out[8 * blockIdx.x + m] = r;
+  for (int h = kMomFold / 2; h >= 8; h >>= 1) {
+    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+    __syncthreads();
   }
+  if (threadIdx.x < 8) out[8 * blockIdx.x + m] = red[threadIdx.x];
 }
 
 // forward x pass alone: physical ux (nv variables) -> X, x 1/n
@@ -1868,8 +1871,8 @@ __global__ void __launch_bounds__(256)
 // D(ik) = 2 nu k^2 E over the mask, ik = int(|k| + 1.5), FP64, with the same
 // bits on every run.  Work-group b owns the fixed column range
 // [b na / B, (b + 1) na / B); each wave takes one column at a time and walks
-// its two y halves (ky >= 0, then ky < 0) in chunks of 64 lanes ordered by
-// |ky| descending, in which the shell index is monotone, so the lanes of one
+// |ky| descending in chunks of 64 lanes, the points ky and -ky (one shell) of
+// a lane summed first; the shell index is monotone, so the lanes of one
 // shell are contiguous: the wave's inclusive prefix sums (DPP moves, a fixed
 // tree) give each shell's run as the difference of the sums at its last
 // lane and before its first, and only the run's last lane adds it to the
@@ -1880,7 +1883,9 @@ __global__ void __launch_bounds__(256)
 // work-group then adds its wave histograms in wave order into its partial
 // row part[b][0..nh) (E) and part[b][nh..2 nh) (D); k_shell_fold_rows and
 // k_shell_fold sum the rows in two fixed levels.  No atomics: the result
-// depends on B only.
+// depends on B only.  512^3 FP32: 274 us with ky and -ky scanned apart and
+// every chunk of the cylinder visited, 159 us this way (0.75 GB on the mask,
+// 4.7 TB/s).
 // ---------------------------------------------------------------------------
 // Inclusive sum over the 64 lanes of a wave with DPP moves only: row shifts
 // by 1, 2, 4 and 8 within each row of 16 lanes, then the total of row 0
@@ -1905,7 +1910,7 @@ __device__ __forceinline__ double wave_prefix_sum(double x) {
 }
 
 constexpr int kShellWaves = 8;      // waves per work-group of k_shell_partial
-constexpr int kShellChunks = 8;     // 64-entry chunks of a column half per pass
+constexpr int kShellChunks = 4;     // 64-entry chunks of |ky| per pass
 
 template <typename R>
 __global__ void __launch_bounds__(64 * kShellWaves)
@@ -1924,56 +1929,58 @@ __global__ void __launch_bounds__(64 * kShellWaves)
     const double tf = x == 0 ? 1.0 : 2.0;
     const BufView<R> s0(un + (size_t)a * n, kOob), s1(un + tot + (size_t)a * n, kOob),
         s2(un + 2 * tot + (size_t)a * n, kOob);
-    for (int half = 0; half < 2; half++) {
-      // half 0: y = 0 .. n/2 - 1; half 1: y = n/2 + 1 .. n - 1
-      const int ylo = half == 0 ? 0 : n / 2 + 1, yhi = half == 0 ? n / 2 : n;
-      // the lanes of a chunk in |ky| descending order (reversed in half 0)
-      const int yl = half == 0 ? 63 - lane : lane;
-      for (int y0 = ylo; y0 < yhi; y0 += 64 * kShellChunks) {
-        // off-mask points (about a third of the cylinder) are not read
-        C<R> v[kShellChunks][3];
+    // chunks above the mask's largest |ky| of this column hold nothing
+    const float ky2 = fmaxf((float)(2 * n * n / 9 - x * x - kz * kz), 0.f);
+    const int kmax = min(n / 2 - 1, (int)__fsqrt_rn(ky2) + 1);
+    for (int kc = __builtin_amdgcn_readfirstlane(kmax / 64); kc >= 0; kc -= kShellChunks) {
+      // off-mask points (about a third of the cylinder) are not read
+      C<R> vp[kShellChunks][3], vm[kShellChunks][3];
 #pragma unroll
-        for (int c = 0; c < kShellChunks; c++) {
-          const int y = y0 + 64 * c + yl;
-          const bool on = y < yhi && in_mask(x, kwave(y, n), kz, y, z, n);
-          const unsigned off = on ? (unsigned)y * (unsigned)sizeof(C<R>) : kOob;
-          v[c][0] = s0.load(off);
-          v[c][1] = s1.load(off);
-          v[c][2] = s2.load(off);
-        }
+      for (int c = 0; c < kShellChunks; c++) {
+        // lanes in |ky| descending order (below 0 past the last chunk)
+        const int ky = 64 * (kc - c) + 63 - lane;
+        const bool on = ky >= 0 && ky < n / 2 && in_mask(x, ky, kz, ky, z, n);
+        const unsigned op = on ? (unsigned)ky * (unsigned)sizeof(C<R>) : kOob;
+        const unsigned om = on && ky > 0 ? (unsigned)(n - ky) * (unsigned)sizeof(C<R>) : kOob;
+        vp[c][0] = s0.load(op);
+        vp[c][1] = s1.load(op);
+        vp[c][2] = s2.load(op);
+        vm[c][0] = s0.load(om);
+        vm[c][1] = s1.load(om);
+        vm[c][2] = s2.load(om);
+      }
 #pragma unroll
-        for (int c = 0; c < kShellChunks; c++) {
-          if (y0 + 64 * c >= yhi) break;  // wave-uniform
-          const int y = y0 + 64 * c + yl, ky = kwave(y, n);
-          const bool on = y < yhi && in_mask(x, ky, kz, y, z, n);
-          const int k2 = x * x + ky * ky + kz * kz;
-          const double rk2 = (double)k2;
-          // ik = int(|k| + 1.5) (ek_shell.f:66): |k|^2 is an integer below
-          // 2^24, and sqrt(k2) + 1.5 is never within 1e-4 of an integer for
-          // k2 <= 2 n^2 / 9 (n <= 1024), far more than FP32 rounding, so the
-          // FP32 square root gives the same index as FP64
-          int key = on ? (int)(__fsqrt_rn((float)k2) + 1.5f) : -1;
-          double e = 0.0;
-          if (on) {
-            double sum = 0.0;
+      for (int c = 0; c < kShellChunks; c++) {
+        if (kc - c < 0) break;  // wave-uniform
+        const int ky = 64 * (kc - c) + 63 - lane;
+        const bool on = ky < n / 2 && in_mask(x, ky, kz, ky, z, n);
+        const int k2 = x * x + ky * ky + kz * kz;
+        const double rk2 = (double)k2;
+        // ik = int(|k| + 1.5) (ek_shell.f:66): |k|^2 is an integer below
+        // 2^24, and sqrt(k2) + 1.5 is never within 1e-4 of an integer for
+        // k2 <= 2 n^2 / 9 (n <= 1024), far more than FP32 rounding, so the
+        // FP32 square root gives the same index as FP64
+        int key = on ? (int)(__fsqrt_rn((float)k2) + 1.5f) : -1;
+        // a point that was not read is zero
+        double sum = 0.0;
 #pragma unroll
-            for (int i = 0; i < 3; i++) sum += (double)v[c][i].x * v[c][i].x + (double)v[c][i].y * v[c][i].y;
-            e = 0.5 * tf * sum;
-          }
-          const double d = 2.0 * viscos * rk2 * e;
-          // runs of equal keys are contiguous: each run's sum is the
-          // difference of the wave's inclusive prefix sums at its last lane
-          // and before its first (run starts from a ballot of key changes)
-          const double pe = wave_prefix_sum(e), pd = wave_prefix_sum(d);
-          const int kp = __shfl_up(key, 1);
-          const unsigned long long starts = __ballot(lane == 0 || kp != key);
-          const int first = 63 - __clzll(starts & ((2ull << lane) - 1ull));
-          const double pe0 = __shfl(pe, first > 0 ? first - 1 : 0), pd0 = __shfl(pd, first > 0 ? first - 1 : 0);
-          const bool last = lane == 63 || (((starts >> lane) >> 1) & 1ull);
-          if (key > 0 && last) {
-            he[key - 1] += first > 0 ? pe - pe0 : pe;
-            hd[key - 1] += first > 0 ? pd - pd0 : pd;
-          }
+        for (int i = 0; i < 3; i++)
+          sum += (double)vp[c][i].x * vp[c][i].x + (double)vp[c][i].y * vp[c][i].y +
+                 ((double)vm[c][i].x * vm[c][i].x + (double)vm[c][i].y * vm[c][i].y);
+        const double e = on ? 0.5 * tf * sum : 0.0;
+        const double d = 2.0 * viscos * rk2 * e;
+        // runs of equal keys are contiguous: each run's sum is the
+        // difference of the wave's inclusive prefix sums at its last lane
+        // and before its first (run starts from a ballot of key changes)
+        const double pe = wave_prefix_sum(e), pd = wave_prefix_sum(d);
+        const int kp = __shfl_up(key, 1);
+        const unsigned long long starts = __ballot(lane == 0 || kp != key);
+        const int first = 63 - __clzll(starts & ((2ull << lane) - 1ull));
+        const double pe0 = __shfl(pe, first > 0 ? first - 1 : 0), pd0 = __shfl(pd, first > 0 ? first - 1 : 0);
+        const bool last = lane == 63 || (((starts >> lane) >> 1) & 1ull);
+        if (key > 0 && last) {
+          he[key - 1] += first > 0 ? pe - pe0 : pe;
+          hd[key - 1] += first > 0 ? pd - pd0 : pd;
         }
       }
     }
@@ -2007,37 +2014,33 @@ __global__ void __launch_bounds__(256) k_shell_fold_rows(double* __restrict__ pa
   }
 }
 // out[0..nshell) = E, out[nshell..2 nshell) = D, out[2 nshell] = TKE,
-// out[2 nshell + 1] = epsilon: the rows b rstride (b < nb) summed in row
-// order, the totals over all nh shells in shell order.  One work-group.
-__global__ void __launch_bounds__(256)
+// out[2 nshell + 1] = epsilon (pinned host memory): the rows b rstride (b <
+// nb) summed in row order, the totals over all nh shells by one wave each
+// (lane l takes l, l + 64, .. in order, then the lanes by pairs).  One
+// work-group.
+constexpr int kShellFold = 1024;
+__global__ void __launch_bounds__(kShellFold)
     k_shell_fold(const double* __restrict__ part, int nb, int rstride, int nh, int nshell, double* __restrict__ out) {
   extern __shared__ double fold[];  // [2][nh]
-  for (int s = threadIdx.x; s < nh; s += blockDim.x) {
-    double e = 0.0, d = 0.0;
-    for (int b = 0; b < nb; b++) {
-      e += part[(size_t)b * rstride * 2 * nh + s];
-      d += part[(size_t)b * rstride * 2 * nh + nh + s];
-    }
-    fold[s] = e;
-    fold[nh + s] = d;
-    if (s < nshell) {
-      out[s] = e;
-      out[nshell + s] = d;
-    }
+  for (int s = threadIdx.x; s < 2 * nh; s += kShellFold) {
+    double v = 0.0;
+#pragma unroll 8
+    for (int b = 0; b < nb; b++) v += part[(size_t)b * rstride * 2 * nh + s];
+    fold[s] = v;
+    const int k = s < nh ? s : s - nh;
+    if (k < nshell) out[s < nh ? k : nshell + k] = v;
   }
-  for (int s = nh + threadIdx.x; s < nshell; s += blockDim.x) {
+  for (int s = nh + threadIdx.x; s < nshell; s += kShellFold) {
     out[s] = 0.0;
     out[nshell + s] = 0.0;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0, e = 0.0;
-    for (int s = 0; s < nh; s++) {
-      t += fold[s];
-      e += fold[nh + s];
-    }
-    out[2 * nshell] = t;
-    out[2 * nshell + 1] = e;
+  if (threadIdx.x < 128) {
+    const double* f = threadIdx.x < 64 ? fold : fold + nh;
+    double t = 0.0;
+    for (int s = threadIdx.x & 63; s < nh; s += 64) t += f[s];
+    t = wave_sum(t);
+    if ((threadIdx.x & 63) == 0) out[2 * nshell + (threadIdx.x >> 6)] = t;
   }
 }
 
@@ -2541,7 +2544,7 @@ struct Launch {
     const unsigned grid = tiles_grid(full, N * (N / X::B));
     hipLaunchKernelGGL(kern, dim3(grid, 2), dim3(X::NT), 0, c.stream, (const CR*)c.xi, (R*)nullptr, c.geo,
                        (const CR*)c.tw, (double*)c.xs);
-    hipLaunchKernelGGL(k_moments_fold, dim3(2), dim3(256), 0, c.stream, (const double*)c.xs, (int)grid, out);
+    hipLaunchKernelGGL(k_moments_fold, dim3(2), dim3(kMomFold), 0, c.stream, (const double*)c.xs, (int)grid, out);
   }
   static void x_r2c(const Ctx& c, int nv) {
     using X = XPass<R, N>;
@@ -2689,7 +2692,7 @@ struct LaunchP {
                        sizeof(double) * kShellWaves * 2 * nh, c.stream, (const CR*)c.un, c.geo, viscos, nh, part);
     static_assert(kShellBlocks % kShellFoldRows == 0, "whole fold chunks");
     hipLaunchKernelGGL(k_shell_fold_rows, dim3(kShellBlocks / kShellFoldRows), dim3(256), 0, c.stream, part, nh);
-    hipLaunchKernelGGL(k_shell_fold, dim3(1), dim3(256), sizeof(double) * 2 * nh, c.stream, part,
+    hipLaunchKernelGGL(k_shell_fold, dim3(1), dim3(kShellFold), sizeof(double) * 2 * nh, c.stream, part,
                        kShellBlocks / kShellFoldRows, kShellFoldRows, nh, nshell, out);
   }
   static void field(const Ctx& c, unsigned long long seed, double kpeak, const int* d_colz0) {
