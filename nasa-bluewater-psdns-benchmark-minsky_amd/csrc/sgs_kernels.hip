@@ -263,11 +263,12 @@ __global__ void __launch_bounds__(256)
 // [feature][point] rows, wave w forms the row block o = 16 w .. of it.
 // What bounds it: the chain of a tile (gather, about 560 matrix instructions
 // of 32 cycles, 52 tanhf, five exchanges through LDS) with one wave per SIMD:
-// 52 us at B = 16384 (a tile per CU), 35 us at B = 1000; its arithmetic (6 x
-// 12164 flops per point) would take 8 us on the matrix cores.
+// 45 us at B = 16384 (a tile per CU), 28 us at B = 1000 (52 and 35 with the
+// weights copied to LDS by loops of a load and its store); its arithmetic (6
+// x 12164 flops per point) would take 8 us on the matrix cores.
 // 20 steps of B = 16384 took 37.4 ms as a gather, five layer kernels, four
 // backward ones, five weight-gradient kernels with their folds and Adam (one
-// thread per output: 286 us for a 64 x 64 weight gradient); 1.18 ms this way.
+// thread per output: 286 us for a 64 x 64 weight gradient); 1.04 ms this way.
 // ---------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -287,16 +288,37 @@ __global__ void __launch_bounds__(256)
   __shared__ float Ts[24 * kTS], taus[6 * kTS];
   __shared__ double red[4];
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
-  for (int i = tid; i < kConv * kW0ld; i += 256) {
-    const int o = i / kW0ld, k = i % kW0ld;
-    W0s[i] = k < kIn0 ? theta[oW0 + o * kIn0 + k] : 0.f;
+  {
+    // all loads first: a loop of a load and its store waits for each
+    f32x4 w2[4], w3[4];
+    float w0[9], w1[6];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      w2[i] = *(const f32x4*)(theta + oW2 + 4 * (tid + 256 * i));
+      w3[i] = *(const f32x4*)(theta + oW3 + 4 * (tid + 256 * i));
+    }
+#pragma unroll
+    for (int i = 0; i < 9; i++) w0[i] = theta[oW0 + min(tid + 256 * i, kConv * kIn0 - 1)];
+#pragma unroll
+    for (int i = 0; i < 6; i++) w1[i] = theta[oW1 + min(tid + 256 * i, kHid * kIn1 - 1)];
+    const float w4 = theta[oW4 + tid];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int e = 4 * (tid + 256 * i), o = e / kHid * kLd + e % kHid;
+      *(f32x4*)(W2s + o) = w2[i];
+      *(f32x4*)(W3s + o) = w3[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+      const int e = tid + 256 * i;
+      if (e < kConv * kIn0) W0s[e / kIn0 * kW0ld + e % kIn0] = w0[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+      if (tid + 256 * i < kHid * kIn1) W1s[tid + 256 * i] = w1[i];
+    W4s[tid / kHid * kLd + tid % kHid] = w4;
+    if (tid < 2 * kConv) W0s[tid / 2 * kW0ld + kIn0 + tid % 2] = 0.f;
   }
-  for (int i = tid; i < kHid * kIn1; i += 256) W1s[i] = theta[oW1 + i];
-  for (int i = tid; i < kHid * kHid; i += 256) {
-    W2s[i / kHid * kLd + i % kHid] = theta[oW2 + i];
-    W3s[i / kHid * kLd + i % kHid] = theta[oW3 + i];
-  }
-  W4s[tid / kHid * kLd + tid % kHid] = theta[oW4 + tid];
   if (tid < kHid) {
     b1s[tid] = theta[ob1 + tid];
     b2s[tid] = theta[ob2 + tid];
