@@ -667,12 +667,13 @@ __global__ void __launch_bounds__(256)
 //
 // What bounds it, BF16 at 128^3: issue. Per 16 points 1,440 cycles of matrix
 // instructions and about 3,000 of VALU (52 tanh per lane, two quarter-rate
-// instructions each), 236 us on end where nothing overlaps; 270 us per call
-// (253 us with the halo left in place, 209 without the tanh, 218 without the
-// convolution's products), against 178 us for the convolution with its 16
-// channels stored and 189 us for the dense layers that read them back. 64^3:
-// 47 us (75), with FP32 layers 89 us (179). Two tiles per wave, sharing each
-// weight read, came to 262-360 us for 2 to 4 waves per SIMD.
+// instructions each), 236 us on end where nothing overlaps; 240 us per call,
+// against 178 us for the convolution with its 16 channels stored and 189 us
+// for the dense layers that read them back.  64^3: 37.5 us (75), with FP32
+// layers 87 us (179).  Before the weights were loaded with all loads in flight
+// and their LDS addresses formed once per tile: 270 us (209 without the tanh,
+// 218 without the convolution's products) and 46 us; two tiles per wave,
+// sharing each weight read, came to 262-360 us for 2 to 4 waves per SIMD.
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
@@ -706,24 +707,19 @@ __device__ __forceinline__ constexpr int in_k(int g, int j) {
 // operand-A blocks in LDS, 64 lanes x 16 bytes each: W1 ob 0..3, W2 (s, ob)
 // 4..11, W3 (s, ob) 12..19, W4 s 20..21 (rows 0..3 of 16)
 constexpr int kOpBlocks = 22;
+// (no branch, so that the loads of several blocks can be in flight)
 __device__ __forceinline__ bf16x8 a_block(const float* __restrict__ theta, int blk, int lane) {
   const int r = lane & 15, g = lane >> 4;
+  const bool first = blk < 4, out = blk >= 20;
+  const int s = out ? blk - 20 : ((blk - 4) % 8) / 4;
+  const int o = first ? 16 * blk + r : (out ? min(r, kBasis - 1) : 16 * ((blk - 4) % 4) + r);
+  const int row = first ? oW1 + o * kIn1 : (out ? oW4 : blk < 12 ? oW2 : oW3) + o * kHid;
+  float w[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) w[j] = theta[row + (first ? max(in_k(g, j), 0) : slot_k(s, g, j))];
   bf16x8 v;
-  if (blk < 4) {
-    const int o = 16 * blk + r;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int k = in_k(g, j);
-      v[j] = (__bf16)(k >= 0 ? theta[oW1 + o * kIn1 + k] : 0.f);
-    }
-    return v;
-  }
-  const int base = blk < 12 ? oW2 : (blk < 20 ? oW3 : oW4);
-  const int s = blk < 20 ? ((blk - 4) % 8) / 4 : blk - 20;
-  const int o = blk < 20 ? 16 * ((blk - 4) % 4) + r : r;
-  const int rows = blk < 20 ? kHid : kBasis;
-#pragma unroll
-  for (int j = 0; j < 8; j++) v[j] = (__bf16)(o < rows ? theta[base + o * kHid + slot_k(s, g, j)] : 0.f);
+  for (int j = 0; j < 8; j++) v[j] = (__bf16)((first && in_k(g, j) < 0) || (out && r >= kBasis) ? 0.f : w[j]);
   return v;
 }
 // accumulator initial values: bias of outputs 16 ob + 4 g + jj (layer 0..2
@@ -766,21 +762,44 @@ struct DenseWeights;
 template <>
 struct DenseWeights<true> {
   bf16x8 op[kOpBlocks][64];
-  __device__ __forceinline__ void fill(const float* __restrict__ theta, int tid, int nt) {
-    for (int i = tid; i < kOpBlocks * 64; i += nt) op[i / 64][i % 64] = a_block(theta, i / 64, i % 64);
+  template <int NT>
+  __device__ __forceinline__ void fill(const float* __restrict__ theta, int tid) {
+    constexpr int n = (kOpBlocks * 64 + NT - 1) / NT;
+    bf16x8 v[n];
+#pragma unroll
+    for (int i = 0; i < n; i++) v[i] = a_block(theta, min((tid + NT * i) / 64, kOpBlocks - 1), tid % 64);
+#pragma unroll
+    for (int i = 0; i < n; i++)
+      if (tid + NT * i < kOpBlocks * 64) op[(tid + NT * i) / 64][tid % 64] = v[i];
   }
 };
 template <>
 struct DenseWeights<false> {
   __attribute__((aligned(16))) float W2[kHid * kLd], W3[kHid * kLd], W4[kBasis * kLd];
   float W1[kHid * kIn1];
-  __device__ __forceinline__ void fill(const float* __restrict__ theta, int tid, int nt) {
-    for (int i = tid; i < kHid * kIn1; i += nt) W1[i] = theta[oW1 + i];
-    for (int i = tid; i < kHid * kHid; i += nt) {
-      W2[i / kHid * kLd + i % kHid] = theta[oW2 + i];
-      W3[i / kHid * kLd + i % kHid] = theta[oW3 + i];
+  template <int NT>
+  __device__ __forceinline__ void fill(const float* __restrict__ theta, int tid) {
+    constexpr int n1 = (kHid * kIn1 + NT - 1) / NT, n2 = kHid * kHid / 4 / NT;
+    static_assert(kHid * kHid % (4 * NT) == 0 && kBasis * kHid <= NT, "whole rounds");
+    f32x4 w2[n2], w3[n2];
+    float w1[n1];
+#pragma unroll
+    for (int i = 0; i < n2; i++) {
+      w2[i] = *(const f32x4*)(theta + oW2 + 4 * (tid + NT * i));
+      w3[i] = *(const f32x4*)(theta + oW3 + 4 * (tid + NT * i));
     }
-    for (int i = tid; i < kBasis * kHid; i += nt) W4[i / kHid * kLd + i % kHid] = theta[oW4 + i];
+#pragma unroll
+    for (int i = 0; i < n1; i++) w1[i] = theta[oW1 + min(tid + NT * i, kHid * kIn1 - 1)];
+    if (tid < kBasis * kHid) W4[tid / kHid * kLd + tid % kHid] = theta[oW4 + tid];
+#pragma unroll
+    for (int i = 0; i < n2; i++) {
+      const int e = 4 * (tid + NT * i), o = e / kHid * kLd + e % kHid;
+      *(f32x4*)(W2 + o) = w2[i];
+      *(f32x4*)(W3 + o) = w3[i];
+    }
+#pragma unroll
+    for (int i = 0; i < n1; i++)
+      if (tid + NT * i < kHid * kIn1) W1[tid + NT * i] = w1[i];
   }
 };
 
@@ -793,11 +812,6 @@ __global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_
   __shared__ float halo[kLam * kHch];
   constexpr int NT = 64 * kCWaves;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
-  wt.fill(theta, tid, NT);
-  for (int i = tid; i < 13 * 4; i += NT) {
-    const int b = i / 4;
-    bias[b][i % 4] = b < 12 ? bias_block(theta, b / 4, b % 4, i % 4) : bias_block(theta, 3, 0, i % 4);
-  }
   // this lane's convolution weights (row c) and bias (rows 4 g + jj)
   constexpr int kSteps = 34;
   float wc[kSteps];
@@ -814,7 +828,6 @@ __global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_
   int off4[kSteps - kTaps];
 #pragma unroll
   for (int q = 0; q < kSteps - kTaps; q++) off4[q] = 4 * kHch + tap_off(min(4 * q + g, kTaps - 1));
-  auto bc = [&](int b) { return bias[b][opaque_lane(lane) >> 4]; };
 
   const size_t P = (size_t)n * n * n;
   const int m = n - 1, nbx = n / kBx, nbz = n / kBz, nblk = nbx * nbz * (n / kBy);
@@ -843,6 +856,11 @@ __global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_
   const int x8 = blockIdx.x % 8, per = gridDim.x / 8, q8 = nblk / 8, end = (x8 + 1) * q8;
   int blk = x8 * q8 + blockIdx.x / 8;
   if (blk < end) load_halo(blk);
+  wt.template fill<NT>(theta, tid);
+  if (tid < 13 * 4) {
+    const int b = tid / 4;
+    bias[b][tid % 4] = b < 12 ? bias_block(theta, b / 4, b % 4, tid % 4) : bias_block(theta, 3, 0, tid % 4);
+  }
   for (; blk < end; blk += per) {
     const int x0 = blk % nbx * kBx, z0 = blk / nbx % nbz * kBz, y0 = blk / (nbx * nbz) * kBy;
     __syncthreads();  // the last block's halo is read
@@ -883,10 +901,14 @@ __global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_
       });
       f32x4 h0;
       f32x4 gc;  // rows 0..3 (lanes 0..15): the basis coefficients of point c
+      // weights and biases are read per tile, through a lane index the compiler
+      // cannot hoist their reads with
+      const int ln = opaque_lane(lane), lg4 = ln >> 4;
+      auto bc = [&](int b) { return bias[b][lg4]; };
       if constexpr (BF16) {
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) h0[jj] = tanh_fast(ca[jj] + cb[jj]);
-        auto wa = [&](int b) { return wt.op[b][opaque_lane(lane)]; };
+        auto wa = [&](int b) { return wt.op[b][ln]; };
         const bf16x8 x = {(__bf16)h0[0], (__bf16)h0[1], (__bf16)h0[2], (__bf16)h0[3],
                           (__bf16)lg,    (__bf16)l4,    (__bf16)0.f,   (__bf16)0.f};
         f32x4 d[4];
