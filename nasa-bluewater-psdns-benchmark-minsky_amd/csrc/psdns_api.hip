@@ -350,9 +350,9 @@ int scalar_gradients(psdns_ctx* c) {
     kd.xi = (char*)c->d_xi + (3 + 3 * (size_t)i) * xb;
     int bad = 0, rc;
     if ((rc = mark_sc(c, 6 * i))) return rc;
-    bad |= psdns::launch_y_grad(k, (char*)c->d_usc + i * vb, c->d_xs);
+    bad |= psdns::launch_y_grad(k, (char*)c->d_usc + i * vb, c->d_xs, 1, 1);
     if ((rc = mark_sc(c, 6 * i + 1))) return rc;
-    bad |= psdns::launch_pass(kd, Pass::ZInv, 3, 2);
+    bad |= psdns::launch_pass(kd, Pass::ZInv, 1, 2);
     if ((rc = mark_sc(c, 6 * i + 2))) return rc;
     if (bad) return fail(PSDNS_EINVAL, "unsupported grid n = %d", c->n);
   }

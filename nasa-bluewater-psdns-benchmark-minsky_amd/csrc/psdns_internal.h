@@ -91,7 +91,7 @@ enum class Pass {
   YInvKx,     // kxtran: zero y Nyquist + y c2c +i, u -> yw
   YInvPlain,  // y c2c +i, u -> yw
   YInvGrad,   // du/dx, dw/dz of un on the mask + y c2c +i, un -> yw (two variables)
-  ZInv,       // gather yw + z c2c +i -> xi (args: number of variables; source 0 W1, 1 y-blocked yw in u, 2 a scalar's two gradient slots in W1 -> three xi slots)
+  ZInv,       // gather yw + z c2c +i -> xi (args: number of variables; source 0 W1, 1 y-blocked yw in u, 2 the gradients of that many variables, two slots each in W1 -> three xi slots each)
   XC2R,       // gather xi + x c2r -> physical (arg: number of variables)
   XR2C,       // physical -> x r2c / n (arg: number of variables)
   XFused,     // c2r u,v,w (xi) -> products (+velmax, arg) -> r2c / n of 5 (X)
@@ -143,13 +143,16 @@ void launch_scale(const Ctx& c, void* p, size_t cnt, double s);
 // phase-shift tables of both stages from gsh(3,2): FP64 s64 and state
 // precision sr (layouts of Ctx::sx/sy/sz and Ctx::sr)
 void launch_shifts(const Ctx& c, double2* s64, void* sr, const double gsh[6]);
-// passive scalars, stage c.kstep: the shifted gradient i k (sx sy sz phi)
-// of one scalar, y-transformed (y c2c +i), into yw slots 0..2; the scalar
+// nv variables phi (cylinder slots), y-transformed for their gradient: on the
+// mask, shifted by stage c.kstep's factors (sh 1: in the state precision, 2:
+// in FP64, 0: not), Y[phi] and Y[i ky phi] into yw slots 2 v and 2 v + 1
+// (Pass::ZInv with source 2 makes the three derivatives of them).  Passive
+// scalars, stage c.kstep: the scalar
 // update from tr, the advection term z-transformed and normalised (one W1
 // slot): its y forward transform and the update in one pass (stage 1 | 2
 // RK2, 11 .. 14 the RK4 substeps with the accumulator u1; dif: nxh + 2 n
 // doubles of scratch for the scalar's integrating factors)
-int launch_y_grad(const Ctx& c, const void* phi, void* yw);
+int launch_y_grad(const Ctx& c, const void* phi, void* yw, int nv, int sh);
 int launch_sc_update(const Ctx& c, int stage, void* u, void* un, const void* tr, double dt2, double rpr,
                      double* dif, void* u1 = nullptr);
 // velocity-gradient moments: the x c2r of xi slots 0 and 1 and the FP64 sums

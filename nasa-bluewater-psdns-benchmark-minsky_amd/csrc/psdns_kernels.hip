@@ -330,39 +330,46 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
 }
 
 // ---------------------------------------------------------------------------
-// Shifted gradient of a passive scalar, y-transformed (phase1.f:44-64,
-// itransform.f:190-203): phi_s = sx sy sz phi on the mask (0 elsewhere);
-// yw slot 0 = Y[phi_s], slot 1 = Y[i ky phi_s] with Y the y c2c +i of a
-// column.  The x and z derivatives multiply slot 0 by i kx and i kz, which
+// Shifted gradient of nv variables, y-transformed (a passive scalar:
+// phase1.f:44-64, itransform.f:190-203; the velocity for the SGS features):
+// phi_s = sx sy sz phi on the mask (0 elsewhere); per variable yw slot 0 =
+// Y[phi_s], slot 1 = Y[i ky phi_s] with Y the y c2c +i of a column.  The x and z derivatives multiply slot 0 by i kx and i kz, which
 // are constant along a column: the inverse z pass applies them (k_z_inv
 // DER), so two slots carry the three derivatives.  Tiles of B columns, natural
 // mapping in and out, yw in the cylinder layout; persistent over tiles as
 // k_y_inv (the next tile's loads in flight during the current transforms;
 // off-mask entries are not read, so they enter as zeros).
-// Shift factors in the state precision: sr = sx[nxh] | sy[n] | sz[n].
+// SH 1: shift factors in the state precision, sr = sx[nxh] | sy[n] | sz[n];
+// SH 2: FP64 factors and product (s64), rounded once; SH 0: no shift.
 // ---------------------------------------------------------------------------
-template <typename R, int N>
+struct Shift64 {
+  const double2 *x, *y, *z;
+};
+template <typename R, int N, int SH>
 __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
-    k_y_grad(const C<R>* __restrict__ phi, C<R>* __restrict__ yw, Geo g, const C<R>* __restrict__ sr,
-             const C<R>* __restrict__ tw, const int* __restrict__ colx, const int* __restrict__ colz) {
+    k_y_grad(const C<R>* __restrict__ phi, C<R>* __restrict__ yw, Geo g, const C<R>* __restrict__ sr, Shift64 s64,
+             const C<R>* __restrict__ tw, int nv, const int* __restrict__ colx, const int* __restrict__ colz) {
   constexpr int T = Team<N>::T, E = Team<N>::E, B = YInv<R>::B;
   using F = TeamFft<R, N, E, B, +1>;
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
-  __shared__ C<R> ssy[N];
+  __shared__ std::conditional_t<SH == 2, double2, C<R>> ssy[SH ? N : 1];
   F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
-  for (int k = threadIdx.x; k < N; k += F::NT) ssy[k] = sr[g.nxh + k];
+  if constexpr (SH == 1)
+    for (int k = threadIdx.x; k < N; k += F::NT) ssy[k] = sr[g.nxh + k];
+  if constexpr (SH == 2)
+    for (int k = threadIdx.x; k < N; k += F::NT) ssy[k] = s64.y[k];
   const int tid = threadIdx.x;
   const Slot<R> io = F::natural(lds, tid);
   const int li0 = F::natural_line(tid);
-  const int nab = (g.na + B - 1) / B;  // tiles
+  const int nab = (g.na + B - 1) / B;  // tiles per variable
   const size_t tot = (size_t)g.na * N;
   __syncthreads();
   // the line of a lane (wave-uniform when a line spans whole waves)
   auto line_of = [&]() { return T >= 64 ? __builtin_amdgcn_readfirstlane(opaque(li0)) : opaque(li0); };
   auto load = [&](Regs<R, E>& b, int t, bool valid) {
-    const int a0 = t * B;
-    const BufView<R> src(phi + (size_t)a0 * N, valid ? kOob : 0u);
+    const int var = t / nab, a0 = (t % nab) * B;
+    const BufView<R> src(phi + var * tot + (size_t)a0 * N, valid ? kOob : 0u);
     // lines past the last column re-read the last column (never stored)
     const int li = line_of(), q = opaque(io.q);
     const int lc = li < g.na - a0 ? li : g.na - 1 - a0;
@@ -375,22 +382,27 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
     }
   };
   auto finish = [&](Regs<R, E>& b, int t) {
-    const int a0 = t * B;
+    const int var = t / nab, a0 = (t % nab) * B;
     const int li = line_of(), q = opaque(io.q);
     const int a = a0 + li < g.na ? a0 + li : g.na - 1;
-    const int x = colx[a], z = colz[a], kz = kwave(z, N);
-    const C<R> sxz = cmul(sr[x], sr[g.nxh + N + z]);
+    const int x = colx[a], z = colz[a];
+    C<R> sxz;
+    double2 dxz;
+    if constexpr (SH == 1) sxz = cmul(sr[x], sr[g.nxh + N + z]);
+    if constexpr (SH == 2) dxz = zmul(s64.x[x], s64.z[z]);
     C<R> b2[E];
 #pragma unroll
     for (int j = 0; j < E; j++) {
       const int y = q + T * j;
       const R ky = (R)kwave(y, N);
-      b.v[j] = cmul(b.v[j], cmul(ssy[y], sxz));
+      if constexpr (SH == 1) b.v[j] = cmul(b.v[j], cmul(ssy[y], sxz));
+      if constexpr (SH == 2) b.v[j] = to_c<R>(zmul(make_double2(b.v[j].x, b.v[j].y), zmul(dxz, ssy[y])));
       b2[j] = {-ky * b.v[j].y, ky * b.v[j].x};
     }
     F::template run<false, false, false, false>(b.v, lds, io, io, stw);
     F::template run<false, false, false, false>(b2, lds, io, io, stw);
-    const BufView<R> d0(yw + (size_t)a0 * N, kOob), d1(yw + tot + (size_t)a0 * N, kOob);
+    C<R>* out = yw + 2 * var * tot + (size_t)a0 * N;
+    const BufView<R> d0(out, kOob), d1(out + tot, kOob);
     const bool act = a0 + li < g.na;
 #pragma unroll
     for (int m = 0; m < E; m++) {
@@ -400,7 +412,7 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
     }
   };
   Regs<R, E> ba, bb;
-  tile_loop(nab, ba, bb, load, finish);
+  tile_loop(nv * nab, ba, bb, load, finish);
 }
 
 // ---------------------------------------------------------------------------
@@ -412,8 +424,8 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
 // (which always holds the z Nyquist) read as zero (kxcomm1_clean.f:238-240);
 // z c2c +i; the last stage leaves the lines in the natural mapping for
 // contiguous stores along z.
-// DER (a passive scalar's gradient, from k_y_grad's two slots Y[phi],
-// Y[i ky phi]): three outputs per kx and y block, taken in turn (v fastest,
+// DER (the gradient of nv variables, from k_y_grad's two slots Y[phi],
+// Y[i ky phi] of each): three outputs per variable, kx and y block, taken in turn (v fastest,
 // so that the second read of Y[phi] meets the cache): xi slot 0 = i kx
 // Z[Y[phi]] (kx constant per tile, applied after the transform), slot 1 =
 // Z[Y[i ky phi]], slot 2 = Z[i kz Y[phi]] (applied before it).
@@ -434,14 +446,15 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
   const Slot<R> out = F::natural(lds, tid);
   const int lt0 = F::transposed_line(tid), ln0 = F::natural_line(tid);
   __syncthreads();
-  // tile t = (var * max_al_x + kx) * NYB + y block; DER: t = (kx * NYB +
-  // y block) * 3 + output, the input slot 1 for output 1, else 0
+  // tile t = (var * max_al_x + kx) * NYB + y block; DER: t = ((variable *
+  // max_al_x + kx) * NYB + y block) * 3 + output, var = 3 variable + output,
+  // from input slot 2 variable + 1 for output 1, else 2 variable
   auto tile = [&](int t, int& var, int& kx, int& y0) {
     if constexpr (DER) {
-      var = t % 3;
-      const int r = t / 3;
-      kx = r / NYB;
+      const int r = t / 3, vk = r / NYB;
       y0 = (r % NYB) * B;
+      var = 3 * (vk / g.max_al_x) + t % 3;
+      kx = vk % g.max_al_x;
     } else {
       const int vk = t / NYB;
       y0 = (t % NYB) * B;
@@ -452,7 +465,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
   auto load = [&](Regs<R, E>& b, int t, bool valid) {
     int var, kx, y0;
     tile(t, var, kx, y0);
-    if constexpr (DER) var = var == 1 ? 1 : 0;
+    if constexpr (DER) var = 2 * (var / 3) + (var % 3 == 1 ? 1 : 0);
     const int c = cutz[kx];
     // YB: the kx's columns in y block y0 / B, one contiguous run; else
     // 64-byte runs along y of the kx's columns
@@ -471,7 +484,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
     int var, kx, y0;
     tile(t, var, kx, y0);
     if constexpr (DER) {
-      if (var == 2) {
+      if (t % 3 == 2) {
         // i kz at line point zz (the FFT index of kz), transposed mapping
         const int qi = opaque(in.q);
 #pragma unroll
@@ -483,7 +496,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
     }
     F::template run<false, false, true, false>(b.v, lds, in, out, stw);
     if constexpr (DER) {
-      if (var == 0) {
+      if (t % 3 == 0) {
         const R rkx = (R)kx;
 #pragma unroll
         for (int m = 0; m < E; m++) b.v[m] = {-rkx * b.v[m].y, rkx * b.v[m].x};
@@ -496,7 +509,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
       dst.store(((unsigned)l * g.max_al_x * N + q + T * m) * (unsigned)sizeof(C<R>), b.v[m]);
   };
   Regs<R, E> ba, bb;
-  tile_loop((DER ? 3 : nv) * g.max_al_x * NYB, ba, bb, load, finish);
+  tile_loop((DER ? 3 * nv : nv) * g.max_al_x * NYB, ba, bb, load, finish);
 }
 
 // ---------------------------------------------------------------------------
@@ -2506,16 +2519,16 @@ struct Launch {
   }
   // yw from the W1 allocation (from_u = 0, column-major cylinder) or
   // y-blocked from the u slots 0..2 (the fused stage-1 update's output)
-  // from_u: 0 yw in W1, 1 y-blocked yw in u, 2 a scalar's gradient (two
-  // slots in W1 -> three xi slots; nv is not used)
+  // from_u: 0 yw in W1, 1 y-blocked yw in u, 2 the gradient of nv variables
+  // (two slots each in W1 -> three xi slots each)
   static void z_inv(const Ctx& c, int nv, int from_u) {
     constexpr int B = RunLines<R>::B, T = Team<N>::T;
-    const int nt = (from_u == 2 ? 3 : nv) * c.geo.max_al_x * (N / B);
+    const int nt = (from_u == 2 ? 3 * nv : nv) * c.geo.max_al_x * (N / B);
     if (from_u == 2) {
       const auto kern = k_z_inv<R, N, false, true>;
       static const unsigned grid = persistent_grid((const void*)kern, B * T);
       hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(B * T), 0, c.stream, (const CR*)c.w1, (CR*)c.xi, c.geo,
-                         (const CR*)c.tw, 3, c.geo.cutz, c.geo.col0);
+                         (const CR*)c.tw, nv, c.geo.cutz, c.geo.col0);
     } else if (from_u) {
       const auto kern = k_z_inv<R, N, true>;
       static const unsigned grid = persistent_grid((const void*)kern, B * T);
@@ -2832,28 +2845,36 @@ void launch_shifts(const Ctx& c, double2* s64, void* sr, const double gsh[6]) {
     hipLaunchKernelGGL((k_shifts<float>), dim3((tot + 255) / 256), dim3(256), 0, c.stream, s64, (C<float>*)sr,
                        c.geo.n, c.geo.nxh, g);
 }
-template <typename R, int N>
-static void y_grad_n(const Ctx& c, const void* phi, void* yw) {
+template <typename R, int N, int SH>
+static void y_grad_n(const Ctx& c, const void* phi, void* yw, int nv) {
   constexpr int NT = YInv<R>::B * Team<N>::T;
-  const auto kern = k_y_grad<R, N>;
+  const auto kern = k_y_grad<R, N, SH>;
   static const unsigned grid = persistent_grid((const void*)kern, NT);
-  hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, (c.geo.na + YInv<R>::B - 1) / YInv<R>::B)), dim3(NT), 0, c.stream, (const C<R>*)phi, (C<R>*)yw, c.geo,
-                     (const C<R>*)c.sr[c.kstep], (const C<R>*)c.tw, c.geo.colx, c.geo.colz);
+  const int k = c.kstep;
+  hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nv * ((c.geo.na + YInv<R>::B - 1) / YInv<R>::B))), dim3(NT), 0,
+                     c.stream, (const C<R>*)phi, (C<R>*)yw, c.geo, (const C<R>*)c.sr[k],
+                     Shift64{c.sx[k], c.sy[k], c.sz[k]}, (const C<R>*)c.tw, nv, c.geo.colx, c.geo.colz);
+}
+template <typename R, int N>
+static void y_grad_s(const Ctx& c, const void* phi, void* yw, int nv, int sh) {
+  if (sh == 0) y_grad_n<R, N, 0>(c, phi, yw, nv);
+  else if (sh == 1) y_grad_n<R, N, 1>(c, phi, yw, nv);
+  else y_grad_n<R, N, 2>(c, phi, yw, nv);
 }
 template <typename R>
-static int y_grad_r(const Ctx& c, const void* phi, void* yw) {
+static int y_grad_r(const Ctx& c, const void* phi, void* yw, int nv, int sh) {
   switch (c.geo.n) {
-    case 32: y_grad_n<R, 32>(c, phi, yw); return 0;
-    case 64: y_grad_n<R, 64>(c, phi, yw); return 0;
-    case 128: y_grad_n<R, 128>(c, phi, yw); return 0;
-    case 256: y_grad_n<R, 256>(c, phi, yw); return 0;
-    case 512: y_grad_n<R, 512>(c, phi, yw); return 0;
-    case 1024: y_grad_n<R, 1024>(c, phi, yw); return 0;
+    case 32: y_grad_s<R, 32>(c, phi, yw, nv, sh); return 0;
+    case 64: y_grad_s<R, 64>(c, phi, yw, nv, sh); return 0;
+    case 128: y_grad_s<R, 128>(c, phi, yw, nv, sh); return 0;
+    case 256: y_grad_s<R, 256>(c, phi, yw, nv, sh); return 0;
+    case 512: y_grad_s<R, 512>(c, phi, yw, nv, sh); return 0;
+    case 1024: y_grad_s<R, 1024>(c, phi, yw, nv, sh); return 0;
   }
   return -1;
 }
-int launch_y_grad(const Ctx& c, const void* phi, void* yw) {
-  return c.prec == 8 ? y_grad_r<double>(c, phi, yw) : y_grad_r<float>(c, phi, yw);
+int launch_y_grad(const Ctx& c, const void* phi, void* yw, int nv, int sh) {
+  return c.prec == 8 ? y_grad_r<double>(c, phi, yw, nv, sh) : y_grad_r<float>(c, phi, yw, nv, sh);
 }
 template <typename R, int N>
 static void sc_update_n(const Ctx& c, int stage, void* u, void* un, const void* tr, double dt2, double* dif,

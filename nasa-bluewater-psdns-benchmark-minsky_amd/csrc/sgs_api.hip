@@ -55,7 +55,7 @@ struct psdns_sgs {
   hipStream_t stream = nullptr;
   // spectral gradient work (sized for FP64 on first use: na from the context)
   int na = 0, max_al_x = 0;
-  void *cyl = nullptr, *yw = nullptr, *xi = nullptr, *A = nullptr;
+  void *yw = nullptr, *xi = nullptr, *A = nullptr;
   int A_prec = 0;     // precision of the gradient in A (that of the last features context)
   // current field: features, target, prediction
   float *lam = nullptr, *T = nullptr, *tau = nullptr, *tau_hat = nullptr;
@@ -170,7 +170,7 @@ int psdns_sgs_create(int n, int max_snapshots, psdns_sgs** out) {
 int psdns_sgs_destroy(psdns_sgs* m) {
   if (!m) return PSDNS_OK;
   if (m->stream) (void)hipStreamSynchronize(m->stream);
-  void* ptrs[] = {m->cyl, m->yw, m->xi, m->A, m->lam, m->T, m->tau, m->tau_hat, m->lam_s, m->T_s,
+  void* ptrs[] = {m->yw, m->xi, m->A, m->lam, m->T, m->tau, m->tau_hat, m->lam_s, m->T_s,
                   m->tau_s, m->theta, m->m, m->v, m->grad, m->work, m->lpart, m->losses};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -227,24 +227,24 @@ int features(psdns_sgs* m, psdns_ctx* c, int stage) {
   // reads the cylinder u slots 0..2; its own buffers for the transforms
   if ((rc = psdns::ctx_access(c, false, false, &k, &n))) return rc;
   if (n != m->n) return set_error(PSDNS_EINVAL, "grid %d: the closure is for n = %d", n, m->n);
-  if (!m->cyl) {
-    const size_t cb = sizeof(double) * 2 * 9 * (size_t)k.geo.na * n;
+  if (!m->yw) {
+    const size_t cb = sizeof(double) * 2 * 6 * (size_t)k.geo.na * n;
     const size_t xb = sizeof(double) * 2 * 9 * (size_t)n * k.geo.max_al_x * n;
-    if ((rc = dalloc((char**)&m->cyl, cb, "the gradient cylinder")) ||
-        (rc = dalloc((char**)&m->yw, cb, "the gradient cylinder")) ||
+    if ((rc = dalloc((char**)&m->yw, cb, "the gradient cylinder")) ||
         (rc = dalloc((char**)&m->xi, xb, "the gradient z pencils")) ||
         (rc = dalloc((char**)&m->A, sizeof(double) * 9 * m->P, "the gradient")))
       return rc;
     m->na = k.geo.na;
     m->max_al_x = k.geo.max_al_x;
   }
+  // the y pass forms Y[u_i] and Y[i ky u_i] on the mask, phase shifted (in FP64)
+  // for a stage; the z pass the three derivatives of each component
   Ctx g = k;
-  g.u = m->cyl;
   g.w1 = m->yw;
   g.xi = m->xi;
   g.ux = m->A;
-  S::launch_grad_spec(k, k.u, m->cyl, stage);
-  if (psdns::launch_pass(g, psdns::Pass::YInvPlain, 9, 0) || psdns::launch_pass(g, psdns::Pass::ZInv, 9, 0) ||
+  g.kstep = stage > 0 ? stage - 1 : 0;
+  if (psdns::launch_y_grad(g, k.u, m->yw, 3, stage > 0 ? 2 : 0) || psdns::launch_pass(g, psdns::Pass::ZInv, 3, 2) ||
       psdns::launch_pass(g, psdns::Pass::XC2R, 9, 0))
     return set_error(PSDNS_EINVAL, "unsupported grid n = %d", n);
   const double delta = 2.0 * M_PI / n;

@@ -41,9 +41,6 @@ constexpr int train_rows(int B) { return (B + 63) / 64 < 256 ? (B + 63) / 64 : 2
 
 // r = 2, 4, .., 32 (the ratios of two grids between 32 and 1024); -1 for another
 int launch_box_filter(hipStream_t st, int prec, const void* u, int n, int r, void* ubar, float* tau);
-// i k_j u_i on the mask; with a stage (1|2) the state is first phase shifted
-// by that stage's factors (phase1 on the fly), stage 0 takes u as it is
-void launch_grad_spec(const Ctx& c, const void* u, void* d, int stage);
 void launch_invariants(hipStream_t st, int prec, const void* A, size_t P, double delta2, float* lam, float* T);
 // the closure's stress of the features: the convolution in FP32, the dense
 // layers in FP32 or on bf16 operands

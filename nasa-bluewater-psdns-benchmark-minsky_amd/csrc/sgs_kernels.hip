@@ -149,39 +149,6 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------------------
-// Gradient in spectral space: d[3 i + j] = i k_j u_i on the mask (0 off it)
-// for the cylinder entries of u slots 0..2 (taken as they are: shifted by
-// phase1 in the LES stage, unshifted for training data).
-// ---------------------------------------------------------------------------
-template <typename R>
-__global__ void __launch_bounds__(256)
-    k_grad_spec(const cpx<R>* __restrict__ u, cpx<R>* __restrict__ d, Geo g, const double2* __restrict__ sx,
-                const double2* __restrict__ sy, const double2* __restrict__ sz) {
-  const size_t tot = (size_t)g.na * g.n;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < tot; i += (size_t)gridDim.x * blockDim.x) {
-    const int a = (int)(i / g.n), y = (int)(i % g.n);
-    const int kx = g.colx[a], z = g.colz[a];
-    const int ky = y <= g.n / 2 ? y : y - g.n, kz = z <= g.n / 2 ? z : z - g.n;
-    const bool m = 9 * (kx * kx + ky * ky + kz * kz) <= 2 * g.n * g.n && y != g.n / 2 && z != g.n / 2;
-    const R k[3] = {(R)kx, (R)ky, (R)kz};
-    // phase1 of the stage (phshift.f:71-135): u sx(kx) sz(kz) sy(ky), in FP64
-    double2 sh = make_double2(1.0, 0.0);
-    if (sx) {
-      const double2 a2 = sx[kx], b2 = sz[z], c2 = sy[y];
-      const double2 ab = make_double2(a2.x * b2.x - a2.y * b2.y, a2.x * b2.y + a2.y * b2.x);
-      sh = make_double2(ab.x * c2.x - ab.y * c2.y, ab.x * c2.y + ab.y * c2.x);
-    }
-#pragma unroll
-    for (int v = 0; v < 3; v++) {
-      cpx<R> c = m ? u[v * tot + i] : cpx<R>{0, 0};
-      if (sx) c = {(R)((double)c.x * sh.x - (double)c.y * sh.y), (R)((double)c.x * sh.y + (double)c.y * sh.x)};
-#pragma unroll
-      for (int j = 0; j < 3; j++) d[(3 * v + j) * tot + i] = {-k[j] * c.y, k[j] * c.x};
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Invariants and tensor basis of A (9 physical fields, A[3 i + j] = du_i/dx_j)
 // per point, in FP64: S = sym(A) - tr(A)/3 I, W = skew(A), q = |S|^2 + |W|^2;
 // lambda = (tr S^2, tr W^2) / q, (tr S^3, tr W^2 S) / q^1.5, tr W^2 S^2 / q^2;
@@ -1072,19 +1039,6 @@ static int box_filter_r(hipStream_t st, const R* u, int n, int r, R* ubar, float
 int launch_box_filter(hipStream_t st, int prec, const void* u, int n, int r, void* ubar, float* tau) {
   return prec == 8 ? box_filter_r(st, (const double*)u, n, r, (double*)ubar, tau)
                    : box_filter_r(st, (const float*)u, n, r, (float*)ubar, tau);
-}
-
-void launch_grad_spec(const Ctx& c, const void* u, void* d, int stage) {
-  const size_t tot = (size_t)c.geo.na * c.geo.n;
-  const double2* sx = stage ? c.sx[stage - 1] : nullptr;
-  const double2* sy = stage ? c.sy[stage - 1] : nullptr;
-  const double2* sz = stage ? c.sz[stage - 1] : nullptr;
-  if (c.prec == 8)
-    hipLaunchKernelGGL(k_grad_spec<double>, dim3(blocks(tot)), dim3(256), 0, c.stream, (const cpx<double>*)u,
-                       (cpx<double>*)d, c.geo, sx, sy, sz);
-  else
-    hipLaunchKernelGGL(k_grad_spec<float>, dim3(blocks(tot)), dim3(256), 0, c.stream, (const cpx<float>*)u,
-                       (cpx<float>*)d, c.geo, sx, sy, sz);
 }
 
 void launch_invariants(hipStream_t st, int prec, const void* A, size_t P, double delta2, float* lam, float* T) {

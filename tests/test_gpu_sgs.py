@@ -105,6 +105,37 @@ def test_features_match_oracle(O, P, shifted):
     assert np.abs(A[0, 0] + A[1, 1] + A[2, 2]).max() < 1e-10 * np.abs(A).max()
 
 
+@pytest.mark.parametrize("kstep", [0, 1, 2])
+@pytest.mark.parametrize("n,prec", [(32, 4), (64, 8), (128, 4)])
+def test_features_stage_sizes(O, P, n, prec, kstep):
+    """features of the state as it is and on each stage's shifted grid, for the
+    gradient kernels' FP32 and FP64 forms and several sizes of line; bounds
+    of the test above (FP32: the transform's rounding)"""
+    print("[gpu case] sgs features sizes", n, prec, kstep, flush=True)
+    g = O.Grid(n)
+    u = g.field(seed=53)
+    gsh = np.array([0.21, 0.63, 0.37, 0.71, 0.12, 0.45])
+    s, m = P.Solver(n, prec), P.Closure(n)
+    try:
+        s.put_state(u)
+        s.set_shifts(gsh)
+        m.features(s, kstep)
+        A_got = m.field(P.SGS_GRADIENT)
+        lam_got, T_got = m.field(P.SGS_LAMBDA), m.field(P.SGS_BASIS)
+    finally:
+        m.close()
+        s.close()
+    uy = u.copy()
+    if kstep:
+        g.set_shifts(gsh)
+        g.phshift_inplace(uy, 3, kstep)
+    A = SG.gradient(g, uy)
+    lam, T = SG.invariants(A, 2 * np.pi / n)
+    assert rel(A_got, A) < 1e-6
+    assert rel(lam_got, lam) < 1e-5
+    assert rel(T_got, T) < 1e-5
+
+
 def _features(O, n, seed):
     g = O.Grid(n)
     A = SG.gradient(g, g.field(seed=seed))
