@@ -7,6 +7,7 @@ import pathlib
 import re
 import subprocess
 
+import numpy as np
 import pytest
 
 from conftest import REPO, load_package
@@ -93,3 +94,23 @@ def test_fortran_interface_and_driver_built(P):
     syms = subprocess.run(["nm", str(P.DRIVER_PATH)], capture_output=True, text=True).stdout
     for f in ("psdns_stage_nonlinear", "psdns_stage_update", "psdns_set_shifts", "psdns_ek_force"):
         assert f in syms
+
+
+@pytest.mark.parametrize("n", [32, 64])
+def test_step_factors_follow_the_viscosity(P, n):
+    """the kept exponents: a viscosity set later, in place too, changes the
+    factors, to the same bits as forming them anew"""
+    s = P.Solver.__new__(P.Solver)
+    s.h, s.n, s._exponents = None, n, (None, None, None)
+    k = np.arange(n)
+    kw = np.where(k > n // 2, k - n, k).astype(np.float64)
+    kx = np.arange(n // 2, dtype=np.float64)
+    inplace = np.array(0.03)
+    for viscos in (0.01, 0.02, inplace, inplace, 0.0):
+        s.viscos = viscos
+        for dt in (1e-3, 7e-3):
+            xf, yf, zf = s.step_factors(dt)
+            assert np.array_equal(xf, np.exp(-viscos * kx * kx * dt))
+            assert np.array_equal(yf, np.exp(-viscos * kw * kw * dt)) and np.array_equal(zf, yf)
+            assert not np.shares_memory(yf, zf)
+        inplace *= 1.5
