@@ -519,9 +519,10 @@ struct TeamFft {
   // being hoisted out of the loop and held in registers across it; without
   // it, calls on the same slots share their address arithmetic.
   // stw is the LDS twiddle table (fill_twiddles).
+  // tid: the thread's index among the NT threads that share `lds`.
   template <bool TO_LDS = false, bool FRESH = true, bool IN_T = true, bool OUT_T = true>
-  static __device__ __forceinline__ void run(cpx<R>* v, R* lds, Slot<R> in, Slot<R> out, const cpx<R>* stw) {
-    int tid = (int)threadIdx.x;
+  static __device__ __forceinline__ void run(cpx<R>* v, R* lds, Slot<R> in, Slot<R> out, const cpx<R>* stw,
+                                             int tid = (int)threadIdx.x) {
     if constexpr (FRESH) {
       int oi = (int)(in.re - lds), qi = in.q, oo = (int)(out.re - lds), qo = out.q;
       asm volatile("" : "+v"(oi), "+v"(qi), "+v"(oo), "+v"(qo), "+v"(tid));

@@ -604,6 +604,26 @@ struct XPass {
           0, 0, 0);
     }
   }
+  // the same for the variables 0..2 of a tile into S[3][M][B], by the first
+  // `waves` (whole) wavefronts of the work-group, 16 rows at a time
+  static __device__ __forceinline__ void stage_load3(C<R>* S, const C<R>* __restrict__ xi, int y, int z0,
+                                                     const Geo& g, int waves) {
+    constexpr int kRowBytes = B * (int)sizeof(C<R>), kSlices = M / 16;
+    static_assert(kRowBytes == 64 && M % 16 == 0, "staging shape");
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = (int)threadIdx.x % 64;
+    if (wave >= waves) return;
+    for (int s = wave; s < 3 * kSlices; s += waves) {
+      const int row = s % kSlices * 16 + lane / 4;
+      const BufView<R> src(xi + xiidx(s / kSlices, y, 0, z0, g), kOob);
+      const unsigned off = row < g.max_al_x
+                               ? (unsigned)row * (unsigned)(N * sizeof(C<R>)) + (unsigned)(lane % 4) * 16u
+                               : kOob;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src.r,
+          (__attribute__((address_space(3))) void*)(reinterpret_cast<char*>(S) + s * 16 * kRowBytes), 16, off, 0, 0,
+          0);
+    }
+  }
   // Makes the staged variable visible to the whole work-group.  The copies
   // into S complete asynchronously and count in vmcnt; the waits the
   // compiler inserts order them only before the same wave's own reads of S,
@@ -620,8 +640,8 @@ struct XPass {
   // refilled; c2r_staged_fft then transforms: v[j] = (a, b) at x = q + T j of
   // this thread's pair in the natural mapping.  kx Nyquist is zero, Im A[0]
   // and Im B[0] are ignored.
-  static __device__ __forceinline__ void c2r_staged_pre(C<R>* v, const C<R>* S) {
-    const int tid = opaque(threadIdx.x);  // per tile, not hoisted out of the tile loop
+  static __device__ __forceinline__ void c2r_staged_pre(C<R>* v, const C<R>* S, int tid0 = threadIdx.x) {
+    const int tid = opaque(tid0);  // per tile, not hoisted out of the tile loop
     const int l = FI::transposed_line(tid), q = (int)((unsigned)tid / PB);
     struct alignas(2 * sizeof(C<R>) < 16 ? 2 * sizeof(C<R>) : 16) Two {
       C<R> a, b;
@@ -643,26 +663,27 @@ struct XPass {
     }
     lds_barrier();
   }
-  static __device__ __forceinline__ void c2r_staged_fft(C<R>* v, R* lds, const C<R>* stw) {
-    const int tid = threadIdx.x;
-    FI::template run<false, true, true, false>(v, lds, FI::transposed(lds, tid), FI::natural(lds, tid), stw);
+  static __device__ __forceinline__ void c2r_staged_fft(C<R>* v, R* lds, const C<R>* stw, int tid = threadIdx.x) {
+    FI::template run<false, true, true, false>(v, lds, FI::transposed(lds, tid), FI::natural(lds, tid), stw, tid);
   }
 
   // r2c of the physical values v of this thread's pair, scaled by `scale` / 2:
   // the last stage leaves Z in LDS; 2 A[k] and 2 B[k] for kx < max_al_x (kx
   // Nyquist dropped).  Without SCALE the values stored are the transform x 2
-  // unnormalized, n times the transform / n (x 2n, exact in binary).
+  // unnormalized, n times the transform / n (x 2n, exact in binary).  vofs: a
+  // further offset in elements that may differ between lanes.
   template <bool SCALE>
   static __device__ __forceinline__ void r2c(C<R>* v, C<R>* __restrict__ xs, int var, int y, int z0,
-                                             const Geo& g, R* lds, const C<R>* stw, R scale) {
-    const int tid = XFRESH ? opaque(threadIdx.x) : (int)threadIdx.x;
+                                             const Geo& g, R* lds, const C<R>* stw, R scale,
+                                             int tid0 = threadIdx.x, unsigned vofs = 0) {
+    const int tid = XFRESH ? opaque(tid0) : tid0;
     const Slot<R> s = FF::natural(lds, tid);
-    FF::template run<true, XFRESH, false, false>(v, lds, s, s, stw);
+    FF::template run<true, XFRESH, false, false>(v, lds, s, s, stw, tid);
     FF::template sync<false>();
     // no branch per point: kx >= max_al_x lanes store nothing (out of range)
     const BufView<R> dst(xs + xidx<K>(var, y, z0, 0, g), kOob);
     const int q = s.q;
-    const unsigned lofs = (unsigned)(2 * FF::natural_line(tid)) * K;
+    const unsigned lofs = vofs + (unsigned)(2 * FF::natural_line(tid)) * K;
     const R half = (R)0.5 * scale;
     // with T a multiple of K, point k = q + T j lies in kx block q / K + j T / K
     // at q % K: one lane offset, and j's part in the scalar offset
@@ -694,6 +715,26 @@ struct XPass {
         dst.store(k < g.max_al_x ? o : kOob, oa);
         dst.store(k < g.max_al_x ? o + kNext : kOob, ob);
       }
+    }
+  }
+
+  // the subgrid stress of product slot sl at this thread's points: x = q + T j
+  // of the lines z0 + 2 line and the next
+  static __device__ __forceinline__ void add_tau(C<R>* q, const float* __restrict__ tau, int sl, int y, int z0,
+                                                 int tid) {
+    constexpr size_t P3 = (size_t)N * N * N;
+    const int line = FI::natural_line(tid), qq = (int)((unsigned)tid % T);
+    const float* base = tau + ((size_t)y * N + z0 + 2 * line) * N + qq;
+    constexpr int ca[5] = {0, 1, 5, 4, 2}, cb[5] = {3, -1, 3, -1, -1};  // + tau[ca] - tau[cb]
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+      const float* p = base + T * j;
+      float ta = p[ca[sl] * P3], tb = p[ca[sl] * P3 + N];
+      if (cb[sl] >= 0) {
+        ta -= p[cb[sl] * P3];
+        tb -= p[cb[sl] * P3 + N];
+      }
+      q[j] = {q[j].x + (R)ta, q[j].y + (R)tb};
     }
   }
 };
@@ -971,29 +1012,61 @@ __attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : XPass<R, N>::kWaves, S
 #pragma unroll
         for (int j = 0; j < E; j++)
           q[j] = {product(sl, pu[j].x, pv[j].x, pw[j].x), product(sl, pu[j].y, pv[j].y, pw[j].y)};
-        if constexpr (TAU) {
-          // this thread's points: x = q + T j of the lines z0 + 2 line and the next
-          constexpr size_t P3 = (size_t)N * N * N;
-          const int line = X::FI::natural_line(threadIdx.x), qq = (int)(threadIdx.x % X::T);
-          const float* base = tau + ((size_t)y * N + z0 + 2 * line) * N + qq;
-          constexpr int ca[5] = {0, 1, 5, 4, 2}, cb[5] = {3, -1, 3, -1, -1};  // + tau[ca] - tau[cb]
-#pragma unroll
-          for (int j = 0; j < E; j++) {
-            const float* p = base + X::T * j;
-            float ta = p[ca[sl] * P3], tb = p[ca[sl] * P3 + N];
-            if (cb[sl] >= 0) {
-              ta -= p[cb[sl] * P3];
-              tb -= p[cb[sl] * P3 + N];
-            }
-            q[j] = {q[j].x + (R)ta, q[j].y + (R)tb};
-          }
-        }
+        if constexpr (TAU) X::add_tau(q, tau, sl, y, z0, threadIdx.x);
         X::template r2c<false>(q, xs, sl, y, z0, g, lds, stw, (R)1);
       }
       if (!more) break;
       t = tn;
     }
   }
+  if (want_velmax) velmax_commit((double)vm * (double)N, velmax);
+}
+
+// The fused x pass of small grids (without scalars), where a tile's chain of three inverse and
+// five forward transforms is what a launch takes: a work-group of five groups
+// of NT threads per tile.  The rows of u, v and w are copied to LDS together;
+// groups 0..2 transform one each (3 and 4 repeat u and v, so that all meet the
+// same barriers) and leave the physical values in LDS; then group s forms
+// product s and transforms it forward: two transforms deep instead of eight,
+// the same operations on each value.
+// SPLIT_NOTE
+template <typename R, int N, bool TAU>
+__global__ void __launch_bounds__((5 * XPass<R, N>::NT))
+    k_x_fused_split(const C<R>* __restrict__ xi, C<R>* __restrict__ xs, Geo g, const C<R>* __restrict__ tw,
+                    unsigned long long* __restrict__ velmax, int want_velmax, const float* __restrict__ tau) {
+  using X = XPass<R, N>;
+  constexpr int E = X::E, B = X::B, M = X::M, NT = X::NT, G = 5;
+  __shared__ R lds[G * X::kLdsReals];
+  __shared__ C<R> stw[X::kTw];
+  __shared__ __attribute__((aligned(16))) C<R> S[3 * M * B];
+  __shared__ C<R> P[3][E * NT];
+  constexpr int NZB = N / B;
+  const int t = tile_walk(N * NZB).t;  // one tile per work-group
+  const int y = t / NZB, z0 = (t % NZB) * B;
+  X::stage_load3(S, xi, y, z0, g, G * NT / 64);
+  X::FI::template fill_twiddles<1>(stw, tw, threadIdx.x, G * NT);
+  const int gr = (int)threadIdx.x / NT, tid = (int)threadIdx.x % NT;
+  R* own = lds + gr * X::kLdsReals;
+  X::stage_publish();
+  C<R> v[E];
+  X::c2r_staged_pre(v, S + gr % 3 * (M * B), tid);
+  X::c2r_staged_fft(v, own, stw, tid);
+  if (gr < 3) {
+#pragma unroll
+    for (int j = 0; j < E; j++) P[gr][j * NT + tid] = v[j];
+  }
+  __syncthreads();
+  R vm = 0;
+#pragma unroll
+  for (int j = 0; j < E; j++) {
+    const C<R> a = P[0][j * NT + tid], b = P[1][j * NT + tid], c = P[2][j * NT + tid];
+    vm = fmax(vm, fabs(a.x) + fabs(b.x) + fabs(c.x));
+    vm = fmax(vm, fabs(a.y) + fabs(b.y) + fabs(c.y));
+    v[j] = {product(gr, a.x, b.x, c.x), product(gr, a.y, b.y, c.y)};
+  }
+  if constexpr (TAU) X::add_tau(v, tau, gr, y, z0, tid);
+  X::template r2c<false>(v, xs, 0, y, z0, g, own, stw, (R)1, tid,
+                         (unsigned)gr * (unsigned)(xidx<X::K>(1, y, z0, 0, g) - xidx<X::K>(0, y, z0, 0, g)));
   if (want_velmax) velmax_commit((double)vm * (double)N, velmax);
 }
 
@@ -1044,21 +1117,22 @@ struct ZFwd {
   using F = TeamFft<R, N, E, B, -1, LineShift<E, B>::IN>;
   using Buf = Regs<R, E>;
 
-  // gathered loads of variable var of tile t = y * nkb + kx block
+  // gathered loads of variable var of tile t = y * nkb + kx block (vofs, also
+  // in store: a further offset in elements that may differ between lanes)
   static __device__ __forceinline__ void load(Buf& b, const C<R>* __restrict__ xs, const Geo& g, int nkb, int t,
-                                              int var, bool valid, int lt0, int q0) {
+                                              int var, bool valid, int lt0, int q0, unsigned vofs = 0) {
     const int y = t / nkb, kx0 = (t % nkb) * B;
     const BufView<R> src(xs + xidx<B>(var, y, 0, kx0, g), valid ? kOob : 0u);
     const int l = opaque(lt0), q = opaque(q0);
     const bool act = kx0 + l < g.max_al_x;
 #pragma unroll
     for (int j = 0; j < E; j++)
-      b.v[j] = src.load(act ? ((unsigned)(q + T * j) * B + l) * (unsigned)sizeof(C<R>) : kOob);
+      b.v[j] = src.load(act ? ((unsigned)(q + T * j) * B + l + vofs) * (unsigned)sizeof(C<R>) : kOob);
   }
   // stores of the cylinder z of a transformed variable (natural mapping)
   static __device__ __forceinline__ void store(const Buf& b, C<R>* __restrict__ w1, const Geo& g,
                                                const int* __restrict__ cutz, int nkb, int t, int var, int ln0,
-                                               int q0) {
+                                               int q0, unsigned vofs = 0) {
     const int y = t / nkb, kx0 = (t % nkb) * B;
     const int l = T >= 64 ? __builtin_amdgcn_readfirstlane(opaque(ln0)) : opaque(ln0), q = opaque(q0);
     const int kx = kx0 + l;
@@ -1069,7 +1143,7 @@ struct ZFwd {
     for (int m = 0; m < E; m++) {
       const int z = q + T * m;
       const bool keep = act && (z < N / 2 - c || z > N / 2 + c);
-      dst.store(keep ? ((unsigned)l * N * N + z) * (unsigned)sizeof(C<R>) : kOob, b.v[m]);
+      dst.store(keep ? ((unsigned)l * N * N + z + vofs) * (unsigned)sizeof(C<R>) : kOob, b.v[m]);
     }
   }
 };
@@ -1138,6 +1212,52 @@ __global__ void __launch_bounds__((ZFwd<R, N>::NT)) __attribute__((amdgpu_waves_
     if (!more) break;
     t = tn;
   }
+}
+
+// k_z_fwd of small grids, as k_x_fused_split: group s of a tile's work-group
+// transforms slot s, P5 goes to groups 0 and 2 through LDS.
+template <typename R, int N>
+__global__ void __launch_bounds__((5 * ZFwd<R, N>::NT))
+    k_z_fwd_split(const C<R>* __restrict__ xs, C<R>* __restrict__ w1, Geo g, const C<R>* __restrict__ tw,
+                  const int* __restrict__ cutz) {
+  using Z = ZFwd<R, N>;
+  using F = typename Z::F;
+  constexpr int T = Z::T, E = Z::E, B = Z::B, NT = Z::NT, G = 5;
+  __shared__ R lds[G * F::kLdsReals];
+  __shared__ C<R> stw[F::kTwEntries];
+  __shared__ C<R> P5[E * NT];
+  const int nkb = (g.max_al_x + B - 1) / B;
+  const TileWalk w = tile_walk(N * nkb);
+  const int t = w.t;  // one tile per work-group
+  if (t >= w.end) return;
+  const int gr = (int)threadIdx.x / NT, tid = (int)threadIdx.x % NT;
+  R* own = lds + gr * F::kLdsReals;
+  const Slot<R> in = F::transposed(own, tid), out = F::natural(own, tid);
+  typename Z::Buf b;
+  Z::load(b, xs, g, nkb, t, 0, true, F::transposed_line(tid), in.q,
+          (unsigned)gr * (unsigned)(xidx<B>(1, 0, 0, 0, g) - xidx<B>(0, 0, 0, 0, g)));
+  F::template fill_twiddles<1>(stw, tw, threadIdx.x, G * NT);
+  __syncthreads();
+  F::template run<false, ZFRESH, true, false>(b.v, own, in, out, stw, tid);
+  if (gr == 4) {
+#pragma unroll
+    for (int j = 0; j < E; j++) P5[j * NT + tid] = b.v[j];
+  }
+  __syncthreads();
+  if (gr == 4) return;
+  if (gr == 0 || gr == 2) {
+    // i (kx P1 + kz P5), i (kx P5 + kz P3)
+    const R kxr = (R)((t % nkb) * B + F::natural_line(tid));
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+      const R kz = (R)kwave(out.q + T * j, N);
+      const C<R> p5 = P5[j * NT + tid], x = gr == 0 ? b.v[j] : p5, z = gr == 0 ? p5 : b.v[j];
+      const C<R> s = {kxr * x.x + kz * z.x, kxr * x.y + kz * z.y};
+      b.v[j] = {-s.y, s.x};
+    }
+  }
+  Z::store(b, w1, g, cutz, nkb, t, 0, F::natural_line(tid), out.q,
+           (unsigned)gr * (unsigned)(w1idx(1, 0, 0, 0, g) - w1idx(0, 0, 0, 0, g)));
 }
 
 // xktran (MODE 1 of the z pass): nv slots, x 1/(ny nz) (xktran.f:121,150-157);
@@ -2488,6 +2608,13 @@ static inline unsigned tiles_grid(unsigned full, int ntiles) {
   return need < full ? need : full;
 }
 
+// Up to this n the fused x and forward z passes split a tile's transforms over
+// five groups of threads.  A pass there has at most four wavefronts per SIMD
+// and takes as long as one tile's chain of transforms; from 128^3 on the
+// groups' LDS and their repeated inverse transforms cost more (x 20.0 -> 26.8
+// us at 128^3 FP32, 35 -> 55 FP64).
+constexpr int kSplitN = 64;
+
 template <typename R, int N>
 struct Launch {
   using CR = C<R>;
@@ -2568,16 +2695,20 @@ struct Launch {
   static void x_fused(const Ctx& c, int want_velmax) {
     using X = XPass<R, N>;
     constexpr int nt = N * (N / X::B);
-    if (c.tau) {
-      const auto kern = k_x_fused<R, N, true>;
-      static const unsigned grid = persistent_grid((const void*)kern, X::NT);
-      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(X::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
-                         (const CR*)c.tw, c.velmax_bits, want_velmax, c.tau, 0, ScGrad{});
-    } else if (c.nsc > 0) {
+    if (!c.tau && c.nsc > 0) {
       const auto kern = k_x_fused<R, N, false, true>;
       static const unsigned grid = persistent_grid((const void*)kern, X::NT);
       hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(X::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
                          (const CR*)c.tw, c.velmax_bits, want_velmax, (const float*)nullptr, c.nsc, c.scg);
+    } else if constexpr (N <= kSplitN) {
+      const auto kern = c.tau ? k_x_fused_split<R, N, true> : k_x_fused_split<R, N, false>;
+      hipLaunchKernelGGL(kern, dim3(nt), dim3(5 * X::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
+                         (const CR*)c.tw, c.velmax_bits, want_velmax, c.tau);
+    } else if (c.tau) {
+      const auto kern = k_x_fused<R, N, true>;
+      static const unsigned grid = persistent_grid((const void*)kern, X::NT);
+      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(X::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
+                         (const CR*)c.tw, c.velmax_bits, want_velmax, c.tau, 0, ScGrad{});
     } else {
       const auto kern = k_x_fused<R, N, false>;
       static const unsigned grid = persistent_grid((const void*)kern, X::NT);
@@ -2589,10 +2720,15 @@ struct Launch {
     constexpr int NT = ZFwd<R, N>::NT, B = ZFwd<R, N>::B;
     const int nt = N * ((c.geo.max_al_x + B - 1) / B) * (mode == 0 ? 1 : nv);
     if (mode == 0) {
-      const auto kern = k_z_fwd<R, N>;
-      static const unsigned grid = persistent_grid((const void*)kern, NT);
-      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(NT), 0, c.stream, (const CR*)c.xs, (CR*)c.w1, c.geo,
-                         (const CR*)c.tw, c.geo.cutz);
+      if constexpr (N <= kSplitN) {
+        hipLaunchKernelGGL((k_z_fwd_split<R, N>), dim3((nt + 7) / 8 * 8), dim3(5 * NT), 0, c.stream,
+                           (const CR*)c.xs, (CR*)c.w1, c.geo, (const CR*)c.tw, c.geo.cutz);
+      } else {
+        const auto kern = k_z_fwd<R, N>;
+        static const unsigned grid = persistent_grid((const void*)kern, NT);
+        hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(NT), 0, c.stream, (const CR*)c.xs, (CR*)c.w1, c.geo,
+                           (const CR*)c.tw, c.geo.cutz);
+      }
     } else {
       const auto kern = k_z_fwd_norm<R, N>;
       static const unsigned grid = persistent_grid((const void*)kern, NT);

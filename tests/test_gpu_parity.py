@@ -212,6 +212,31 @@ def test_fused_stages(O, P, ctxs, n, prec, peek):
     assert rel(s.get_field(P.FIELD_U, 3), uy2[:3], m) < TOL[prec]
 
 
+@pytest.mark.parametrize("n,prec", [(32, 8), (32, 4), (64, 8), (64, 4), (128, 4)])
+def test_stage_with_and_without_scalars(O, P, ctxs, n, prec):
+    """The x pass of small grids splits a tile over five groups of threads
+    (up to 64^3), with scalars it does not: the same velocity from both, the
+    same operations per value up to the contraction of their sums."""
+    banner("stage with and without scalars", n, prec)
+    g = O.Grid(n)
+    gsh = np.array([0.35, 0.15, 0.65, 0.85, 0.65, 0.15])
+    u0 = g.field(seed=78)
+    m = g.mask()[None]
+    out = []
+    for nc in (0, 1):
+        s = ctxs(n, prec) if nc == 0 else P.Solver(n, prec, viscos=0.01, nc=1, pr=[1.0])
+        s.set_shifts(gsh)
+        s.put_state(u0 if nc == 0 else np.concatenate([u0, g.field(seed=79)[:1]]))
+        vm = s.stage_nonlinear(1)
+        xf, yf, zf = s.step_factors(0.02)
+        s.stage_update(1, 0.02, xf, yf, zf)
+        vm2 = s.stage_nonlinear(2)
+        s.stage_update(2, 0.02, xf, yf, zf)
+        out.append((vm, vm2, s.get_state()[:3]))
+    assert out[0][:2] == pytest.approx(out[1][:2], rel=1e-12 if prec == 8 else 2e-6)
+    assert rel(out[0][2], out[1][2], m) < TOL[prec]
+
+
 @pytest.mark.parametrize("n,prec", [(64, 8), (64, 4)])
 def test_deferred_update_keeps_its_shifts(O, P, ctxs, n, prec):
     """stage_update(1) runs in the next call; new shifts set in between apply
