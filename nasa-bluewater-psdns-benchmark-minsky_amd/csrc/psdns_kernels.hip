@@ -531,7 +531,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
 // the forward transform writes its lines into the kx blocks of X (natural
 // mapping: the tile's B lines together fill B x 64 contiguous bytes per block).
 // ---------------------------------------------------------------------------
-template <typename R, int N>
+template <typename R, int N, bool WIDE = false>
 struct XPass {
   static constexpr int M = N / 2;
   static constexpr int K = RunLines<R>::B;  // one 64-byte run of z (or of kx in X)
@@ -541,7 +541,12 @@ struct XPass {
   // points per thread, up to 16 in FP32 and 8 in FP64 (16 of its accumulators
   // do not fit the registers)
   static constexpr int EMAX = sizeof(R) == 4 ? 16 : 8;
-  static constexpr int E = Team<N, EMAX>::E, T = N / E;
+  // WIDE: 8 points (one exchange through LDS less) also at 256 FP32.  The
+  // velocity pass there 132 -> 117 us, with two scalars 352 -> 273 us, two
+  // variables' moments 99 -> 73 us; but the lanes of a line then span 128 bytes
+  // instead of 256 of a physical row: c2r of nine variables 225 -> 245 us, the
+  // pass that reads the subgrid stress 195 -> 236 us, so those keep 4 points.
+  static constexpr int E = WIDE && sizeof(R) == 4 && N == 256 ? 8 : Team<N, EMAX>::E, T = N / E;
   static constexpr int NT = PB * T;
   // waves per SIMD the registers of the fused pass are sized for
   static constexpr int kWaves = E >= 16 ? 2 : 4;
@@ -759,10 +764,10 @@ __device__ __forceinline__ double wave_sum(double v) {
 // stored fields with one FP64 atomic per wave and power, and 212 us for one
 // that formed the derivatives (now on load in the y pass).
 template <typename R, int N, bool MOM>
-__global__ void __launch_bounds__((XPass<R, N>::NT))
+__global__ void __launch_bounds__((XPass<R, N, MOM>::NT))
     k_x_c2r(const C<R>* __restrict__ xi, R* __restrict__ ux, Geo g, const C<R>* __restrict__ tw,
             double* __restrict__ part) {
-  using X = XPass<R, N>;
+  using X = XPass<R, N, MOM>;
   constexpr int E = X::E, B = X::B, NZB = N / B;
   __shared__ R lds[X::kLdsReals];
   __shared__ C<R> stw[X::kTw];
@@ -941,13 +946,14 @@ __device__ __forceinline__ R product(int s, R u, R v, R w) {
 #define PSDNS_XSC_WAVES 2
 #endif
 template <typename R, int N, bool TAU, bool SC = false>
-__global__ void __launch_bounds__((XPass<R, N>::NT))
-__attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : XPass<R, N>::kWaves, SC ? PSDNS_XSC_WAVES : XPass<R, N>::kWaves)))
+__global__ void __launch_bounds__((XPass<R, N, !TAU>::NT))
+__attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : XPass<R, N, !TAU>::kWaves,
+                                    SC ? PSDNS_XSC_WAVES : XPass<R, N, !TAU>::kWaves)))
     k_x_fused(const C<R>* __restrict__ xi, C<R>* __restrict__ xs, Geo g, const C<R>* __restrict__ tw,
               unsigned long long* __restrict__ velmax, int want_velmax, const float* __restrict__ tau, int nsc,
               ScGrad scg) {
   static_assert(!(TAU && SC), "an LES stage carries no scalars");
-  using X = XPass<R, N>;
+  using X = XPass<R, N, !TAU>;
   constexpr int E = X::E, B = X::B;
   __shared__ R lds[X::kLdsReals];
   __shared__ C<R> stw[X::kTw];
@@ -2678,7 +2684,7 @@ struct Launch {
   // the moments of the variables 0 and 1 of xi into out[16]; X holds the
   // partial rows
   static void x_moments(const Ctx& c, double* out) {
-    using X = XPass<R, N>;
+    using X = XPass<R, N, true>;
     const auto kern = k_x_c2r<R, N, true>;
     static const unsigned full = persistent_grid((const void*)kern, X::NT, 4);
     const unsigned grid = tiles_grid(full, N * (N / X::B));
@@ -2694,11 +2700,12 @@ struct Launch {
   }
   static void x_fused(const Ctx& c, int want_velmax) {
     using X = XPass<R, N>;
+    using XW = XPass<R, N, true>;
     constexpr int nt = N * (N / X::B);
     if (!c.tau && c.nsc > 0) {
       const auto kern = k_x_fused<R, N, false, true>;
-      static const unsigned grid = persistent_grid((const void*)kern, X::NT);
-      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(X::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
+      static const unsigned grid = persistent_grid((const void*)kern, XW::NT);
+      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(XW::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
                          (const CR*)c.tw, c.velmax_bits, want_velmax, (const float*)nullptr, c.nsc, c.scg);
     } else if constexpr (N <= kSplitN) {
       const auto kern = c.tau ? k_x_fused_split<R, N, true> : k_x_fused_split<R, N, false>;
@@ -2711,8 +2718,8 @@ struct Launch {
                          (const CR*)c.tw, c.velmax_bits, want_velmax, c.tau, 0, ScGrad{});
     } else {
       const auto kern = k_x_fused<R, N, false>;
-      static const unsigned grid = persistent_grid((const void*)kern, X::NT);
-      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(X::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
+      static const unsigned grid = persistent_grid((const void*)kern, XW::NT);
+      hipLaunchKernelGGL(kern, dim3(tiles_grid(grid, nt)), dim3(XW::NT), 0, c.stream, (const CR*)c.xi, (CR*)c.xs, c.geo,
                          (const CR*)c.tw, c.velmax_bits, want_velmax, (const float*)nullptr, 0, ScGrad{});
     }
   }
