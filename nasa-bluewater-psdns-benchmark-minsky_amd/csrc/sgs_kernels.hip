@@ -630,7 +630,8 @@ __global__ void __launch_bounds__(256)
 // operand B, so the activations stay in the lane's registers from layer to
 // layer (no LDS tile, no cross-lane exchange).  The weights are in LDS, for
 // BF16 as operand-A blocks in that order; the biases are the accumulators'
-// initial values.  The sums, biases and tanh are FP32.
+// initial values.  The sums and biases are FP32; the activations are tanhf, but
+// for those of the dense layers with BF16 (tanh_fast).
 //
 // What bounds it, BF16 at 128^3: issue. Per 16 points 1,440 cycles of matrix
 // instructions and about 3,000 of VALU (52 tanh per lane, two quarter-rate
@@ -703,10 +704,12 @@ __device__ __forceinline__ f32x4 bias_block(const float* __restrict__ theta, int
 }
 
 // tanh(x) = 1 - 2 / (exp(2 x) + 1) with the hardware exponential and
-// reciprocal, v_exp_f32 and v_rcp_f32 (relative error ~1e-6, far below the
-// bf16 operands' 4e-3; saturates to +-1 for large |x|).  A division here
-// (even __fdividef) compiles to the full IEEE sequence, several times the
-// cost of the rest of the activation.
+// reciprocal, v_exp_f32 and v_rcp_f32; saturates to +-1 for large |x|.  Its error
+// is absolute, about 1e-7 whatever the size of the result: next to the 4e-3
+// relative rounding of the bf16 operands of which a dense layer sums 64, of
+// order one, but not for the activations of the convolution, which may be small
+// throughout.  A division here (even __fdividef) compiles to the full IEEE
+// sequence, several times the cost of the rest of the activation.
 __device__ __forceinline__ float tanh_fast(float x) {
   // exp(2 x) as v_exp_f32 (2^v) of 2 x log2(e)
   return fmaf(-2.f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(2.8853900817779268f * x) + 1.f), 1.f);
@@ -874,7 +877,7 @@ __global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_
       auto bc = [&](int b) { return bias[b][lg4]; };
       if constexpr (BF16) {
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) h0[jj] = tanh_fast(ca[jj] + cb[jj]);
+        for (int jj = 0; jj < 4; jj++) h0[jj] = tanhf(ca[jj] + cb[jj]);
         auto wa = [&](int b) { return wt.op[b][ln]; };
         const bf16x8 x = {(__bf16)h0[0], (__bf16)h0[1], (__bf16)h0[2], (__bf16)h0[3],
                           (__bf16)lg,    (__bf16)l4,    (__bf16)0.f,   (__bf16)0.f};

@@ -206,6 +206,48 @@ def test_predict_fp32_and_bf16_match_oracle(O, P):
     assert e16 < 3e-2
 
 
+def _predict_and_oracle(P, n, lam, T, theta):
+    """FP32 and bf16 predictions of given features and the FP64 stress, all
+    (6, n^3)"""
+    m = P.Closure(n)
+    try:
+        m.put_fields(lam, T)
+        m.set_params(theta)
+        m.predict(bf16=False)
+        got32 = m.field(P.SGS_PREDICTED).reshape(6, -1)
+        m.predict(bf16=True)
+        got16 = m.field(P.SGS_PREDICTED).reshape(6, -1)
+    finally:
+        m.close()
+    idx = np.arange(n ** 3)
+    X0 = SG.conv_inputs(lam.astype(np.float64), np.stack([idx // (n * n), (idx // n) % n, idx % n], axis=1))
+    want, _ = SG.forward(theta.astype(np.float64), X0, lam.reshape(5, -1).T.astype(np.float64),
+                         T.reshape(4, 6, -1).transpose(2, 0, 1).astype(np.float64))
+    return got32, got16, want.T
+
+
+@pytest.mark.parametrize("size", [2e-7, 1e-4])
+def test_predict_small_convolution_activations(P, size):
+    """The convolution and its tanh are FP32 in both modes, so activations of
+    any size reach the bf16 layers with bf16's relative rounding (2^-9 per
+    operand: the bound of the other predictions): here they are small, and the
+    first dense layer's weights bring them back to order one."""
+    print("[gpu case] sgs small convolution", size, flush=True)
+    n = 32
+    rng = np.random.default_rng(8)
+    lam = rng.standard_normal((5, n, n, n)).astype(np.float32)
+    T = rng.standard_normal((4, 6, n, n, n)).astype(np.float32)
+    p = SG.unpack(_theta(19))
+    p["W0"] = size / np.sqrt(SG.NIN0) * rng.standard_normal(p["W0"].shape)
+    p["b0"] = np.zeros(SG.NCONV)
+    p["W1"] = np.concatenate([np.zeros((SG.NHID, SG.NLAM)),
+                              rng.standard_normal((SG.NHID, SG.NCONV)) / (size * np.sqrt(SG.NCONV))], axis=1)
+    got32, got16, want = _predict_and_oracle(P, n, lam, T, SG.pack(p).astype(np.float32))
+    print("rel L2", rel(got32, want), rel(got16, want), flush=True)
+    assert rel(got32, want) < 1e-5
+    assert rel(got16, want) < 3e-2
+
+
 def _store(O, P, n, nsnap, seed):
     m = P.Closure(n, nsnap)
     rng = np.random.default_rng(seed)
