@@ -349,10 +349,12 @@ __global__ void __launch_bounds__(256)
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     // gather: point lane of the tile; wave w takes every fourth row of three
     // x neighbours, basis entry and stress component (points past B read
-    // point 0 and are left out of the loss)
+    // point 0 and hold zeros, so that nothing of a point that was not drawn,
+    // a NaN of it either, meets the sums)
     {
       const int b = t * kTS + lane;
-      const uint64_t gidx = b < B ? splitmix64(base + (uint64_t)b) % ((uint64_t)nsnap * P) : 0;
+      const bool live = b < B;
+      const uint64_t gidx = live ? splitmix64(base + (uint64_t)b) % ((uint64_t)nsnap * P) : 0;
       const size_t s = gidx / P, p = gidx % P;
       const int y = (int)(p / ((size_t)n * n)), z = (int)((p / n) & m), x = (int)(p & m);
       const float* lam = lam_s + s * kLam * P;
@@ -374,12 +376,12 @@ __global__ void __launch_bounds__(256)
       for (int i = 0; i < 12; i++)
         if (w + 4 * i < kLam * 9)
 #pragma unroll
-          for (int d = 0; d < 3; d++) X0s[(3 * (w + 4 * i) + d) * kLd + lane] = v[i][d];
+          for (int d = 0; d < 3; d++) X0s[(3 * (w + 4 * i) + d) * kLd + lane] = live ? v[i][d] : 0.f;
 #pragma unroll
-      for (int i = 0; i < 6; i++) Ts[(w + 4 * i) * kTS + lane] = tv[i];
+      for (int i = 0; i < 6; i++) Ts[(w + 4 * i) * kTS + lane] = live ? tv[i] : 0.f;
 #pragma unroll
       for (int i = 0; i < 2; i++)
-        if (w + 4 * i < 6) taus[(w + 4 * i) * kTS + lane] = uv[i];
+        if (w + 4 * i < 6) taus[(w + 4 * i) * kTS + lane] = live ? uv[i] : 0.f;
     }
     __syncthreads();
     // forward

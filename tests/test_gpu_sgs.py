@@ -319,6 +319,39 @@ def test_minibatch_gradient_tile_edges(O, P, B):
         off += cnt
 
 
+@pytest.mark.parametrize("B", [1, 63, 65])
+def test_minibatch_gradient_of_drawn_points_only(O, P, B):
+    """a tile that the batch does not fill takes nothing from the store for its
+    other points: with every point that the batch does not read a NaN, the
+    gradient and the loss keep their bits"""
+    print("[gpu case] sgs gradient, points not drawn", B, flush=True)
+    n, seed, step = 32, 5, 3
+    lam, T = _features(O, n, 61)
+    tau = (0.02 * np.random.default_rng(61).standard_normal((6, n, n, n))).astype(np.float32)
+    idx = SG.sample_points(seed, step, B, 1, n ** 3)
+    read = np.zeros((n, n, n), bool)
+    for p in np.asarray(idx).ravel():
+        y, z, x = int(p) // (n * n), int(p) // n % n, int(p) % n
+        read[np.ix_(*[[(c - 1) % n, c, (c + 1) % n] for c in (y, z, x)])] = True
+    assert not read[0, 0, 0]
+    out = []
+    for fill in (None, np.nan):
+        a = [f.copy() for f in (lam, T, tau)]
+        if fill is not None:
+            for f in a:
+                f[..., ~read] = fill
+        m = P.Closure(n, 1)
+        try:
+            m.put_fields(*a)
+            m.add_snapshot()
+            m.set_params(_theta(7))
+            out.append(m.gradient(B, seed, step, 1e-3))
+        finally:
+            m.close()
+    assert np.isfinite(out[0][0]).all()
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
 def test_adam_step_matches_oracle(O, P):
     print("[gpu case] sgs adam", flush=True)
     n, nsnap, B, seed, lr = 32, 2, 1024, 9, 1e-3
