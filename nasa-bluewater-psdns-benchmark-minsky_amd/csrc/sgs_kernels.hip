@@ -348,13 +348,13 @@ __global__ void __launch_bounds__(256)
   const int ntiles = (B + kTS - 1) / kTS;
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     // gather: point lane of the tile; wave w takes every fourth row of three
-    // x neighbours, basis entry and stress component (points past B read
-    // point 0 and hold zeros, so that nothing of a point that was not drawn,
-    // a NaN of it either, meets the sums)
+    // x neighbours, basis entry and stress component (points past B repeat the
+    // batch's last one with a zero gradient, so that no value meets the sums
+    // that the batch does not have: not a point that was not drawn, and not a
+    // zero input to an infinite weight)
     {
-      const int b = t * kTS + lane;
-      const bool live = b < B;
-      const uint64_t gidx = live ? splitmix64(base + (uint64_t)b) % ((uint64_t)nsnap * P) : 0;
+      const int b = min(t * kTS + lane, B - 1);
+      const uint64_t gidx = splitmix64(base + (uint64_t)b) % ((uint64_t)nsnap * P);
       const size_t s = gidx / P, p = gidx % P;
       const int y = (int)(p / ((size_t)n * n)), z = (int)((p / n) & m), x = (int)(p & m);
       const float* lam = lam_s + s * kLam * P;
@@ -376,12 +376,12 @@ __global__ void __launch_bounds__(256)
       for (int i = 0; i < 12; i++)
         if (w + 4 * i < kLam * 9)
 #pragma unroll
-          for (int d = 0; d < 3; d++) X0s[(3 * (w + 4 * i) + d) * kLd + lane] = live ? v[i][d] : 0.f;
+          for (int d = 0; d < 3; d++) X0s[(3 * (w + 4 * i) + d) * kLd + lane] = v[i][d];
 #pragma unroll
-      for (int i = 0; i < 6; i++) Ts[(w + 4 * i) * kTS + lane] = live ? tv[i] : 0.f;
+      for (int i = 0; i < 6; i++) Ts[(w + 4 * i) * kTS + lane] = tv[i];
 #pragma unroll
       for (int i = 0; i < 2; i++)
-        if (w + 4 * i < 6) taus[(w + 4 * i) * kTS + lane] = live ? uv[i] : 0.f;
+        if (w + 4 * i < 6) taus[(w + 4 * i) * kTS + lane] = uv[i];
     }
     __syncthreads();
     // forward
@@ -400,7 +400,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int jj = 0; jj < 4; jj++) d[jj] = b1s[16 * ob + 4 * g + jj];
       d = mm(wr[g], l0, d);
-      d = mm(wr[4], l1, d);
+      d = mm(g == 0 ? wr[4] : 0.f, l1, d);  // an empty slot is zero in both operands
 #pragma unroll
       for (int jj = 0; jj < 4; jj++) d = mm(wr[kLam + 4 * g + jj], h0[jj], d);
 #pragma unroll
@@ -619,10 +619,13 @@ __global__ void __launch_bounds__(256)
 // The convolution runs on v_mfma_f32_16x16x4_f32 (FP32 operands and sums), K =
 // 135 in 34 steps: steps 0 .. 26 are the taps of channels 0 .. 3 (slot g =
 // channel g, so a tap's LDS reads differ by a lane constant and hit all 64
-// banks once), steps 27 .. 33 four taps each of channel 4.  On the VALU, a
-// point per thread with its 135 neighbours from the cache, it took 178 us at
-// 128^3 (116 us at the full FP32 rate; packed FP32 is off), and an earlier
-// matrix form with gathered global reads and a fourth of its slots empty 207.
+// banks once), steps 27 .. 33 four taps each of channel 4.  The slot past its
+// last tap is zero in both operands, as are the empty slots of layer 1: zero
+// times an infinite value would be a NaN that the point does not have.  On the
+// VALU, a point per thread with its 135 neighbours from the cache, the
+// convolution took 178 us at 128^3 (116 us at the full FP32 rate; packed FP32 is
+// off), and an earlier matrix form with gathered global reads and a fourth of
+// its slots empty 207.
 //
 // The dense layers, BF16: v_mfma_f32_16x16x32_bf16 (bf16 operands, FP32
 // accumulation), eight K slots (g, j) per lane and step; else
@@ -864,6 +867,7 @@ __global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_
         float v;
         if constexpr (s < kTaps) v = hp[g * kHch + tap_off(s)];
         else v = hp[off4[s - kTaps]];
+        if constexpr (s == kSteps - 1) v = g == 3 ? 0.f : v;  // past the last tap
         if constexpr (s == 13) lg = v;
         if constexpr (s == kTaps + 3) l4 = g == 1 ? v : 0.f;
         f32x4& acc = s % 2 ? cb : ca;
@@ -908,7 +912,7 @@ __global__ void __launch_bounds__(64 * kCWaves) __attribute__((amdgpu_waves_per_
         for (int ob = 0; ob < 4; ob++) {
           const float* wr = wt.W1 + (16 * ob + c) * kIn1;
           d[ob] = mm(wr[g], lg, bc(ob));
-          d[ob] = mm(wr[4], l4, d[ob]);
+          d[ob] = mm(g == 1 ? wr[4] : 0.f, l4, d[ob]);
 #pragma unroll
           for (int jj = 0; jj < 4; jj++) d[ob] = mm(wr[kLam + 4 * g + jj], h0[jj], d[ob]);
         }

@@ -248,6 +248,54 @@ def test_predict_small_convolution_activations(P, size):
     assert rel(got16, want) < 3e-2
 
 
+@pytest.mark.parametrize("where", ["weight", "field"])
+def test_infinite_value_saturates(P, where):
+    """An infinite weight of lambda_4 in the first dense layer, or one infinite
+    value of the invariant field, saturates the units that it reaches (tanh = +-1)
+    and no others: the matrix steps' empty slots add nothing to the sums.  The
+    bounds are those of the other predictions."""
+    print("[gpu case] sgs infinite", where, flush=True)
+    n = 32
+    rng = np.random.default_rng(12)
+    lam = (0.5 * rng.standard_normal((5, n, n, n))).astype(np.float32)
+    T = rng.standard_normal((4, 6, n, n, n)).astype(np.float32)
+    p = SG.unpack(_theta(23).astype(np.float64))
+    if where == "weight":
+        p["W1"] = p["W1"].copy()
+        p["W1"][11, 4] = np.inf
+    else:
+        lam[4, 3, 30, 17] = np.inf
+    got32, got16, want = _predict_and_oracle(P, n, lam, T, SG.pack(p).astype(np.float32))
+    assert np.isfinite(want).all()
+    assert rel(got32, want) < 1e-5
+    assert rel(got16, want) < 3e-2
+
+
+def test_gradient_with_an_infinite_weight(O, P):
+    """the same weight in training: the unit is saturated, its own gradient zero
+    and the others as the oracle's (the bound of the gradient tests)"""
+    print("[gpu case] sgs gradient, infinite weight", flush=True)
+    n, B, seed, step = 32, 200, 5, 3
+    m, lam_s, T_s, tau_s = _store(O, P, n, 1, 61)
+    p = SG.unpack(_theta(7).astype(np.float64))
+    p["W1"] = p["W1"].copy()
+    p["W1"][11, 4] = np.inf
+    theta = SG.pack(p).astype(np.float32)
+    try:
+        sigma2 = m.target_scale()
+        m.set_params(theta)
+        grad, loss = m.gradient(B, seed, step, sigma2)
+    finally:
+        m.close()
+    idx = SG.sample_points(seed, step, B, 1, n ** 3)
+    X0, lam_pt, T, tau = SG.batch_arrays(lam_s, T_s.reshape(1, 4, 6, n, n, n), tau_s, idx)
+    assert (lam_pt[:, 4] != 0).all()
+    L, g = SG.loss_and_grad(theta.astype(np.float64), X0, lam_pt, T, tau, sigma2)
+    assert np.isfinite(g).all()
+    assert abs(loss - L) <= 1e-5 * L
+    assert rel(grad, g) < 1e-4
+
+
 def _store(O, P, n, nsnap, seed):
     m = P.Closure(n, nsnap)
     rng = np.random.default_rng(seed)
