@@ -53,8 +53,7 @@ struct psdns_sgs {
   size_t P = 0;       // n^3
   int max_snap = 0, nsnap = 0;
   hipStream_t stream = nullptr;
-  // spectral gradient work (sized for FP64 on first use: na from the context)
-  int na = 0, max_al_x = 0;
+  // spectral gradient work (sized for FP64 on first use)
   void *yw = nullptr, *xi = nullptr, *A = nullptr;
   int A_prec = 0;     // precision of the gradient in A (that of the last features context)
   // current field: features, target, prediction
@@ -227,16 +226,14 @@ int features(psdns_sgs* m, psdns_ctx* c, int stage) {
   // reads the cylinder u slots 0..2; its own buffers for the transforms
   if ((rc = psdns::ctx_access(c, false, false, &k, &n))) return rc;
   if (n != m->n) return set_error(PSDNS_EINVAL, "grid %d: the closure is for n = %d", n, m->n);
-  if (!m->yw) {
-    const size_t cb = sizeof(double) * 2 * 6 * (size_t)k.geo.na * n;
-    const size_t xb = sizeof(double) * 2 * 9 * (size_t)n * k.geo.max_al_x * n;
-    if ((rc = dalloc((char**)&m->yw, cb, "the gradient cylinder")) ||
-        (rc = dalloc((char**)&m->xi, xb, "the gradient z pencils")) ||
-        (rc = dalloc((char**)&m->A, sizeof(double) * 9 * m->P, "the gradient")))
-      return rc;
-    m->na = k.geo.na;
-    m->max_al_x = k.geo.max_al_x;
-  }
+  // (each by itself: a call that ran out of memory leaves the ones it got, and a
+  // later call the ones that are missing)
+  const size_t cb = sizeof(double) * 2 * 6 * (size_t)k.geo.na * n;
+  const size_t xb = sizeof(double) * 2 * 9 * (size_t)n * k.geo.max_al_x * n;
+  if ((!m->yw && (rc = dalloc((char**)&m->yw, cb, "the gradient cylinder"))) ||
+      (!m->xi && (rc = dalloc((char**)&m->xi, xb, "the gradient z pencils"))) ||
+      (!m->A && (rc = dalloc((char**)&m->A, sizeof(double) * 9 * m->P, "the gradient"))))
+    return rc;
   // the y pass forms Y[u_i] and Y[i ky u_i] on the mask, phase shifted (in FP64)
   // for a stage; the z pass the three derivatives of each component
   Ctx g = k;
