@@ -210,18 +210,21 @@ int ensure_force_list(psdns_ctx* c, int kfor) {
       list.push_back(make_int2(a, y));
     }
   }
+  // no list until the new one is whole (a call may fail on the way)
+  c->force_kfor = -1;
+  c->nforce = c->c.nforce = 0;
+  c->c.force_list = nullptr;
   if (c->d_force) HIPCHK(hipFree(c->d_force));
-  if (c->d_force_terms) HIPCHK(hipFree(c->d_force_terms));
   c->d_force = nullptr;
+  if (c->d_force_terms) HIPCHK(hipFree(c->d_force_terms));
   c->d_force_terms = nullptr;
-  c->nforce = (int)list.size();
   if (!list.empty()) {
     HIPCHK(hipMalloc(&c->d_force, sizeof(int2) * list.size()));
     HIPCHK(hipMalloc(&c->d_force_terms, (sizeof(double) + sizeof(int)) * list.size()));
     HIPCHK(hipMemcpy(c->d_force, list.data(), sizeof(int2) * list.size(), hipMemcpyHostToDevice));
   }
   c->c.force_list = c->d_force;
-  c->c.nforce = c->nforce;
+  c->nforce = c->c.nforce = (int)list.size();
   c->force_kfor = kfor;
   return 0;
 }

@@ -49,7 +49,7 @@ def harness(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["features"])
+@pytest.mark.parametrize("case", ["features", "force_list"])
 def test_call_after_a_failed_allocation(harness, case):
     r = subprocess.run([str(harness), case], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
