@@ -744,9 +744,32 @@ struct XPass {
   }
 };
 
-// The wave's sums over its lanes, by pairs (a fixed order).
+// Lanes of this wave in a work-group of NT threads (NT % 64 zero or a power of
+// two): the reductions below exchange between these only, as a shuffle from a
+// lane that the work-group does not have is undefined.
+template <int NT>
+__device__ __forceinline__ int wave_lanes() {
+  constexpr int kRest = NT % 64;
+  static_assert((kRest & (kRest - 1)) == 0, "the last wave's lanes pair up");
+  if (kRest == 0) return 64;
+  if (NT < 64) return NT;
+  return __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64) == NT / 64 ? kRest : 64;
+}
+// The wave's sum and maximum over its lanes, by pairs (a fixed order).
+template <int NT = 64>
 __device__ __forceinline__ double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  const int lanes = wave_lanes<NT>();
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    if (off < lanes) v += __shfl_xor(v, off);
+  return v;
+}
+template <int NT = 64>
+__device__ __forceinline__ double wave_max(double v) {
+  const int lanes = wave_lanes<NT>();
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    if (off < lanes) v = fmax(v, __shfl_xor(v, off));
   return v;
 }
 
@@ -825,7 +848,7 @@ __global__ void __launch_bounds__((XPass<R, N, MOM>::NT))
     __shared__ double red[NW][8];
 #pragma unroll
     for (int m = 0; m < 8; m++) {
-      const double v = wave_sum(s[m]);
+      const double v = wave_sum<X::NT>(s[m]);
       if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][m] = v;
     }
     __syncthreads();
@@ -882,11 +905,12 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
 // 256 bytes apart, chosen by work-group, so that the atomics spread over
 // the L2 channels instead of queueing on one address; k_velmax_reduce takes
 // the maximum of the slots and clears them for the next use.  Non-negative doubles order as their bit patterns.
-// Every thread of the work-group calls it (one barrier inside).
+// Every thread of the work-group (NT) calls it (one barrier inside).
+template <int NT>
 __device__ __forceinline__ void velmax_commit(double m, unsigned long long* velmax) {
-  __shared__ double wmax[16];
-  for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off));
-  const int nw = (blockDim.x + 63) >> 6;
+  constexpr int nw = (NT + 63) / 64;
+  __shared__ double wmax[nw];
+  m = wave_max<NT>(m);
   if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -1025,7 +1049,7 @@ __attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : XPass<R, N, !TAU>::kWa
       t = tn;
     }
   }
-  if (want_velmax) velmax_commit((double)vm * (double)N, velmax);
+  if (want_velmax) velmax_commit<X::NT>((double)vm * (double)N, velmax);
 }
 
 // The fused x pass of small grids (without scalars), where a tile's chain of three inverse and
@@ -1073,7 +1097,7 @@ __global__ void __launch_bounds__((5 * XPass<R, N>::NT))
   if constexpr (TAU) X::add_tau(v, tau, gr, y, z0, tid);
   X::template r2c<false>(v, xs, 0, y, z0, g, own, stw, (R)1, tid,
                          (unsigned)gr * (unsigned)(xidx<X::K>(1, y, z0, 0, g) - xidx<X::K>(0, y, z0, 0, g)));
-  if (want_velmax) velmax_commit((double)vm * (double)N, velmax);
+  if (want_velmax) velmax_commit<G * NT>((double)vm * (double)N, velmax);
 }
 
 // realspace_vel alone on physical ux (slots 0..4)
@@ -1088,7 +1112,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int s = 0; s < 5; s++) ux[s * n3 + i] = product(s, u, v, w);
   }
-  if (want_velmax) velmax_commit(vm * xnorm, velmax);
+  if (want_velmax) velmax_commit<256>(vm * xnorm, velmax);
 }
 
 // ---------------------------------------------------------------------------

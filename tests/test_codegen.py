@@ -73,3 +73,15 @@ def test_no_wide_store_data_overwritten_by_next_instruction(disassembly):
             if a <= hi and b >= lo:
                 bad.append((l.strip(), lines[i + 1].strip()))
     assert not bad, f"{len(bad)} wide stores whose data the next instruction writes, e.g. {bad[0]}"
+
+
+@pytest.mark.parametrize("kernel,threads,values", [
+    ("k_x_c2rIfLi32ELb1E", 32, 8), ("k_x_c2rIdLi32ELb1E", 16, 8), ("k_x_c2rIdLi64ELb1E", 32, 8),
+    ("k_x_c2rIfLi64ELb1E", 64, 8), ("k_x_fusedIfLi32ELb0ELb1E", 32, 1), ("k_x_fusedIdLi32ELb0ELb1E", 16, 1)])
+def test_reductions_exchange_within_the_work_group(disassembly, kernel, threads, values):
+    """The moment sums and the velocity maximum of a work-group smaller than a
+    wavefront take log2(threads) exchanges of a double (two words): a further one
+    would read lanes that the work-group does not have."""
+    code = re.search(rf"<_ZN5psdns\d+{kernel}\w*>:\n(.*?)(?:\n\n|\Z)", disassembly, re.S)
+    assert code, f"no kernel {kernel}"
+    assert code.group(1).count("ds_bpermute_b32") == 2 * values * (threads.bit_length() - 1)
