@@ -57,7 +57,11 @@ __device__ __forceinline__ size_t pidx(int y, int z, int x, int n) { return ((si
 // right end tap from the neighbour's line.  A fine row is read by up to four
 // coarse rows, which are close in time on one XCD (xcd_block): from memory
 // about once.  512^3 FP32 to 64^3: 1650 us with a thread per coarse point and
-// strided taps, 394 us this way (1.6 GB read, 4.1 TB/s).
+// strided taps, 394 us this way (1.6 GB read, 4.1 TB/s).  A row's loads are kept
+// ahead of its sums, which the compiler does by itself in FP32 but not in FP64
+// from r = 8 on: 512^3 FP64 to 32^3 2.49 ms with strided taps, 3.95 ms with the
+// loads among the sums, 0.86 ms (3.2 GB, 3.8 TB/s); 1024^3 FP64 to 32^3 18.7,
+// 30.1 and 5.5 ms; 256^3 FP64 to 32^3 268, 168 and 95 us.
 // ---------------------------------------------------------------------------
 template <typename R, int H>
 struct Half {  // H consecutive values
@@ -102,6 +106,9 @@ __global__ void __launch_bounds__(256)
         hi[v].load(row + v * N3 + x1);
         end[v] = row[v * N3 + x2];
       }
+      // the lanes of a wave are r values apart: a line that is not taken whole by
+      // loads in a row is gone from the cache before its next one
+      if constexpr (sizeof(R) == 8) __builtin_amdgcn_sched_barrier(0);
       double t[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
       for (int i = 0; i <= r; i++) {

@@ -73,6 +73,39 @@ def test_box_filter_ratios(O, P, n, nc, prec):
         assert np.abs(got_t[:, y, z, x] - tau).max() < 1.2e-7 * np.abs(tau).max()
 
 
+@pytest.mark.parametrize("n,prec", [(256, 8), (512, 8), (1024, 4), (1024, 8)])
+def test_box_filter_wide_ratios(P, n, prec):
+    """ratios 8, 16 and 32 in FP64 and 32 in FP32, of a random solenoidal field
+    in physical space, at coarse points on the sides and inside; direct FP64
+    sums and the bounds of the test above"""
+    print("[gpu case] sgs box wide ratios", n, prec, flush=True)
+    nc = 32
+    r = n // nc
+    fine, coarse, m = P.Solver(n, prec), P.Solver(nc, prec), P.Closure(nc)
+    try:
+        fine.init_field(seed=n + prec, kpeak=6.0, tke=0.5)
+        fine.kxtran(3)
+        m.filter(fine, coarse)
+        u = fine.get_field(P.FIELD_UX, 3)
+        got_u = coarse.get_field(P.FIELD_UX, 3)
+        got_t = m.field(P.SGS_TARGET)
+    finally:
+        m.close()
+        fine.close()
+        coarse.close()
+    offs, w = SG.box_weights(r)
+    w3 = w[:, None, None] * w[None, :, None] * w[None, None, :]
+    for c in [(0, 0, 0), (nc - 1, 0, nc - 1), (0, nc - 1, 1), (5, 7, nc // 2), (30, 31, 30)]:
+        at = np.ix_(range(3), *[(r * ci + offs) % n for ci in c])
+        b = u[at].astype(np.float64)
+        ub = (b * w3).sum((1, 2, 3))
+        tau = np.array([(b[i] * b[j] * w3).sum() - ub[i] * ub[j] for i, j in SG.SYM])
+        tau[[0, 3, 5]] -= (tau[0] + tau[3] + tau[5]) / 3.0
+        y, z, x = c
+        assert rel(got_u[:, y, z, x], ub) < (1e-13 if prec == 8 else 1.2e-7)
+        assert np.abs(got_t[:, y, z, x] - tau).max() < 1.2e-7 * np.abs(tau).max()
+
+
 @pytest.mark.parametrize("shifted", [False, True], ids=["unshifted", "phase1"])
 def test_features_match_oracle(O, P, shifted):
     print("[gpu case] sgs features", shifted, flush=True)
