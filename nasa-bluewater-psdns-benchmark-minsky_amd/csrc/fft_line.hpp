@@ -327,27 +327,38 @@ struct TeamFft {
   }
   static constexpr int kTwEntries = tw_off(L);
 
-  // Fill the LDS table from tw[k] = exp(-2 pi i k / (L TSTRIDE)), k < L
-  // TSTRIDE (a table that may belong to a longer transform); all threads
-  // tid < nthr of the work-group take part.  Readers must pass a barrier
+  // Fill the LDS table from tw[k] = exp(-2 pi i k / L), k < L; the threads tid <
+  // NTHR of the work-group take part, each with all of its loads in flight (a
+  // loop of a load and its store waits for each).  Readers must pass a barrier
   // first (every run() does before its first twiddle).
-  template <int TSTRIDE>
-  static __device__ __forceinline__ void fill_twiddles(cpx<R>* stw, const cpx<R>* __restrict__ tw, int tid,
-                                                       int nthr) {
-    for (int e = tid; e < kTwEntries; e += nthr) {
-      int s = E, off = 0;
-      while (e >= off + tw_entries(s)) {
-        off += tw_entries(s);
-        s *= rad_at(s);
-      }
-      const int k = e - off, rad = rad_at(s);
-      int m;
-      if (two_level(s)) {
-        m = (k < s / 16 ? 16 * k : k - s / 16) * (L / (2 * s));
-      } else {
-        m = (k % s) * (k / s + 1) * (L / (s * rad));
-      }
-      stw[e] = tw[m * TSTRIDE];
+  template <int NTHR>
+  static __device__ __forceinline__ void fill_twiddles(cpx<R>* stw, const cpx<R>* __restrict__ tw, int tid) {
+    constexpr int n = (kTwEntries + NTHR - 1) / NTHR;
+    cpx<R> v[n];
+#pragma unroll
+    for (int i = 0; i < n; i++) {
+      const int e = tid + i * NTHR;
+      v[i] = tw[tw_index<E>(e < kTwEntries ? e : kTwEntries - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < n; i++)
+      if ((i + 1) * NTHR <= kTwEntries || tid + i * NTHR < kTwEntries) stw[tid + i * NTHR] = v[i];
+  }
+  // m of entry e, which belongs to the stage of span S or a later one
+  template <int S>
+  static __device__ __forceinline__ int tw_index(int e) {
+    constexpr int rad = rad_at(S), next = tw_off(S) + tw_entries(S);
+    const unsigned k = (unsigned)(e - tw_off(S));
+    int m;
+    if constexpr (two_level(S)) {
+      m = (int)(k < S / 16 ? 16 * k : k - S / 16) * (L / (2 * S));
+    } else {
+      m = (int)((k % S) * (k / S + 1)) * (L / (S * rad));
+    }
+    if constexpr (next < kTwEntries) {
+      return e < next ? m : tw_index<S * rad>(e);
+    } else {
+      return m;
     }
   }
 

@@ -272,7 +272,7 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
   __shared__ C<R> ssy[MODE == 0 ? N : 1];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   if constexpr (MODE == 0)
     for (int k = threadIdx.x; k < N; k += F::NT) ssy[k] = sr[g.nxh + k];
   const int tid = threadIdx.x;
@@ -354,7 +354,7 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
   __shared__ std::conditional_t<SH == 2, double2, C<R>> ssy[SH ? N : 1];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   if constexpr (SH == 1)
     for (int k = threadIdx.x; k < N; k += F::NT) ssy[k] = sr[g.nxh + k];
   if constexpr (SH == 2)
@@ -440,7 +440,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T)) __attribute__((
   using F = TeamFft<R, N, E, B, +1, LineShift<E, B>::IN>;
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   const int tid = threadIdx.x;
   const Slot<R> in = F::transposed(lds, tid);
   const Slot<R> out = F::natural(lds, tid);
@@ -572,7 +572,7 @@ struct XPass {
 
   // stage twiddles of a work-group in LDS (fill ends with a barrier)
   static __device__ __forceinline__ void fill(C<R>* stw, const C<R>* __restrict__ tw) {
-    FI::template fill_twiddles<1>(stw, tw, threadIdx.x, NT);
+    FI::template fill_twiddles<NT>(stw, tw, threadIdx.x);
     __syncthreads();
   }
 
@@ -795,7 +795,6 @@ __global__ void __launch_bounds__((XPass<R, N, MOM>::NT))
   __shared__ R lds[X::kLdsReals];
   __shared__ C<R> stw[X::kTw];
   __shared__ __attribute__((aligned(16))) C<R> S[X::M * B];
-  X::fill(stw, tw);
   const int var = blockIdx.y;
   const TileWalk w = tile_walk(N * NZB);
   double s[MOM ? 8 : 1];
@@ -804,6 +803,7 @@ __global__ void __launch_bounds__((XPass<R, N, MOM>::NT))
   int t = w.t;
   if (t < w.end) {
     X::stage_load(S, xi, var, t / NZB, (t % NZB) * B, g, true);
+    X::fill(stw, tw);
     for (;;) {
       const int y = t / NZB, z0 = (t % NZB) * B, tn = t + w.step;
       C<R> v[E];
@@ -880,14 +880,19 @@ __global__ void __launch_bounds__(kMomFold)
   if (threadIdx.x < 8) out[8 * blockIdx.x + m] = red[threadIdx.x];
 }
 
-// forward x pass alone: physical ux (nv variables) -> X, x 1/n
+// forward x pass alone: physical ux (nv variables) -> X, x 1/n.  A tile per
+// work-group, its loads issued ahead of the table fill: with the fill first, and
+// waiting for each of its loads, the pass took 1200 us for three variables at
+// 512^3 FP64, 178 at 256^3 and 5.5 ms at 1024^3 FP32, this way 1095-1150, 150-160
+// us and 4.3 ms (1117, 153 us and 4.7 ms with half-length transforms, whose table
+// is half as long).  Persistent work-groups with the next tile loaded ahead: 1300
+// us at 512^3 FP64.
 template <typename R, int N>
 __global__ void __launch_bounds__((XPass<R, N>::NT))
     k_x_r2c(const R* __restrict__ ux, C<R>* __restrict__ xs, Geo g, const C<R>* __restrict__ tw) {
   using X = XPass<R, N>;
   __shared__ R lds[X::kLdsReals];
   __shared__ C<R> stw[X::kTw];
-  X::fill(stw, tw);
   const int2 blk = xcd_block2();
   const int var = blk.y;
   const int y = blk.x / (N / X::B), z0 = (blk.x % (N / X::B)) * X::B;
@@ -896,6 +901,8 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
   C<R> v[X::E];
 #pragma unroll
   for (int j = 0; j < X::E; j++) v[j] = {src[q + X::T * j], src[N + q + X::T * j]};
+  issue_fence();
+  X::fill(stw, tw);
   X::template r2c<true>(v, xs, var, y, z0, g, lds, stw, (R)1 / (R)N);
 }
 
@@ -1074,7 +1081,7 @@ __global__ void __launch_bounds__((5 * XPass<R, N>::NT))
   const int t = tile_walk(N * NZB).t;  // one tile per work-group
   const int y = t / NZB, z0 = (t % NZB) * B;
   X::stage_load3(S, xi, y, z0, g, G * NT / 64);
-  X::FI::template fill_twiddles<1>(stw, tw, threadIdx.x, G * NT);
+  X::FI::template fill_twiddles<G * NT>(stw, tw, threadIdx.x);
   const int gr = (int)threadIdx.x / NT, tid = (int)threadIdx.x % NT;
   R* own = lds + gr * X::kLdsReals;
   X::stage_publish();
@@ -1191,7 +1198,7 @@ __global__ void __launch_bounds__((ZFwd<R, N>::NT)) __attribute__((amdgpu_waves_
   constexpr int T = Z::T, E = Z::E, B = Z::B;
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   const int tid = threadIdx.x;
   const Slot<R> in = F::transposed(lds, tid);
   const Slot<R> out = F::natural(lds, tid);
@@ -1266,7 +1273,7 @@ __global__ void __launch_bounds__((5 * ZFwd<R, N>::NT))
   typename Z::Buf b;
   Z::load(b, xs, g, nkb, t, 0, true, F::transposed_line(tid), in.q,
           (unsigned)gr * (unsigned)(xidx<B>(1, 0, 0, 0, g) - xidx<B>(0, 0, 0, 0, g)));
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, G * NT);
+  F::template fill_twiddles<G * NT>(stw, tw, threadIdx.x);
   __syncthreads();
   F::template run<false, ZFRESH, true, false>(b.v, own, in, out, stw, tid);
   if (gr == 4) {
@@ -1301,7 +1308,7 @@ __global__ void __launch_bounds__((ZFwd<R, N>::NT)) __attribute__((amdgpu_waves_
   constexpr int E = Z::E, B = Z::B;
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   const int tid = threadIdx.x;
   const Slot<R> in = F::transposed(lds, tid);
   const Slot<R> out = F::natural(lds, tid);
@@ -1349,7 +1356,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T))
   using F = TeamFft<R, N, E, B, -1, LineShift<E, B>::IN>;
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   const int tid = threadIdx.x;
   const int2 blk = xcd_block2();
   const int var = blk.y;
@@ -1601,7 +1608,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * YUpd<R, N>::T))
   __shared__ C<R> ssy[N];
   __shared__ R syf[IF ? N : 1];  // yfac in the state precision
   __shared__ C<R> ssy2[INV2 ? N : 1];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   for (int k = threadIdx.x; k < N; k += F::NT) {
     ssy[k] = sr[g.nxh + k];
     if constexpr (IF) syf[k] = (R)yfac[k];
@@ -2274,7 +2281,7 @@ __global__ void __launch_bounds__((RunLines<R>::B * Team<N>::T))
   using F = TeamFft<R, N, E, B, -1, LineShift<E, B>::IN>;
   __shared__ R lds[F::kLdsReals];
   __shared__ C<R> stw[F::kTwEntries];
-  F::template fill_twiddles<1>(stw, tw, threadIdx.x, F::NT);
+  F::template fill_twiddles<F::NT>(stw, tw, threadIdx.x);
   const int tid = threadIdx.x;
   const int2 grp = g.grp[xcd_block(blockIdx.x, gridDim.x)];
   const Slot<R> in = F::transposed(lds, tid);

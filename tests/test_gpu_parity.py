@@ -237,6 +237,31 @@ def test_stage_with_and_without_scalars(O, P, ctxs, n, prec):
     assert rel(out[0][2], out[1][2], m) < TOL[prec]
 
 
+@pytest.mark.parametrize("n,prec", [(32, 8), (128, 8), (256, 4), (256, 8), (512, 4), (512, 8), (1024, 4)])
+def test_transform_pair_returns_the_field(P, n, prec):
+    """kxtran and xktran of a field on the mask give the field back, for each
+    number of points per thread and threads per line of the x passes (the
+    rounding of two three-dimensional transforms of 3 log2(n) stages, below
+    10 eps in the L2 norm)"""
+    banner("kxtran, xktran", n, prec)
+    s = P.Solver(n, prec, viscos=0.01)
+    try:
+        s.init_field(seed=n + prec, kpeak=n / 8, tke=0.5)
+        u = s.get_state()
+        for _ in range(2):
+            s.kxtran(3)
+            s.xktran(3)
+        got = s.get_field(P.FIELD_U, 3)
+    finally:
+        s.close()
+    on = u != 0
+    assert on.mean() > 0.3
+    d = np.where(on, got - u, 0)
+    err = np.linalg.norm(d.ravel()) / np.linalg.norm(u.ravel())
+    print(f"two transform pairs: rel L2 {err:.2e}", flush=True)
+    assert err < 20 * np.finfo(np.float64 if prec == 8 else np.float32).eps
+
+
 @pytest.mark.parametrize("n,prec", [(64, 8), (64, 4)])
 def test_deferred_update_keeps_its_shifts(O, P, ctxs, n, prec):
     """stage_update(1) runs in the next call; new shifts set in between apply
