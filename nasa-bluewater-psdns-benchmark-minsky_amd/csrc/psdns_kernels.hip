@@ -973,13 +973,19 @@ __device__ __forceinline__ R product(int s, R u, R v, R w) {
 // its r2c x 1/n into X slot 5 + s, so the velocity's c2r serves every
 // scalar; the gradients go through the same staging buffer in order, the
 // last one followed by the next tile's u.
-#ifndef PSDNS_XSC_WAVES
-#define PSDNS_XSC_WAVES 2
-#endif
+// Waves per SIMD that the registers of the pass with scalars are sized for: two
+// hold u, v, w, the sum and a gradient of 16 points FP32 or 8 points FP64 but
+// for some spills, which at 512^3 FP64 (50 registers) cost more than the second
+// wave brings: 4.9 ms, with one wave 3.85 (4.1-4.25 with half-length transforms of
+// 4 points; 4 points here 4.2).  At 1024^3 one wave is slower, in FP64 38.4-39.2
+// -> 40.6 ms (36.8 with half-length transforms, whose lines were one wave each), in
+// FP32 18.6 -> 21.2 (19.0).
+template <typename R, int N>
+constexpr int kScWaves = sizeof(R) == 8 && N == 512 ? 1 : 2;
 template <typename R, int N, bool TAU, bool SC = false>
 __global__ void __launch_bounds__((XPass<R, N, !TAU>::NT))
-__attribute__((amdgpu_waves_per_eu(SC ? PSDNS_XSC_WAVES : XPass<R, N, !TAU>::kWaves,
-                                    SC ? PSDNS_XSC_WAVES : XPass<R, N, !TAU>::kWaves)))
+__attribute__((amdgpu_waves_per_eu(SC ? kScWaves<R, N> : XPass<R, N, !TAU>::kWaves,
+                                    SC ? kScWaves<R, N> : XPass<R, N, !TAU>::kWaves)))
     k_x_fused(const C<R>* __restrict__ xi, C<R>* __restrict__ xs, Geo g, const C<R>* __restrict__ tw,
               unsigned long long* __restrict__ velmax, int want_velmax, const float* __restrict__ tau, int nsc,
               ScGrad scg) {

@@ -241,8 +241,8 @@ def test_stage_with_and_without_scalars(O, P, ctxs, n, prec):
 def test_transform_pair_returns_the_field(P, n, prec):
     """kxtran and xktran of a field on the mask give the field back, for each
     number of points per thread and threads per line of the x passes (the
-    rounding of two three-dimensional transforms of 3 log2(n) stages, below
-    10 eps in the L2 norm)"""
+    rounding of two pairs, four transforms of 3 log2(n) radix-2 stages, stays
+    below 20 eps in the L2 norm)"""
     banner("kxtran, xktran", n, prec)
     s = P.Solver(n, prec, viscos=0.01)
     try:

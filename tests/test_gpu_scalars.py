@@ -116,3 +116,39 @@ def test_scalars_1024_fp32_properties(P):
         assert np.array_equal(st[3], st[4])  # same Sc and gradient: same bits
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("n", [256, 512])
+def test_scalar_stage_precisions_agree(P, n):
+    """One RK2 step with a scalar in FP64 and FP32: the x pass with scalars has
+    its own points per thread and registers for each.  The FP64 velocity is that
+    of a step without scalars (the same operations up to the contraction of their
+    sums); FP32 differs from FP64 by its rounding, the bound of the other FP32
+    steps."""
+    print("[gpu case] scalar stage precisions", n, flush=True)
+    gsh = np.array([0.35, 0.15, 0.65, 0.85, 0.65, 0.15])
+    u0, out = None, []
+    for prec, nc in ((8, 0), (8, 1), (4, 1)):
+        s = P.Solver(n, prec, viscos=0.01, nc=nc, pr=[0.7] * nc, grad=[[0.0, 1.0, 0.5]] * nc)
+        try:
+            if u0 is None:
+                s.init_field(seed=n, kpeak=6.0, tke=0.5)
+                u0 = s.get_state()
+            # the scalar starts as a copy of the third component
+            s.put_state(np.concatenate([u0, u0[2:]]) if nc else u0)
+            s.set_shifts(gsh)
+            vm = s.stage_nonlinear(1)
+            xf, yf, zf = s.step_factors(2e-3)
+            s.stage_update(1, 2e-3, xf, yf, zf)
+            s.stage_nonlinear(2)
+            s.stage_update(2, 2e-3, xf, yf, zf)
+            out.append((vm, s.get_state()))
+        finally:
+            s.close()
+    (vm0, a), (vm1, b), (vm2, c) = out
+    assert vm1 == pytest.approx(vm0, rel=1e-12) and vm2 == pytest.approx(vm0, rel=2e-6)
+    m = u0[0] != 0
+    assert rel(b[:3], a, m) < 1e-12
+    assert rel(b[3], u0[2], m) > 1e-3  # the scalar was advected
+    for i in range(4):
+        assert rel(c[i], b[i], m) < TOL[4]
