@@ -61,7 +61,9 @@ __device__ __forceinline__ size_t pidx(int y, int z, int x, int n) { return ((si
 // ahead of its sums, which the compiler does by itself in FP32 but not in FP64
 // from r = 8 on: 512^3 FP64 to 32^3 2.49 ms with strided taps, 3.95 ms with the
 // loads among the sums, 0.86 ms (3.2 GB, 3.8 TB/s); 1024^3 FP64 to 32^3 18.7,
-// 30.1 and 5.5 ms; 256^3 FP64 to 32^3 268, 168 and 95 us.
+// 30.1 and 5.5 ms; 256^3 FP64 to 32^3 268, 168 and 95 us.  r = 2 takes its right
+// half and end tap as one vector: 256^3 to 128^3 FP32 118 -> 93 us (114 with
+// strided taps).
 // ---------------------------------------------------------------------------
 template <typename R, int H>
 struct Half {  // H consecutive values
@@ -103,8 +105,15 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int v = 0; v < 3; v++) {
         lo[v].load(row + v * N3 + x0);
-        hi[v].load(row + v * N3 + x1);
-        end[v] = row[v * N3 + x2];
+        if constexpr (r == 2) {
+          Half<R, 2> p;  // x2 is x1 + 1
+          p.load(row + v * N3 + x1);
+          hi[v].v[0] = p.v[0];
+          end[v] = p.v[1];
+        } else {
+          hi[v].load(row + v * N3 + x1);
+          end[v] = row[v * N3 + x2];
+        }
       }
       // the lanes of a wave are r values apart: a line that is not taken whole by
       // loads in a row is gone from the cache before its next one
