@@ -616,6 +616,38 @@ def test_les_fused_matches_per_routine(O, P, prec):
     assert err < (1e-10 if prec == 8 else 2e-5)
 
 
+@pytest.mark.parametrize("n,prec", [(64, 4), (128, 8), (128, 4), (256, 8), (256, 4)])
+def test_les_fused_sizes(P, n, prec):
+    """the stress in the fused x pass at the sizes past those whose tiles are
+    split over groups of threads (64^3 the largest of these), 256^3 FP32 with its
+    own points per thread: one step against the per-routine LES step, the bounds
+    of the test above"""
+    print("[gpu case] fused les sizes", n, prec, flush=True)
+    nu = 0.02
+    gsh = np.random.default_rng(21).random(6)
+    theta = _theta(13)
+    theta[-4:] += [-0.3, 0.1, 0.1, 0.1]  # a stress well above the rounding
+    u0, out = None, []
+    for closure, fused in ((False, True), (True, False), (True, True)):
+        s, m = P.Solver(n, prec, viscos=nu), P.Closure(n)
+        try:
+            if u0 is None:
+                s.init_field(seed=n, kpeak=n / 16, tke=0.5)
+                u0 = s.get_state()
+            s.put_state(u0)
+            m.set_params(theta)
+            P.Les(s, nu, np.pi, closure=m if closure else None, bf16=False, kf_shell=3, fused=fused).step(gsh)
+            out.append(s.get_state())
+        finally:
+            m.close()
+            s.close()
+    on = u0 != 0
+    err, effect = rel(out[2], out[1], on), rel(out[2], out[0], on)
+    print(f"fused vs per-routine {err:.2e}, effect of the stress {effect:.2e}", flush=True)
+    assert effect > 1e-3
+    assert err < (1e-10 if prec == 8 else 2e-5)
+
+
 def test_les_stage_with_scalars_is_refused(O, P):
     """The fused x pass carries either the subgrid stress or the scalars'
     advection terms: attaching a stress to a context with passive scalars
