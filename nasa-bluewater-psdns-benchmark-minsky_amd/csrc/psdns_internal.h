@@ -91,7 +91,9 @@ enum class Pass {
   YInvKx,     // kxtran: zero y Nyquist + y c2c +i, u -> yw
   YInvPlain,  // y c2c +i, u -> yw
   YInvGrad,   // du/dx, dw/dz of un on the mask + y c2c +i, un -> yw (two variables)
-  ZInv,       // gather yw + z c2c +i -> xi (args: number of variables; source 0 W1, 1 y-blocked yw in u, 2 the gradients of that many variables, two slots each in W1 -> three xi slots each)
+  ZInv,       // gather yw + z c2c +i -> xi (args: number of variables; source 0 W1, 1
+              // y-blocked yw in u, 2 the gradients of that many variables, two slots
+              // each in W1 -> three xi slots each)
   XC2R,       // gather xi + x c2r -> physical (arg: number of variables)
   XR2C,       // physical -> x r2c / n (arg: number of variables)
   XFused,     // c2r u,v,w (xi) -> products (+velmax, arg) -> r2c / n of 5 (X)

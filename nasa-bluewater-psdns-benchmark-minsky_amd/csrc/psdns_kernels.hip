@@ -333,12 +333,13 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
 // Shifted gradient of nv variables, y-transformed (a passive scalar:
 // phase1.f:44-64, itransform.f:190-203; the velocity for the SGS features):
 // phi_s = sx sy sz phi on the mask (0 elsewhere); per variable yw slot 0 =
-// Y[phi_s], slot 1 = Y[i ky phi_s] with Y the y c2c +i of a column.  The x and z derivatives multiply slot 0 by i kx and i kz, which
-// are constant along a column: the inverse z pass applies them (k_z_inv
-// DER), so two slots carry the three derivatives.  Tiles of B columns, natural
-// mapping in and out, yw in the cylinder layout; persistent over tiles as
-// k_y_inv (the next tile's loads in flight during the current transforms;
-// off-mask entries are not read, so they enter as zeros).
+// Y[phi_s], slot 1 = Y[i ky phi_s] with Y the y c2c +i of a column.  The x and
+// z derivatives multiply slot 0 by i kx and i kz, which are constant along a
+// column: the inverse z pass applies them (k_z_inv DER), so two slots carry
+// the three derivatives.  Tiles of B columns, natural mapping in and out, yw in
+// the cylinder layout; persistent over tiles as k_y_inv (the next tile's loads
+// in flight during the current transforms; off-mask entries are not read, so
+// they enter as zeros).
 // SH 1: shift factors in the state precision, sr = sx[nxh] | sy[n] | sz[n];
 // SH 2: FP64 factors and product (s64), rounded once; SH 0: no shift.
 // ---------------------------------------------------------------------------
@@ -425,8 +426,8 @@ __global__ void __launch_bounds__((YInv<R>::B * Team<N>::T))
 // z c2c +i; the last stage leaves the lines in the natural mapping for
 // contiguous stores along z.
 // DER (the gradient of nv variables, from k_y_grad's two slots Y[phi],
-// Y[i ky phi] of each): three outputs per variable, kx and y block, taken in turn (v fastest,
-// so that the second read of Y[phi] meets the cache): xi slot 0 = i kx
+// Y[i ky phi] of each): three outputs per variable, kx and y block, taken in
+// turn (v fastest, so that the second read of Y[phi] meets the cache): xi slot 0 = i kx
 // Z[Y[phi]] (kx constant per tile, applied after the transform), slot 1 =
 // Z[Y[i ky phi]], slot 2 = Z[i kz Y[phi]] (applied before it).
 // ---------------------------------------------------------------------------
@@ -554,7 +555,10 @@ struct XPass {
 #define PSDNS_XMFMA 0
 #endif
   // radix-8 stages on the matrix cores: 0 VALU (default), 1 FP32 MFMA,
-  // 2 split bf16 x 3 (a tuning build: build.py --define PSDNS_XMFMA=1)
+  // 2 split bf16 x 3 (a tuning build: build.py --define PSDNS_XMFMA=1).  They
+  // take lines of one wavefront with 8 points per thread, which a line of full
+  // length is at 512^3 FP32 only; at 1024^3 (16 points) the define changes
+  // nothing.  1024^3 was measured with half-length transforms.
   static constexpr int MX = PSDNS_XMFMA;
   // line stride: bank model of the transposed first stage's writes, 2-way at
   // most on 32 and 64 banks
@@ -779,13 +783,14 @@ __device__ __forceinline__ double wave_max(double v) {
 // of f^m, m = 1..8, in FP64 (each thread over its points, then the waves'
 // lanes, then the waves, in fixed orders).
 // Persistent over tiles and staged as k_x_fused: the copy of the next tile's
-// rows into LDS runs under the transform of the current one.  Three variables
-// at 512^3 FP32: 760 us with one tile per work-group and gathered register
-// loads, 575 us this way (3.1 GB, 5.4 TB/s: the copy rate).  The moments of two
-// variables there: 339 us, bound by VALU (the transform and 12 FP64 operations
-// per value), against 508 us for the transform, 1016 us for a kernel over the
-// stored fields with one FP64 atomic per wave and power, and 212 us for one
-// that formed the derivatives (now on load in the y pass).
+// rows into LDS runs under the transform of the current one, and that of the
+// first tile under the table fill.  Three variables at 512^3 FP32: 770 us with one
+// tile per work-group and gathered register loads, 545-575 us this way (3.1 GB, at
+// the copy rate); 256^3 FP64 188 and 160 us (210 with the fill first).  The
+// moments of two variables at 512^3 FP32: 339 us, bound by VALU (the transform
+// and 12 FP64 operations per value), against 508 us for the transform, 1016 us
+// for a kernel over the stored fields with one FP64 atomic per wave and power,
+// and 212 us for one that formed the derivatives (now on load in the y pass).
 template <typename R, int N, bool MOM>
 __global__ void __launch_bounds__((XPass<R, N, MOM>::NT))
     k_x_c2r(const C<R>* __restrict__ xi, R* __restrict__ ux, Geo g, const C<R>* __restrict__ tw,
@@ -911,7 +916,8 @@ __global__ void __launch_bounds__((XPass<R, N>::NT))
 // one thread applies it with an atomic max to one of kVelmaxSlots slots,
 // 256 bytes apart, chosen by work-group, so that the atomics spread over
 // the L2 channels instead of queueing on one address; k_velmax_reduce takes
-// the maximum of the slots and clears them for the next use.  Non-negative doubles order as their bit patterns.
+// the maximum of the slots and clears them for the next use.  Non-negative
+// doubles order as their bit patterns.
 // Every thread of the work-group (NT) calls it (one barrier inside).
 template <int NT>
 __device__ __forceinline__ void velmax_commit(double m, unsigned long long* velmax) {
@@ -937,7 +943,7 @@ __global__ void __launch_bounds__(kVelmaxSlots) k_velmax_reduce(unsigned long lo
   velmax[(size_t)threadIdx.x * kVelmaxStride] = 0;
   __syncthreads();
   for (int h = kVelmaxSlots / 2; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) s[threadIdx.x] = s[threadIdx.x] > s[threadIdx.x + h] ? s[threadIdx.x] : s[threadIdx.x + h];
+    if ((int)threadIdx.x < h && s[threadIdx.x] < s[threadIdx.x + h]) s[threadIdx.x] = s[threadIdx.x + h];
     __syncthreads();
   }
   if (threadIdx.x == 0) *out = s[0];
@@ -1065,14 +1071,14 @@ __attribute__((amdgpu_waves_per_eu(SC ? kScWaves<R, N> : XPass<R, N, !TAU>::kWav
   if (want_velmax) velmax_commit<X::NT>((double)vm * (double)N, velmax);
 }
 
-// The fused x pass of small grids (without scalars), where a tile's chain of three inverse and
-// five forward transforms is what a launch takes: a work-group of five groups
-// of NT threads per tile.  The rows of u, v and w are copied to LDS together;
-// groups 0..2 transform one each (3 and 4 repeat u and v, so that all meet the
-// same barriers) and leave the physical values in LDS; then group s forms
-// product s and transforms it forward: two transforms deep instead of eight,
-// the same operations on each value.
-// SPLIT_NOTE
+// The fused x pass of small grids (without scalars), where a tile's chain of
+// three inverse and five forward transforms is what a launch takes: a work-group
+// of five groups of NT threads per tile.  The rows of u, v and w are copied to
+// LDS together; groups 0..2 transform one each (3 and 4 repeat u and v, so that
+// all meet the same barriers) and leave the physical values in LDS; then group s
+// forms product s and transforms it forward: two transforms deep instead of
+// eight, the same operations on each value.  Per launch 8.0 -> 5.1 us at 32^3
+// FP32 and 12.6 -> 9.4 at 64^3 FP64.
 template <typename R, int N, bool TAU>
 __global__ void __launch_bounds__((5 * XPass<R, N>::NT))
     k_x_fused_split(const C<R>* __restrict__ xi, C<R>* __restrict__ xs, Geo g, const C<R>* __restrict__ tw,
@@ -1258,7 +1264,8 @@ __global__ void __launch_bounds__((ZFwd<R, N>::NT)) __attribute__((amdgpu_waves_
 }
 
 // k_z_fwd of small grids, as k_x_fused_split: group s of a tile's work-group
-// transforms slot s, P5 goes to groups 0 and 2 through LDS.
+// transforms slot s, P5 goes to groups 0 and 2 through LDS (7.8 -> 6.5 us per
+// launch at 64^3 FP64).
 template <typename R, int N>
 __global__ void __launch_bounds__((5 * ZFwd<R, N>::NT))
     k_z_fwd_split(const C<R>* __restrict__ xs, C<R>* __restrict__ w1, Geo g, const C<R>* __restrict__ tw,
@@ -2801,9 +2808,9 @@ struct Launch {
                                : k_y_fwd_update<R, N, 2, false>;
     static unsigned grids[4] = {0, 0, 0, 0};
     if (!grids[v]) grids[v] = persistent_grid((const void*)kern, NT, kYScale);
-    hipLaunchKernelGGL(kern, dim3(tiles_grid(grids[v], c.geo.ngrp)), dim3(NT), 0, c.stream, (const CR*)c.w1, (CR*)c.u, (CR*)c.un, c.geo,
-                       norm, sr, sr2, c.xfac, c.yfac, c.zfac, (const CR*)c.tw, c.geo.grp, c.geo.colx, c.geo.colz,
-                       (CR*)nullptr);
+    hipLaunchKernelGGL(kern, dim3(tiles_grid(grids[v], c.geo.ngrp)), dim3(NT), 0, c.stream, (const CR*)c.w1,
+                       (CR*)c.u, (CR*)c.un, c.geo, norm, sr, sr2, c.xfac, c.yfac, c.zfac, (const CR*)c.tw, c.geo.grp,
+                       c.geo.colx, c.geo.colz, (CR*)nullptr);
   }
   // RK4 substep k: y forward pass + wavespace_vel + advanc_k, shifts of
   // stage (k - 1) % 2 + 1
@@ -2817,9 +2824,9 @@ struct Launch {
                                : k_y_fwd_update<R, N, 14, false>;
     static unsigned grids[4] = {0, 0, 0, 0};
     if (!grids[k - 1]) grids[k - 1] = persistent_grid((const void*)kern, NT, kYScale);
-    hipLaunchKernelGGL(kern, dim3(tiles_grid(grids[k - 1], c.geo.ngrp)), dim3(NT), 0, c.stream, (const CR*)c.w1, (CR*)c.u, (CR*)c.un, c.geo,
-                       norm, sr, sr, c.xfac, c.yfac, c.zfac, (const CR*)c.tw, c.geo.grp, c.geo.colx, c.geo.colz,
-                       (CR*)u1);
+    hipLaunchKernelGGL(kern, dim3(tiles_grid(grids[k - 1], c.geo.ngrp)), dim3(NT), 0, c.stream, (const CR*)c.w1,
+                       (CR*)c.u, (CR*)c.un, c.geo, norm, sr, sr, c.xfac, c.yfac, c.zfac, (const CR*)c.tw, c.geo.grp,
+                       c.geo.colx, c.geo.colz, (CR*)u1);
   }
 };
 

@@ -45,8 +45,6 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
   return x ^ (x >> 31);
 }
 
-__device__ __forceinline__ size_t pidx(int y, int z, int x, int n) { return ((size_t)y * n + z) * n + x; }
-
 // ---------------------------------------------------------------------------
 // Box filter: coarse point (y, z, x) = fine point (r y, r z, r x); separable
 // (r + 1)-tap top-hat [1/2, 1, .., 1, 1/2] / r per direction (periodic).
@@ -655,14 +653,15 @@ __global__ void __launch_bounds__(256)
 // for those of the dense layers with BF16 (tanh_fast).
 //
 // What bounds it, BF16 at 128^3: issue. Per 16 points 1,440 cycles of matrix
-// instructions and about 3,000 of VALU (52 tanh per lane, two quarter-rate
-// instructions each), 236 us on end where nothing overlaps; 240 us per call,
-// against 178 us for the convolution with its 16 channels stored and 189 us
-// for the dense layers that read them back.  64^3: 37.5 us (75), with FP32
-// layers 87 us (179).  Before the weights were loaded with all loads in flight
-// and their LDS addresses formed once per tile: 270 us (209 without the tanh,
-// 218 without the convolution's products) and 46 us; two tiles per wave,
-// sharing each weight read, came to 262-360 us for 2 to 4 waves per SIMD.
+// instructions and about 3,000 of VALU (52 tanh per lane, 48 of them two
+// quarter-rate instructions each), 236 us on end where nothing overlaps; 258 us
+// per call (240 with the fast form for the convolution's four tanh too, which is
+// not exact enough there), against 178 us for the convolution with its 16
+// channels stored and 189 us for the dense layers that read them back.  64^3: 39
+// us (75), with FP32 layers 87 us (179).  Before the weights were loaded with all
+// loads in flight and their LDS addresses formed once per tile: 270 us (209
+// without the tanh, 218 without the convolution's products) and 46 us; two tiles
+// per wave, sharing each weight read, came to 262-360 us for 2 to 4 waves per SIMD.
 // ---------------------------------------------------------------------------
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
